@@ -127,7 +127,7 @@ int launch_gemm_tn_small(const double *A, size_t lda, int M, const double *B, si
                          const double *w, size_t K, int symm, double *out, hipStream_t s);
 /* tile list of a symmetric product restricted to some tiles (k_gemm_tn_splitk) */
 struct GramTiles {
-   int on, noff, nd;
+   int noff, nd, halves;
    unsigned char otm[32], otn[32], dt[8];
 };
 int launch_gemm_tn_splitk(const double *A, size_t lda, int M, const double *B, size_t ldb,
@@ -146,7 +146,7 @@ int launch_reduce_partials_kb(const double *partial, int splits, int nproj, int 
  * whose diagonal and off-diagonal tiles use different split counts */
 int launch_reduce_partials_symm(const double *partial, int M, size_t K, int splits, double *out,
                                 hipStream_t s);
-/* split counts a symmetric product uses: off-diagonal tiles and diagonal pairs */
+/* split counts a symmetric product uses: off-diagonal and diagonal tiles */
 void gemm_tn_symm_splits(int M, size_t K, int splits, int *sp_off, int *sp_dd);
 /* the same for a product restricted to noff off-diagonal and nd diagonal
  * tiles over about wgs workgroups (diagonal tiles as two half-range splits) */
@@ -177,7 +177,7 @@ struct TallArgs {
     * record per K block in fpart */
    const double2 *Bp; const double *w, *Gp; int ngp; double *fpart;
    const double *Kp = nullptr;     /* EPI_PRECOND: [K / 2] */
-   int ntn, per;                   /* set by the launcher */
+   int ntn, blocks;                /* set by the launcher */
 };
 int launch_gemm_tall(int epi, const TallArgs &a, hipStream_t s);
 

@@ -7,381 +7,283 @@
  *   - hml             -gcdotc(c1_i, cpsi_j)         ccpsdv3/cpsd.c:497-513
  *   - KB apply        c2_i += sw * beta (daxpy)     ccpsdv3/cpsd.c:290
  *   - constraint      c2 += dte c1 lmd (dgemm)      ccpsdv3/cpsd.c:482-488
- * Here they are two kernels built on v_mfma_f64_4x4x4_4b_f64, which on
- * gfx950 sustains ~74 TFLOP/s against ~36-49 for the 16x16x4 FP64 form:
+ * Here they are two kernels built on v_mfma_f64_16x16x4_f64 (mfma64.h):
  *   k_gemm_tn_splitk : small M x N output, reduction over the huge K = 2*ngp
  *                      real coefficients, split over blockIdx.z; 128 x 128
- *                      output tiles (8 waves of 64 x 32); the G-space weight
+ *                      output tiles; the G-space weight
  *                      (1 on the kx = 0 plane, 2 elsewhere: the
  *                      2*sum - sum_{kx=0} of ccpsdv3/gcdotc.c:25-27) is
  *                      applied to the A operand.
  *   k_gemm_tall      : tall output [ncol][K] = X^T A with a short reduction
- *                      (projectors or orbitals), 64-column x 128-row output
- *                      tiles over 8 waves, SD epilogues fused; the nonlocal
- *                      force (ccpsdv3/cpsd.c:291-304) reduces its output
- *                      against the projectors instead of storing it.
- * The instruction layout and the rotated-operand scheme are described in
- * mfma64.h.
+ *                      (projectors or orbitals), 128- or 64-column x 128-row
+ *                      output tiles over 8 waves, SD epilogues fused; the
+ *                      nonlocal force (ccpsdv3/cpsd.c:291-304) reduces its
+ *                      output against the projectors instead of storing it.
  */
 #include "cpsd_internal.h"
 #include "mfma64.h"
 #include <type_traits>
 #include <cstring>
 
+/* 16 bytes at base + off: a scalar base and a 32-bit lane offset */
+__device__ __forceinline__ double2 load2(const char *base, unsigned off)
+{
+   typedef double d2 __attribute__((ext_vector_type(2)));
+   const d2 v = *reinterpret_cast<const d2 *>(base + off);
+   return make_double2(v[0], v[1]);
+}
+
+/* sum over the 64 lanes of a wave, same tree in every wave */
+__device__ __forceinline__ double wave_sum(double v)
+{
+#pragma unroll
+   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+   return v;
+}
+
 /* ------------------------------------------------------- split-K TN */
 
-/* the split-K kernel's rotated B operands: 1 reads each rotation from LDS
- * (the swizzled tiles keep those reads conflict-free), 0 forms them with DPP
- * row rotations of one read.  At the 64-water cell the LDS reads made the
- * carried Gram 4-6% faster; the same change in the tall kernel made it
- * 3-5% slower, so that one keeps the DPP form. */
-#ifndef SPLITK_LDS_ROT
-#define SPLITK_LDS_ROT 1
-#endif
+/* scheduling hint: N times, one instruction of the kind MASK (0x100 LDS read,
+ * 0x200 LDS write, 0x20 global read) after M MFMAs */
+template<int MASK, int N, int M>
+__device__ __forceinline__ void sched_mix()
+{
+#pragma unroll
+   for (int i = 0; i < N; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, M, 0);
+      __builtin_amdgcn_sched_group_barrier(MASK, 1, 0);
+   }
+}
+
+template<int V> using template_int = std::integral_constant<int, V>;
+
 #define TT 128  /* output tile edge */
-#define KT 32   /* K step */
-#define TP (TT + 2)  /* row pitch of the epilogue staging tile */
+#define KT 16   /* K step */
+#define KC 32   /* K ranges are multiples of this */
+#define KP (KT + 2)  /* LDS row pitch: a 16-byte read of 8 rows covers the banks once */
 
-/* Diagonal-pair roles (see k_gemm_tn_splitk).  A diagonal tile's 36 upper
- * 16 x 16 blocks are split between four waves: two take half of the upper
- * right quadrant each (block rows 2h, 2h+1 x columns 4-7, 8 blocks), two the
- * upper triangle of a diagonal quadrant (rows and columns o..o+3, o = 0 or
- * 4, 10 blocks).  Role 1 is the quadrant half, role 2 the triangle; block b
- * of a role multiplies A row block dg_ai and B column block dg_bj. */
-__device__ constexpr int dg_nblk(int dm) { return dm == 1 ? 8 : 10; }
-__device__ constexpr int dg_na(int dm) { return dm == 1 ? 2 : 4; }
-__device__ constexpr int dg_ai(int dm, int b)
-{
-   return dm == 1 ? b >> 2 : (b < 4 ? 0 : b < 7 ? 1 : b < 9 ? 2 : 3);
-}
-__device__ constexpr int dg_bj(int dm, int b)
-{
-   return dm == 1 ? b & 3 : (b < 4 ? b : b < 7 ? b - 3 : b < 9 ? b - 5 : 3);
-}
+/* The blocks of a diagonal tile.  Its 36 upper 16 x 16 blocks are split
+ * evenly between the four waves: waves 0-2 take 3 x 3 squares on or above the
+ * diagonal (rows dg_row.., columns dg_col..), wave 3 the three remaining
+ * corners (p, p), (p, p+1), (p+1, p+1) at p = 0, 3, 6. */
+__device__ __forceinline__ int dg_row(int wave) { return wave == 1 ? 3 : 0; }
+__device__ __forceinline__ int dg_col(int wave) { return wave == 2 ? 2 : 5; }
+/* operand fragment f of a corner wave is block row dg_tri(f); block b of it
+ * multiplies fragments dg_ta(b) and dg_tb(b) */
+__device__ constexpr int dg_tri(int f) { return 3 * (f >> 1) + (f & 1); }
+__device__ constexpr int dg_ta(int b) { return 2 * (b / 3) + (b % 3 == 2); }
+__device__ constexpr int dg_tb(int b) { return 2 * (b / 3) + (b % 3 != 0); }
 
-/* 8 waves, each a (TMR/2) x 32 block of the TMR x 128 tile (TMR = 128, or 96
- * when that pads the row count less, e.g. 192 projectors).  One workgroup per
- * (tile, K split); the grid is 1D over the valid pairs only.  Workgroups go
- * to the 8 XCDs round-robin by block id, so block b is given pair
- * (b % 8) * per + b / 8: the workgroups one XCD runs together hold
- * consecutive pairs, i.e. all tiles of the same K range, which then share
- * that XCD's L2 (per = pairs / 8; 0 falls back to b itself).
+/* partial[z][m][n] = sum_{k in split z} w[k] A[m][k] B[n][k].  TMR x 128 output
+ * tiles (TMR = 128, or 96 when that pads the row count less, e.g. 192
+ * projectors), four waves of (TMR/2) x 64, K steps of 16 double-buffered in 72
+ * KB of LDS: two workgroups share a CU, so one's barriers and loads overlap
+ * the other's MFMAs.  The operands of the next 8 k are read from LDS between
+ * the MFMAs of the current ones; the weight is applied to the A rows on their
+ * way into LDS.  Each sum runs over k in order, one fused multiply-add per
+ * term (what the FP64 MFMA does with its four k), so a split's result does
+ * not depend on the tiling.
  *
- * A symmetric product (A = B, M = N) forms the tiles above the diagonal and
- * the diagonal tiles two at a time: a diagonal-pair workgroup loads the same
- * 256 rows as the off-diagonal tile (2d, 2d+1) and forms the 2 x 36 blocks on
- * or above the diagonals of tiles 2d and 2d+1 (waves 0-3 the first, 4-7 the
- * second), 18 blocks per SIMD against 16 for an off-diagonal tile, so the
- * workgroups of a launch take about the same time.
+ * One workgroup per (tile, K split); the grid is 1D over the pairs.
+ * Workgroups go to the 8 XCDs round-robin by block id, so block b is given
+ * pair (b % 8) * per + b / 8 with per = pairs / 8 rounded up (ids past the
+ * last pair exit): the workgroups one XCD runs together hold consecutive
+ * pairs, i.e. all tiles of the same K range, which then share that XCD's L2.
  *
- * With a tile list (tl.on), a symmetric product forms only the listed
- * off-diagonal tiles and the listed diagonal tiles, each diagonal tile by a
- * diagonal-pair workgroup whose two halves take the two halves of its K
- * range (rows of the same tile at k and at k + half) and write them as two
- * K splits, 2z and 2z + 1 (SELF instances only). */
-template<int TMR, bool SELF>
-__global__ void __launch_bounds__(512)
+ * A symmetric product (SYM: A = B, M = N) forms the listed tiles only: tiles
+ * above the diagonal in full, diagonal tiles by their upper 36 blocks, nine
+ * to a wave against 16 in a full tile.  Split z of a diagonal tile is the
+ * whole range z of kchunk_dd (tl.halves 1) or half h of range z' (z = 2 z' +
+ * h, tl.halves 2).
+ *
+ * Bound by the MFMA issue: at 64 waters (128^3, 256 orbitals, 384
+ * projectors) the KB projection takes 3.39 ms (64 TFLOP/s) and the Gram with
+ * <c1|c1> carried 3.68 ms (60); the form with four v_mfma_f64_4x4x4_4b
+ * per 16 x 16 block, 8 waves of 64 x 32 and one workgroup per CU took 4.24 and
+ * 4.46 ms (51 and 49 TFLOP/s). */
+template<int TMR, bool SYM>
+__global__ void __launch_bounds__(256, 2)
 k_gemm_tn_splitk(const double *__restrict__ A, size_t lda, int M,
                  const double *__restrict__ B, size_t ldb, int N,
-                 const double *__restrict__ w, size_t K, size_t kchunk, size_t kchunk_dd, int symm,
-                 int ntm, int ntile, long poff, int per, GramTiles tl, double *__restrict__ partial)
+                 const double *__restrict__ w, size_t K, size_t kchunk, size_t kchunk_dd,
+                 int ntm, int ntile, long poff, long pairs, GramTiles tl, double *__restrict__ partial)
 {
-   const int bid = blockIdx.x;
-   const long g = per > 0 ? (long)(bid & 7) * per + (bid >> 3) : bid;
+   /* a symmetric product's off-diagonal pairs and its shorter diagonal pairs
+    * are spread over the XCDs each by themselves, the longer ones first */
+   const long x = blockIdx.x & 7, t8 = blockIdx.x >> 3, po = SYM ? (poff + 7) >> 3 : gridDim.x >> 3;
+   const bool dd = SYM && t8 >= po;
+   const long g = dd ? x * ((gridDim.x >> 3) - po) + t8 - po : x * po + t8;
+   if (g >= (SYM && !dd ? poff : dd ? pairs - poff : pairs)) return;
    int tm, tn, kz;
-   bool dd = false, selfdd = false;
    size_t kc = kchunk;
-   if (SELF && symm && tl.on) {
-      if (g < poff) {
-         const int t = (int)(g % tl.noff);
-         kz = (int)(g / tl.noff);
-         tm = tl.otm[t];
-         tn = tl.otn[t];
-      } else {
-         const long h = g - poff;
-         tm = tn = tl.dt[h % tl.nd];
-         kz = (int)(h / tl.nd);
-         dd = selfdd = true;
-         kc = kchunk_dd;
-      }
-   } else if (symm) {
-      const int noff = ntm * (ntm - 1) / 2, ndd = (ntm + 1) / 2;
-      if (g < poff) {   /* tiles strictly above the diagonal, row by row */
-         int rem = (int)(g % noff);
-         kz = (int)(g / noff);
-         tm = 0;
-         while (rem >= ntm - 1 - tm) { rem -= ntm - 1 - tm; ++tm; }
-         tn = tm + 1 + rem;
-      } else {          /* diagonal pair (tm, tm + 1); tile ntm, if named, is empty */
-         const long h = g - poff;
-         tm = 2 * (int)(h % ndd);
-         kz = (int)(h / ndd);
-         tn = tm + 1;
-         dd = true;
-         kc = kchunk_dd;
-      }
+   if (dd) {
+      tm = tn = tl.dt[g % tl.nd];
+      kz = (int)(g / tl.nd);
+      kc = kchunk_dd;
+   } else if (SYM) {
+      const int t = (int)(g % tl.noff);
+      kz = (int)(g / tl.noff);
+      tm = tl.otm[t];
+      tn = tl.otn[t];
    } else {
       const int t = (int)(g % ntile);
       kz = (int)(g / ntile);
       tm = t % ntm;
       tn = t / ntm;
    }
-   const size_t kb = (size_t)kz * kc;
-   const size_t ke = min(K, kb + kc);
-   /* a single diagonal tile's second half starts khalf after the first */
-   const size_t khalf = (SELF && selfdd && ke > kb) ? ((ke - kb) / KT + 1) / 2 * KT : 0;
-   const size_t kend = (SELF && selfdd) ? min(ke, kb + khalf) : ke;
-   /* S[buf][0] holds the A tile, S[buf][1] the B tile, rows of KT doubles
-    * with the k index XOR-swizzled by the row: element (row, k) sits at
-    * column k ^ (row & 15).  An operand read takes 16 rows at one k per
-    * 16-lane group; unswizzled (or with any even pad) those rows would share
-    * bank pairs, swizzled they cover 16 distinct ones.  The loader's
-    * 16-byte stores keep a (k, k+1) pair together: column pair
-    * lq ^ (row & 14), its two values swapped when row is odd.  The same
-    * memory stages the output tile for the epilogue. */
-   __shared__ double Sbuf[2 * 2 * TT * KT > TT * TP ? 2 * 2 * TT * KT : TT * TP];
-   double (*const S)[2][TT][KT] = reinterpret_cast<double (*)[2][TT][KT]>(Sbuf);
-   __shared__ double Ws[2][SELF ? 2 : 1][KT];   /* weights of the A rows ([0]) and B rows ([1]) */
-   /* the wave index is uniform: read it as a scalar */
+   size_t kb = (size_t)(SYM && dd && tl.halves == 2 ? kz >> 1 : kz) * kc;
+   size_t ke = min(K, kb + kc);
+   if (SYM && dd && tl.halves == 2) {
+      const size_t khalf = ke > kb ? ((ke - kb) / KC + 1) / 2 * KC : 0;
+      if (kz & 1) kb += khalf;
+      else ke = min(ke, kb + khalf);
+   }
+   /* S[buf][0]: the weighted A rows, S[buf][1]: the B rows (of a diagonal
+    * tile the same rows without the weight).  Of each 8 k the pairs (q, q + 4)
+    * are adjacent: one 16-byte read hands a lane its slot of two successive
+    * instructions */
+   __shared__ __align__(16) double S[2][2][TT][KP];
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
    const int wm = wave & 1, wn = wave >> 1;
-#if SPLITK_LDS_ROT
-   /* the rotated B operands read straight from LDS: rotation r takes column
-    * 4 ((c / 4 + r) % 4) + c % 4 of the 16-column block (c = lane % 16) */
-   const int s1 = 1;
-   int rrow[4];
-#pragma unroll
-   for (int r = 0; r < 4; ++r) rrow[r] = 4 * ((((lane & 15) >> 2) + r) & 3) + (lane & 3);
-#else
-   const int s1 = rot_step(lane);
-#endif
-   /* loader: rows lr + 32 h (h < 4) of the tile, k pair 2 (tid % 16): 16
-    * lanes cover one 256-byte row segment, contiguous in global memory and,
-    * as 16-byte stores, conflict-free in LDS */
-   const int lr = tid >> 4, lq = (tid & 15) * 2;
+   const int l16 = lane & 15, lq4 = lane >> 4;
    constexpr int BI = TMR / 32;   /* 16-row blocks per wave */
-   constexpr int BA = BI > 4 ? BI : 4;
 
-   double acc[BA][2][4];   /* [row block][column block][rotation] */
-   double accx[2][4];      /* blocks 8, 9 of a triangle role */
+   /* Row addresses without branches: rows past M or N repeat the last one
+    * (their outputs are not written), so a load is a 32-bit lane offset on a
+    * scalar base that moves along K.  Rows lr + 32 h, 8 lanes to the 128-byte
+    * piece of a row. */
+   const int lr = tid >> 3, lc = tid & 7;
+   const int ar0 = tm * TMR, br0 = tn * TT;
+   const char *const abase = reinterpret_cast<const char *>(A + (size_t)ar0 * lda);
+   const char *const bbase = reinterpret_cast<const char *>(B + (size_t)br0 * ldb);
+   unsigned aoff[4], boff[4];
 #pragma unroll
-   for (int i = 0; i < BA; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-         for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0;
-#pragma unroll
-   for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) accx[j][r] = 0.0;
-
-   /* K tile k+1 waits in registers while tile k is multiplied; it is moved
-    * to the other LDS buffer halfway through tile k's MFMA stream and tile
-    * k+2 is requested right after, so loads, LDS stores and MFMAs overlap
-    * with one barrier per tile */
+   for (int h = 0; h < 4; ++h) {
+      aoff[h] = (unsigned)min(lr + 32 * h, M - 1 - ar0) * (unsigned)(lda * 8) + lc * 16;
+      boff[h] = (unsigned)min(lr + 32 * h, N - 1 - br0) * (unsigned)(ldb * 8) + lc * 16;
+   }
+   /* K tile t + 1 waits in registers while tile t is multiplied */
    double2 ra[4], rb[4], rw;
-   /* the B rows sit khalf further along K (0 except for a single diagonal
-    * tile), and are zero past the workgroup's K range */
    auto gload = [&](size_t k0) {
-      if constexpr (SELF) {
-         const bool bin = k0 + khalf < ke;
+      const char *const ak = abase + k0 * 8;
+      const char *const bk = bbase + k0 * 8;
 #pragma unroll
-         for (int h = 0; h < 4; ++h) {
-            const int r = lr + 32 * h, am = tm * TMR + r, bn = tn * TT + r;
-            ra[h] = make_double2(0.0, 0.0);
-            rb[h] = make_double2(0.0, 0.0);
-            if (r < TMR && am < M) ra[h] = *reinterpret_cast<const double2 *>(A + (size_t)am * lda + k0 + lq);
-            if (bn < N && bin) rb[h] = *reinterpret_cast<const double2 *>(B + (size_t)bn * ldb + k0 + khalf + lq);
-         }
-         if (tid < KT) {
-            const int hb = tid / (KT / 2), kq = 2 * (tid % (KT / 2));
-            rw = make_double2(0.0, 0.0);
-            if (hb == 0 || bin) rw = *reinterpret_cast<const double2 *>(w + k0 + (hb ? khalf : 0) + kq);
-         }
-      } else {
+      for (int h = 0; h < 4; ++h)
+         if (32 * h < TMR) ra[h] = load2(ak, aoff[h]);
+      if (!SYM || !dd) {
 #pragma unroll
-         for (int h = 0; h < 4; ++h) {
-            const int r = lr + 32 * h, am = tm * TMR + r, bn = tn * TT + r;
-            ra[h] = make_double2(0.0, 0.0);
-            rb[h] = make_double2(0.0, 0.0);
-            if (r < TMR && am < M) ra[h] = *reinterpret_cast<const double2 *>(A + (size_t)am * lda + k0 + lq);
-            if (bn < N) rb[h] = *reinterpret_cast<const double2 *>(B + (size_t)bn * ldb + k0 + lq);
-         }
-         if (tid < KT / 2) rw = *reinterpret_cast<const double2 *>(w + k0 + 2 * tid);
+         for (int h = 0; h < 4; ++h) rb[h] = load2(bk, boff[h]);
       }
+      rw = load2(reinterpret_cast<const char *>(w + k0), lc * 16);
    };
-   /* rows lr + 32 h all have row & 15 == lr & 15 */
-   const int sq = lq ^ (lr & 14);
-   const bool swp = lr & 1;
+   /* k = 2 lc, 2 lc + 1 of rows lr + 32 h */
+   const int sq = 8 * (lc >> 2) + 4 * (lc & 1) + ((lc >> 1) & 1);
+   auto lput = [&](double *row, double2 v) {
+      row[sq] = v.x;
+      row[sq + 2] = v.y;
+   };
    auto lstore = [&](int bf) {
 #pragma unroll
       for (int h = 0; h < 4; ++h) {
-         *reinterpret_cast<double2 *>(&S[bf][0][lr + 32 * h][sq]) = swp ? make_double2(ra[h].y, ra[h].x) : ra[h];
-         *reinterpret_cast<double2 *>(&S[bf][1][lr + 32 * h][sq]) = swp ? make_double2(rb[h].y, rb[h].x) : rb[h];
+         if (32 * h < TMR) lput(S[bf][0][lr + 32 * h], make_double2(ra[h].x * rw.x, ra[h].y * rw.y));
+         lput(S[bf][1][lr + 32 * h], SYM && dd ? ra[h] : rb[h]);
       }
-      if constexpr (SELF) {
-         if (tid < KT) {
-            const int hb = tid / (KT / 2), kq = 2 * (tid % (KT / 2));
-            Ws[bf][hb][kq] = rw.x;
-            Ws[bf][hb][kq + 1] = rw.y;
-         }
-      } else {
-         if (tid < KT / 2) { Ws[bf][0][2 * tid] = rw.x; Ws[bf][0][2 * tid + 1] = rw.y; }
-      }
+   };
+   /* k = 8 ks + lq4 and 8 ks + 4 + lq4 of a row */
+   auto pair_at = [&](int bf, int half, int row, int ks) {
+      return *reinterpret_cast<const double2 *>(&S[bf][half][row][8 * ks + 2 * lq4]);
    };
 
-   /* diagonal pair: wave w works on tile half hs = w / 4 (operand S[.][hs]);
-    * waves 0, 1, 6, 7 take role 1 (quadrant half 2h, 2h+1 with h = w % 2),
-    * waves 2-5 role 2 (triangle o = 4 (w % 2)).  Block b is accumulated in
-    * acc[b / 2][b % 2] (b < 8) or accx[b - 8]. */
-   const int hs = wave >> 2;
-   const int dm = !dd ? 0 : (wave == 0 || wave == 1 || wave == 6 || wave == 7) ? 1 : 2;
-   const int drow0 = dm == 1 ? 2 * (wave & 1) : 4 * (wave & 1);   /* first A row block */
-   const int dcol0 = dm == 1 ? 4 : drow0;                         /* first B column block */
-   auto blk = [&](int b, int r) -> double & { return b < 8 ? acc[(b & 7) >> 1][b & 1][r] : accx[b & 1][r]; };
-   auto mma_diag = [&](auto role, int bf, int ks) {
-      constexpr int DM = decltype(role)::value;
-      const int kk = 4 * ks + (lane >> 4), kx = kk ^ (lane & 15);
-      const double wk = Ws[bf][SELF ? hs : 0][kk];
-      double a[4], bv[4][4];
+   /* the K loop, specialised per wave role: NA x NB fragments, blocks
+    * (ia(b), jb(b)), b < NBLK */
+   auto kloop = [&](auto na_, auto nb_, auto nblk_, auto arow, auto brow, auto ia, auto jb, mfma_d4 *acc) {
+      constexpr int NA = decltype(na_)::value, NB = decltype(nb_)::value, NBLK = decltype(nblk_)::value;
+      struct Frag { double2 a[NA], b[NB]; };
+      auto fread = [&](Frag &f, int bf, int ks) {
 #pragma unroll
-      for (int i = 0; i < dg_na(DM); ++i) a[i] = S[bf][hs][16 * (drow0 + i) + (lane & 15)][kx] * wk;
-#if SPLITK_LDS_ROT
+         for (int i = 0; i < NA; ++i) f.a[i] = pair_at(bf, 0, 16 * arow(i) + l16, ks);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-         for (int r = 0; r < 4; ++r) bv[j][r] = S[bf][hs][16 * (dcol0 + j) + rrow[r]][kk ^ rrow[r]];
-#else
-#pragma unroll
-      for (int j = 0; j < 4; ++j) rotations(S[bf][hs][16 * (dcol0 + j) + (lane & 15)][kx], bv[j]);
-#endif
-#pragma unroll
-      for (int b = 0; b < dg_nblk(DM); ++b)
-#pragma unroll
-         for (int r = 0; r < 4; ++r) blk(b, r) = mfma4(a[dg_ai(DM, b)], bv[dg_bj(DM, b)][r], blk(b, r));
-   };
-   auto mma_full = [&](int bf, int ks) {
-      const int kk = 4 * ks + (lane >> 4), kx = kk ^ (lane & 15);
-      const double wk = Ws[bf][0][kk];
-      double a[BI];
-#pragma unroll
-      for (int i = 0; i < BI; ++i) a[i] = S[bf][0][(TMR / 2) * wm + 16 * i + (lane & 15)][kx] * wk;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-         double b[4];
-#if SPLITK_LDS_ROT
-#pragma unroll
-         for (int r = 0; r < 4; ++r) b[r] = S[bf][1][32 * wn + 16 * j + rrow[r]][kk ^ rrow[r]];
-#else
-         rotations(S[bf][1][32 * wn + 16 * j + (lane & 15)][kx], b);
-#endif
-#pragma unroll
-         for (int i = 0; i < BI; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[i][j][r] = mfma4(a[i], b[r], acc[i][j][r]);
-      }
-   };
-
-   /* the K loop, specialised per wave role so that no branch sits between
-    * the unrolled MFMA steps */
-   auto kloop = [&](auto role) {
-      constexpr int DM = decltype(role)::value;
-      if (kb < kend) {
-         gload(kb);
-         lstore(0);
-      }
-      __syncthreads();
-      if (kb + KT < kend) gload(kb + KT);
-      int buf = 0;
-      for (size_t k0 = kb; k0 < kend; k0 += KT) {
-#pragma unroll
-         for (int ks = 0; ks < KT / 8; ++ks) DM ? mma_diag(role, buf, ks) : mma_full(buf, ks);
-         if (k0 + KT < kend) {
-            lstore(buf ^ 1);
-            if (k0 + 2 * KT < kend) gload(k0 + 2 * KT);
-         }
-#pragma unroll
-         for (int ks = KT / 8; ks < KT / 4; ++ks) DM ? mma_diag(role, buf, ks) : mma_full(buf, ks);
-         __syncthreads();
-         buf ^= 1;
-      }
-   };
-   if (TMR != TT || dm == 0) kloop(std::integral_constant<int, 0>{});
-   else if (dm == 1) kloop(std::integral_constant<int, 1>{});
-   else kloop(std::integral_constant<int, 2>{});
-
-   /* stage the tile in LDS, then write whole 1 KB rows of the partial */
-   double (*T)[TP] = reinterpret_cast<double (*)[TP]>(Sbuf);
-   const int q = lane >> 4, ab = (lane >> 2) & 3, bb = lane & 3;
-   auto put = [&](int m, int n, int ml, int zz) {
-      double *dst = partial + ((size_t)zz * M + m) * N + n;
-      if (n + 1 < N && !(N & 1)) {
-         *reinterpret_cast<double2 *>(dst) = make_double2(T[ml][2 * lane], T[ml][2 * lane + 1]);
-      } else {
-         dst[0] = T[ml][2 * lane];
-         if (n + 1 < N) dst[1] = T[ml][2 * lane + 1];
-      }
-   };
-   if (TMR == TT && dd) {
-      auto stage = [&](auto role) {
-         constexpr int DM = decltype(role)::value;
-#pragma unroll
-         for (int b = 0; b < dg_nblk(DM); ++b) {
-            const int I = drow0 + dg_ai(DM, b), J = dcol0 + dg_bj(DM, b);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) T[16 * I + 4 * ab + q][16 * J + 4 * ((ab + s1 * r) & 3) + bb] = blk(b, r);
-         }
+         for (int j = 0; j < NB; ++j) f.b[j] = pair_at(bf, 1, 16 * brow(j) + l16, ks);
       };
-      /* one diagonal tile at a time; only its upper 16 x 16 blocks exist */
+      auto mma = [&](const Frag &f) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-         if (hs == h) {
-            if (dm == 1) stage(std::integral_constant<int, 1>{});
-            else stage(std::integral_constant<int, 2>{});
-         }
-         __syncthreads();
-         const int t0 = (tm + ((SELF && selfdd) ? 0 : h)) * TT, n = t0 + 2 * lane;
-         if (n < N) {
-            for (int ml = wave; ml < TT; ml += 8) {
-               const int m = t0 + ml;
-               if (m >= M) break;
-               if (2 * lane < 16 * (ml >> 4)) continue;
-               put(m, n, ml, (SELF && selfdd) ? 2 * kz + h : kz);
-            }
-         }
-         __syncthreads();
+         for (int b = 0; b < NBLK; ++b) acc[b] = mfma16(f.a[ia(b)].x, f.b[jb(b)].x, acc[b]);
+#pragma unroll
+         for (int b = 0; b < NBLK; ++b) acc[b] = mfma16(f.a[ia(b)].y, f.b[jb(b)].y, acc[b]);
+      };
+#pragma unroll
+      for (int b = 0; b < NBLK; ++b) acc[b] = mfma_d4{0.0, 0.0, 0.0, 0.0};
+      if (kb >= ke) return;
+      const int nt = (int)((ke - kb + KT - 1) / KT);
+      gload(kb);
+      lstore(0);
+      gload(kb + (nt > 1 ? KT : 0));
+      __syncthreads();
+      Frag f0, f1;
+      fread(f0, 0, 0);
+      int buf = 0;
+      /* branch-free body: one workgroup's MFMA stream has to stay fed from one
+       * wave per SIMD, so the LDS reads and writes and the loads of the next
+       * tile are spread between the MFMAs (64 cycles each) */
+      for (int t = 0; t + 1 < nt; ++t) {
+         fread(f1, buf, 1);
+         mma(f0);
+         lstore(buf ^ 1);
+         sched_mix<0x100, NA + NB, 1>();
+         sched_mix<0x200, TMR / 32 + 4, 1>();
+         __syncthreads();   /* every read of this tile has been issued and has returned */
+         buf ^= 1;
+         fread(f0, buf, 0);
+         gload(kb + (size_t)min(t + 2, nt - 1) * KT);
+         mma(f1);
+         sched_mix<0x100, NA + NB, 1>();
+         sched_mix<0x20, TMR / 32 + 5, 1>();
       }
-      return;
-   }
+      fread(f1, buf, 1);
+      mma(f0);
+      mma(f1);
+   };
+   auto store_block = [&](int m0, int n0, const mfma_d4 &v) {
+      const int n = n0 + l16;
 #pragma unroll
-   for (int i = 0; i < BI; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-         for (int r = 0; r < 4; ++r)
-            T[(TMR / 2) * wm + 16 * i + 4 * ab + q][32 * wn + 16 * j + 4 * ((ab + s1 * r) & 3) + bb] =
-               acc[i][j][r];
-   __syncthreads();
-   const int n = tn * TT + 2 * lane;
-   if (n < N) {
-#pragma unroll 4
-      for (int ml = wave; ml < TMR; ml += 8) {
-         const int m = tm * TMR + ml;
-         if (m >= M) break;
-         put(m, n, ml, kz);
+      for (int r = 0; r < 4; ++r) {
+         const int m = m0 + mfma16_row(r, lane);
+         if (m < M && n < N) partial[((size_t)kz * M + m) * N + n] = v[r];
       }
+   };
+   template_int<BI> nbi;
+   template_int<4> n4;
+   if (!SYM || !dd) {
+      mfma_d4 acc[BI * 4];
+      kloop(nbi, n4, template_int<BI * 4>{}, [&](int i) { return BI * wm + i; }, [&](int j) { return 4 * wn + j; },
+            [](int b) { return b % BI; }, [](int b) { return b / BI; }, acc);
+#pragma unroll
+      for (int b = 0; b < BI * 4; ++b)
+         store_block(ar0 + 16 * (BI * wm + b % BI), br0 + 16 * (4 * wn + b / BI), acc[b]);
+   } else if (wave < 3) {
+      mfma_d4 acc[9];
+      const int r0 = dg_row(wave), c0 = dg_col(wave);
+      kloop(template_int<3>{}, template_int<3>{}, template_int<9>{}, [&](int i) { return r0 + i; },
+            [&](int j) { return c0 + j; }, [](int b) { return b % 3; }, [](int b) { return b / 3; }, acc);
+#pragma unroll
+      for (int b = 0; b < 9; ++b) store_block(ar0 + 16 * (r0 + b % 3), br0 + 16 * (c0 + b / 3), acc[b]);
+   } else {
+      mfma_d4 acc[9];
+      kloop(template_int<6>{}, template_int<6>{}, template_int<9>{}, [](int i) { return dg_tri(i); },
+            [](int j) { return dg_tri(j); }, [](int b) { return dg_ta(b); }, [](int b) { return dg_tb(b); }, acc);
+#pragma unroll
+      for (int b = 0; b < 9; ++b)
+         store_block(ar0 + 16 * dg_tri(dg_ta(b)), br0 + 16 * dg_tri(dg_tb(b)), acc[b]);
    }
 }
 
 /* K splits of a symmetric product: the tiles above the diagonal take sp_off
- * and the diagonal pairs sp_dd, in the ratio of their work per SIMD (16 : 18
- * blocks of 16 x 16), so that both kinds of workgroup take about as long;
- * the total is about what `splits` for every tile would give */
+ * and the diagonal tiles sp_dd, in the ratio 16 : 18 */
 void gemm_tn_symm_splits(int M, size_t K, int splits, int *sp_off, int *sp_dd)
 {
    const int ntm = (M + TT - 1) / TT;
    const int noff = ntm * (ntm - 1) / 2, ndd = (ntm + 1) / 2;
-   const int kmax = (int)(K / KT) > 0 ? (int)(K / KT) : 1;
+   const int kmax = (int)(K / KC) > 0 ? (int)(K / KC) : 1;
    if (noff == 0) {
       *sp_off = 0;
       *sp_dd = splits < kmax ? splits : kmax;
@@ -396,71 +298,12 @@ void gemm_tn_symm_splits(int M, size_t K, int splits, int *sp_off, int *sp_dd)
    *sp_dd = sd < kmax ? sd : kmax;
 }
 
-/* tiles of one K split: all of them, or for a symmetric product those above
- * the diagonal plus the diagonal pairs */
-int gemm_tn_tiles(int M, int N, int symm)
-{
-   if (symm) {
-      const int ntm = (M + TT - 1) / TT;
-      return ntm * (ntm - 1) / 2 + (ntm + 1) / 2;
-   }
-   const int pad128 = (M + 127) / 128 * 128 - M, pad96 = (M + 95) / 96 * 96 - M;
-   const int tmr = pad96 < pad128 ? 96 : TT;
-   return ((M + tmr - 1) / tmr) * ((N + TT - 1) / TT);
-}
-
-
-int launch_gemm_tn_splitk(const double *A, size_t lda, int M, const double *B, size_t ldb,
-                          int N, const double *w, size_t K, int splits, int symm,
-                          double *partial, hipStream_t s)
-{
-   if (K % KT) { cpsd_set_error("gemm_tn: K=%zu not a multiple of %d", K, KT); return -1; }
-   if (symm && M != N) { cpsd_set_error("gemm_tn: symmetric product needs M == N"); return -1; }
-   auto chunk = [&](int sp) {
-      size_t kc = (K + sp - 1) / sp;
-      return (kc + KT - 1) / KT * KT;
-   };
-   /* row tile: 128, or 96 when that leaves fewer padding rows (a symmetric
-    * product keeps square tiles) */
-   const int pad128 = (M + 127) / 128 * 128 - M, pad96 = (M + 95) / 96 * 96 - M;
-   const int tmr = (!symm && pad96 < pad128) ? 96 : TT;
-   const int ntm = (M + tmr - 1) / tmr;
-   const int ntile = gemm_tn_tiles(M, N, symm);
-   long pairs, poff = 0;
-   size_t kchunk, kchunk_dd = 0;
-   if (symm) {
-      int so, sd;
-      gemm_tn_symm_splits(M, K, splits, &so, &sd);
-      const int noff = ntm * (ntm - 1) / 2, ndd = (ntm + 1) / 2;
-      poff = (long)noff * so;
-      pairs = poff + (long)ndd * sd;
-      kchunk = so > 0 ? chunk(so) : 0;
-      kchunk_dd = chunk(sd);
-   } else {
-      pairs = (long)ntile * splits;
-      kchunk = chunk(splits);
-   }
-   const int per = pairs % 8 == 0 ? (int)(pairs / 8) : 0;
-   GramTiles tl;
-   memset(&tl, 0, sizeof tl);
-   if (tmr == 96)
-      hipLaunchKernelGGL((k_gemm_tn_splitk<96, false>), dim3((unsigned)pairs), dim3(512), 0, s, A, lda, M, B,
-                         ldb, N, w, K, kchunk, kchunk_dd, symm, ntm, ntile, poff, per, tl, partial);
-   else
-      hipLaunchKernelGGL((k_gemm_tn_splitk<TT, false>), dim3((unsigned)pairs), dim3(512), 0, s, A, lda, M, B,
-                         ldb, N, w, K, kchunk, kchunk_dd, symm, ntm, ntile, poff, per, tl, partial);
-   CPSD_CHECK(hipGetLastError());
-   return 0;
-}
-
-/* K splits of a symmetric product restricted to the tiles of a list: the
- * off-diagonal tiles take sp_off splits and the diagonal tiles sp_dd, each of
- * the latter formed as two half-range splits (2 sp_dd partials).  A diagonal
- * workgroup does 18 blocks per SIMD over half its range against 16 over the
- * whole range for an off-diagonal one, so sp_dd = 9/16 sp_off balances them */
+/* the same for a product restricted to noff off-diagonal and nd diagonal
+ * tiles over about wgs workgroups, each diagonal range formed as two halves
+ * (2 sp_dd partials) */
 void gemm_tn_list_splits(int noff, int nd, size_t K, long wgs, int *sp_off, int *sp_dd)
 {
-   const int kmax = (int)(K / KT) > 0 ? (int)(K / KT) : 1;
+   const int kmax = (int)(K / KC) > 0 ? (int)(K / KC) : 1;
    const int kmax2 = kmax / 2 > 0 ? kmax / 2 : 1;
    int so = noff > 0 ? (int)(16 * wgs / (16L * noff + 9L * nd)) : 0;
    if (noff > 0 && so < 1) so = 1;
@@ -472,13 +315,87 @@ void gemm_tn_list_splits(int noff, int nd, size_t K, long wgs, int *sp_off, int 
    *sp_dd = sd;
 }
 
+/* tiles of one K split (pairs of diagonal tiles count as one) */
+int gemm_tn_tiles(int M, int N, int symm)
+{
+   if (symm) {
+      const int ntm = (M + TT - 1) / TT;
+      return ntm * (ntm - 1) / 2 + (ntm + 1) / 2;
+   }
+   const int pad128 = (M + 127) / 128 * 128 - M, pad96 = (M + 95) / 96 * 96 - M;
+   const int tmr = pad96 < pad128 ? 96 : TT;
+   return ((M + tmr - 1) / tmr) * ((N + TT - 1) / TT);
+}
+
+/* whole rounds of the 8 XCDs */
+static dim3 xcd_grid(long blocks) { return dim3((unsigned)((blocks + 7) / 8 * 8)); }
+
+static size_t k_chunk(size_t K, int sp)
+{
+   const size_t kc = (K + sp - 1) / sp;
+   return (kc + KC - 1) / KC * KC;
+}
+
+/* the listed tiles of the symmetric product A W A^T, so and sd K ranges */
+static int launch_tn_list(const GramTiles &tl, const double *A, size_t lda, int M, const double *w, size_t K, int so,
+                          int sd, double *partial, hipStream_t s)
+{
+   const long poff = (long)tl.noff * so;
+   const long pairs = poff + (long)tl.nd * sd * tl.halves;
+   hipLaunchKernelGGL((k_gemm_tn_splitk<TT, true>), dim3(xcd_grid(poff).x + xcd_grid(pairs - poff).x), dim3(256), 0, s, A, lda,
+                      M, A, lda, M,
+                      w, K, so > 0 ? k_chunk(K, so) : 0, sd > 0 ? k_chunk(K, sd) : 0, 0, 0, poff, pairs, tl, partial);
+   CPSD_CHECK(hipGetLastError());
+   return 0;
+}
+
+int launch_gemm_tn_splitk(const double *A, size_t lda, int M, const double *B, size_t ldb,
+                          int N, const double *w, size_t K, int splits, int symm,
+                          double *partial, hipStream_t s)
+{
+   if (K % KC) { cpsd_set_error("gemm_tn: K=%zu not a multiple of %d", K, KC); return -1; }
+   if (symm && (M != N || M > 8 * TT)) { cpsd_set_error("gemm_tn: symmetric product of %d x %d", M, N); return -1; }
+   /* 32-bit lane offsets of the rows of a tile */
+   if (lda * 8 * TT >= (1ull << 32) || ldb * 8 * TT >= (1ull << 32)) {
+      cpsd_set_error("gemm_tn: rows of %zu doubles", lda > ldb ? lda : ldb);
+      return -1;
+   }
+   GramTiles tl;
+   memset(&tl, 0, sizeof tl);
+   if (symm) {
+      const int ntm = (M + TT - 1) / TT;
+      for (int i = 0; i < ntm; ++i) {
+         for (int j = i + 1; j < ntm; ++j) { tl.otm[tl.noff] = (unsigned char)i; tl.otn[tl.noff] = (unsigned char)j; ++tl.noff; }
+         tl.dt[tl.nd++] = (unsigned char)i;
+      }
+      tl.halves = 1;
+      int so, sd;
+      gemm_tn_symm_splits(M, K, splits, &so, &sd);
+      return launch_tn_list(tl, A, lda, M, w, K, so, sd, partial, s);
+   }
+   /* row tile: 128, or 96 when that leaves fewer padding rows */
+   const int pad128 = (M + 127) / 128 * 128 - M, pad96 = (M + 95) / 96 * 96 - M;
+   const int tmr = pad96 < pad128 ? 96 : TT;
+   const int ntm = (M + tmr - 1) / tmr, ntile = gemm_tn_tiles(M, N, 0);
+   const long pairs = (long)ntile * splits;
+   const size_t kchunk = k_chunk(K, splits);
+   if (tmr == 96)
+      hipLaunchKernelGGL((k_gemm_tn_splitk<96, false>), xcd_grid(pairs), dim3(256), 0, s, A, lda, M, B,
+                         ldb, N, w, K, kchunk, 0, ntm, ntile, 0, pairs, tl, partial);
+   else
+      hipLaunchKernelGGL((k_gemm_tn_splitk<TT, false>), xcd_grid(pairs), dim3(256), 0, s, A, lda, M, B,
+                         ldb, N, w, K, kchunk, 0, ntm, ntile, 0, pairs, tl, partial);
+   CPSD_CHECK(hipGetLastError());
+   return 0;
+}
+
 /* the Gram of [C1 C2] (M = 2 ne rows of stride lda, ne a multiple of 128)
  * without the C1 x C1 block: every 128 x 128 tile with a row or column in the
  * C2 block (rows [c2row, c2row + ne)) */
 int launch_gram_c2(const double *A, size_t lda, int M, int c2row, const double *w, size_t K, long wgs,
                    double *partial, size_t partial_cap, int *sp_off, int *sp_dd, hipStream_t s)
 {
-   if (K % KT) { cpsd_set_error("gram: K=%zu not a multiple of %d", K, KT); return -1; }
+   if (K % KC || lda * 8 * TT >= (1ull << 32)) { cpsd_set_error("gram: K=%zu not a multiple of %d, or too long", K, KC); return -1; }
    if (M % TT || c2row % TT || M > 8 * TT) {
       cpsd_set_error("gram: %d rows (C2 from row %d) are not whole 128-row tiles (at most 8)", M, c2row);
       return -1;
@@ -487,7 +404,6 @@ int launch_gram_c2(const double *A, size_t lda, int M, int c2row, const double *
    auto in_c2 = [&](int t) { return t >= c0 && t < c1; };
    GramTiles tl;
    memset(&tl, 0, sizeof tl);
-   tl.on = 1;
    for (int i = 0; i < ntm; ++i)
       for (int j = i + 1; j < ntm; ++j)
          if (in_c2(i) || in_c2(j)) { tl.otm[tl.noff] = (unsigned char)i; tl.otn[tl.noff] = (unsigned char)j; ++tl.noff; }
@@ -495,25 +411,15 @@ int launch_gram_c2(const double *A, size_t lda, int M, int c2row, const double *
       if (in_c2(i)) tl.dt[tl.nd++] = (unsigned char)i;
    int so, sd;
    gemm_tn_list_splits(tl.noff, tl.nd, K, wgs, &so, &sd);
+   tl.halves = 2;
    const int zmax = so > 2 * sd ? so : 2 * sd;
    if ((size_t)zmax * M * M > partial_cap) {
       cpsd_set_error("gram: %d splits of %d x %d do not fit the partial buffer", zmax, M, M);
       return -1;
    }
-   auto chunk = [&](int sp) {
-      size_t kc = (K + sp - 1) / sp;
-      return (kc + KT - 1) / KT * KT;
-   };
-   const long poff = (long)tl.noff * so;
-   const long pairs = poff + (long)tl.nd * sd;
-   const int per = pairs % 8 == 0 ? (int)(pairs / 8) : 0;
-   const size_t kchunk = so > 0 ? chunk(so) : 0, kchunk_dd = chunk(sd);
-   hipLaunchKernelGGL((k_gemm_tn_splitk<TT, true>), dim3((unsigned)pairs), dim3(512), 0, s, A, lda, M, A, lda, M,
-                      w, K, kchunk, kchunk_dd, 1, ntm, 0, poff, per, tl, partial);
-   CPSD_CHECK(hipGetLastError());
    *sp_off = so;
    *sp_dd = 2 * sd;
-   return 0;
+   return launch_tn_list(tl, A, lda, M, w, K, so, sd, partial, s);
 }
 
 /* out[m][n] = sum_z partial[z][m][n] over the splits that formed (m, n):
@@ -613,14 +519,6 @@ int launch_reduce_partials_symm(const double *partial, int M, size_t K, int spli
 
 /* ------------------------------------------------- small M x N (TN) */
 
-/* sum over the 64 lanes of a wave, same tree in every wave */
-__device__ __forceinline__ double wave_sum(double v)
-{
-#pragma unroll
-   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-   return v;
-}
-
 /* out[m][n] = sum_k w[k] A[m][k] B[n][k] for small M, N: one 1024-thread
  * workgroup per output (per upper-triangle pair m <= n when symm, mirrored),
  * its 16 waves taking interleaved 16-byte pieces of K so that many loads are
@@ -684,184 +582,241 @@ int launch_gemm_tn_small(const double *A, size_t lda, int M, const double *B, si
 #define MC 16   /* reduction step */
 
 
-/* waves arranged WK (along K) x WN (along the output columns) = 8; at most
- * 128 VGPRs and 68 KB of LDS, so that two workgroups share a CU and one's
- * epilogue traffic overlaps the other's MFMA stream */
+/* Output tile: TK = 128 rows of K x NT columns over 4 waves: 64 K rows x 64
+ * columns each (NT = 128), or 32 K rows x 64 columns (NT = 64).  32 K rows are
+ * two 16-column MFMA blocks, the even and the odd ones, so that one 16-byte
+ * LDS read feeds both and a lane ends up with whole complex coefficients: 16
+ * lanes hold 256 contiguous bytes of an output row and the SD epilogues run
+ * straight from the accumulators.  At most 256 VGPRs and 70 KB of LDS: two
+ * workgroups share a CU and one's epilogue traffic overlaps the other's MFMA
+ * stream.  Bound by the MFMA issue and, for short reductions, by the C2
+ * update: at 64 waters the KB apply takes 3.4 ms (64
+ * TFLOP/s) and the constraint 2.5 (4.28 and 2.93 ms with v_mfma_f64_4x4x4_4b
+ * and DPP-rotated operands). */
 template<int EPI, int NT>
-__global__ void __launch_bounds__(512, 4) k_gemm_tall(TallArgs a)
+__global__ void __launch_bounds__(256, 2) k_gemm_tall(TallArgs a)
 {
-   constexpr int WN = NT / 64, WK = 8 / WN;
-   constexpr int BI = TK / WK / 16;          /* 16-row blocks of K per wave */
    constexpr int BJ = 4;                     /* 16-column blocks per wave */
-   constexpr int AP = TK + 16;   /* A panel pitch: a 64-bit read of 16 rows x 2 k is conflict-free */
-   constexpr int AS = 2 * MC * AP, XS = 2 * NT * (MC + 1), TS = 64 * (TK + 2);
-   constexpr int LD = AS + XS > TS ? AS + XS : TS;
-   /* main loop: As[2][MC][AP] and Xs[2][NT][MC+1]; epilogue: T[64][TK+2],
-    * one 64-column half of the output tile at a time */
-   __shared__ double lds[LD];
-   double (*As)[MC][AP] = reinterpret_cast<double (*)[MC][AP]>(lds);
-   double (*Xs)[NT][MC + 1] = reinterpret_cast<double (*)[NT][MC + 1]>(lds + AS);
-   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-   const int q = lane >> 4, ab = (lane >> 2) & 3, bb = lane & 3;
+   constexpr int WN = NT / 64, WK = 4 / WN;  /* waves along the columns and along K */
+   constexpr int BP = TK / WK / 32;          /* block pairs along K per wave */
+   constexpr int XP = MC + 2;                /* X pitch: 16-byte reads of 8 rows cover the banks once */
+   __shared__ __align__(16) double panels[2 * MC * TK + 2 * NT * XP];
+   double (*const As)[MC][TK] = reinterpret_cast<double (*)[MC][TK]>(panels);
+   double (*const Xs)[NT][XP] = reinterpret_cast<double (*)[NT][XP]>(panels + 2 * MC * TK);
+   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+   const int l16 = lane & 15, lq4 = lane >> 4;
    const int wk = wave % WK, wn = wave / WK;
-   const int s1 = rot_step(lane);
    /* block -> (K block, column tile) with the column tile fastest, remapped
     * so that the workgroups one XCD runs together (block id mod 8) hold
     * consecutive pairs: the column tiles of one K block then read its A
     * rows through the same L2 */
-   const int bid = blockIdx.x;
-   const int g = a.per > 0 ? (bid & 7) * a.per + (bid >> 3) : bid;
+   const int g = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+   if (g >= a.blocks) return;
    const size_t k0 = (size_t)(g / a.ntn) * TK;
    const int n0 = (g % a.ntn) * NT;
-   double acc[BI][BJ][4];   /* [K block][column block][rotation] */
+   mfma_d4 acc[BJ][BP][2];   /* [column block][K pair][even, odd K rows] */
 #pragma unroll
-   for (int i = 0; i < BI; ++i)
+   for (int j = 0; j < BJ; ++j)
+#pragma unroll
+      for (int p = 0; p < BP; ++p) acc[j][p][0] = acc[j][p][1] = mfma_d4{0.0, 0.0, 0.0, 0.0};
+
+   /* loaders: A chunk MC x TK, rows ar + 4 h with 64 lanes per 1 KB row; X
+    * chunk NT x MC.  No branches: rows past Mr repeat the last one with X = 0,
+    * columns past Nc repeat the last one and are not written. */
+   constexpr int XQ = NT * MC / 256;
+   static_assert(TK == 128 && MC == 16, "A loader covers 16 rows of 128");
+   const int ar = tid >> 6, ac = (tid & 63) * 2;
+   double2 ra[4];
+   double rx[XQ];
+   const char *const xbase = reinterpret_cast<const char *>(a.X);
+   unsigned xo[XQ];
+#pragma unroll
+   for (int u = 0; u < XQ; ++u) xo[u] = (unsigned)min(n0 + (tid + 256 * u) / MC, a.Nc - 1) * (unsigned)(a.ldx * 8);
+   const int xm = tid % MC, xp = (xm & 8) + 2 * (xm & 3) + ((xm >> 2) & 1);   /* m and m + 4 adjacent */
+   auto gload = [&](int m0) {
+      const char *const ab = reinterpret_cast<const char *>(a.A + (size_t)m0 * a.lda + k0);
+      const int last = a.Mr - 1 - m0;
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+         ra[h] = load2(ab, (unsigned)min(ar + 4 * h, last) * (unsigned)(a.lda * 8) + ac * 8);
+      const unsigned xr = (unsigned)(m0 + min(xm, last)) * (unsigned)(a.xsm * 8);
+#pragma unroll
+      for (int u = 0; u < XQ; ++u) rx[u] = *reinterpret_cast<const double *>(xbase + (xo[u] + xr));
+   };
+   auto lstore = [&](int bf, int m0) {
+#pragma unroll
+      for (int h = 0; h < 4; ++h) *reinterpret_cast<double2 *>(&As[bf][ar + 4 * h][ac]) = ra[h];
+#pragma unroll
+      for (int u = 0; u < XQ; ++u) Xs[bf][(tid + 256 * u) / MC][xp] = m0 + xm < a.Mr ? rx[u] : 0.0;
+   };
+   /* 8 of the chunk's rows m, in order: lane group lq4 supplies rows 8 ks +
+    * lq4 and 8 ks + 4 + lq4 to two successive instructions */
+   struct Frag { double2 x[BJ], b[BP][2]; };
+   auto fread = [&](Frag &f, int bf, int ks) {
+#pragma unroll
+      for (int j = 0; j < BJ; ++j)
+         f.x[j] = *reinterpret_cast<const double2 *>(&Xs[bf][64 * wn + 16 * j + l16][8 * ks + 2 * lq4]);
+#pragma unroll
+      for (int p = 0; p < BP; ++p)
+#pragma unroll
+         for (int u = 0; u < 2; ++u)
+            f.b[p][u] = *reinterpret_cast<const double2 *>(&As[bf][8 * ks + 4 * u + lq4][(TK / WK) * wk + 32 * p + 2 * l16]);
+   };
+   auto mma = [&](const Frag &f) {
 #pragma unroll
       for (int j = 0; j < BJ; ++j)
 #pragma unroll
-         for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0;
-
-   /* loaders: A chunk MC x TK, rows ar + 8 h with 64 lanes per 1 KB row (two
-    * 16-byte pieces per thread); X chunk NT x MC */
-   constexpr int XQ = NT * MC / 512;
-   static_assert(TK == 128 && MC == 16, "A loader covers 16 rows of 128");
-   const int ar = tid >> 6, ac = (tid & 63) * 2;
-   double2 ra[2];
-   double rx[XQ];
-   auto gload = [&](int m0) {
+         for (int p = 0; p < BP; ++p) {
+            acc[j][p][0] = mfma16(f.x[j].x, f.b[p][0].x, acc[j][p][0]);
+            acc[j][p][1] = mfma16(f.x[j].x, f.b[p][0].y, acc[j][p][1]);
+         }
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-         const int m = m0 + ar + 8 * h;
-         ra[h] = make_double2(0.0, 0.0);
-         if (m < a.Mr) ra[h] = *reinterpret_cast<const double2 *>(a.A + (size_t)m * a.lda + k0 + ac);
-      }
+      for (int j = 0; j < BJ; ++j)
 #pragma unroll
-      for (int u = 0; u < XQ; ++u) {
-         const int e = tid + 512 * u;
-         const int n = e / MC, mm = e % MC;
-         const int mg = m0 + mm, ng = n0 + n;
-         rx[u] = (mg < a.Mr && ng < a.Nc) ? a.X[(size_t)mg * a.xsm + (size_t)ng * a.ldx] : 0.0;
-      }
-   };
-   auto lstore = [&](int bf) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) *reinterpret_cast<double2 *>(&As[bf][ar + 8 * h][ac]) = ra[h];
-#pragma unroll
-      for (int u = 0; u < XQ; ++u) {
-         const int e = tid + 512 * u;
-         Xs[bf][e / MC][e % MC] = rx[u];
-      }
-   };
-   auto mma = [&](int bf, int ks) {
-      const int mm = 4 * ks + (lane >> 4);
-      double x[BJ];
-#pragma unroll
-      for (int j = 0; j < BJ; ++j) x[j] = Xs[bf][64 * wn + 16 * j + (lane & 15)][mm];
-#pragma unroll
-      for (int i = 0; i < BI; ++i) {
-         double b[4];
-         rotations(As[bf][mm][(TK / WK) * wk + 16 * i + (lane & 15)], b);
-#pragma unroll
-         for (int j = 0; j < BJ; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[i][j][r] = mfma4(x[j], b[r], acc[i][j][r]);
-      }
+         for (int p = 0; p < BP; ++p) {
+            acc[j][p][0] = mfma16(f.x[j].y, f.b[p][1].x, acc[j][p][0]);
+            acc[j][p][1] = mfma16(f.x[j].y, f.b[p][1].y, acc[j][p][1]);
+         }
    };
 
-   /* chunk c+1 waits in registers while chunk c is multiplied and is moved
-    * to the other LDS buffer halfway through, chunk c+2 requested right
-    * after: one barrier per chunk */
-   gload(0);
-   lstore(0);
-   __syncthreads();
-   if (MC < a.Mr) gload(MC);
-   int buf = 0;
-   for (int m0 = 0; m0 < a.Mr; m0 += MC) {
-#pragma unroll
-      for (int ks = 0; ks < MC / 8; ++ks) mma(buf, ks);
-      if (m0 + MC < a.Mr) {
-         lstore(buf ^ 1);
-         if (m0 + 2 * MC < a.Mr) gload(m0 + 2 * MC);
-      }
-#pragma unroll
-      for (int ks = MC / 8; ks < MC / 4; ++ks) mma(buf, ks);
+   /* chunk c+1 waits in registers while chunk c is multiplied; the operands of
+    * the next 8 rows are read from LDS between the current ones' MFMAs; one
+    * barrier per chunk, after which every read of the chunk has returned */
+   if (a.Mr > 0) {   /* an empty reduction (no projectors) leaves the product zero */
+      const int nc = (a.Mr + MC - 1) / MC;
+      gload(0);
+      lstore(0, 0);
+      gload(nc > 1 ? MC : 0);
       __syncthreads();
-      buf ^= 1;
+      Frag f0, f1;
+      fread(f0, 0, 0);
+      int buf = 0;
+      for (int c = 0; c + 1 < nc; ++c) {
+         fread(f1, buf, 1);
+         mma(f0);
+         lstore(buf ^ 1, (c + 1) * MC);
+         sched_mix<0x100, BJ + 2 * BP, 1>();
+         sched_mix<0x200, 4 + XQ, 1>();
+         __syncthreads();
+         buf ^= 1;
+         fread(f0, buf, 0);
+         gload(min(c + 2, nc - 1) * MC);
+         mma(f1);
+         sched_mix<0x100, BJ + 2 * BP, 1>();
+         sched_mix<0x20, 4 + XQ, 1>();
+      }
+      fread(f1, buf, 1);
+      mma(f0);
+      mma(f1);
    }
 
-   /* epilogue per 64-column half: the half's waves stage their tile in LDS,
-    * then all waves apply the update along whole 1 KB rows */
-   double (*T)[TK + 2] = reinterpret_cast<double (*)[TK + 2]>(lds);
+   /* epilogue: register r of block (j, p) is row n of the output at complex
+    * coefficient (k0 + 32 p') / 2 + l16; the loads of a block pair are issued
+    * before its stores */
+   const size_t kw = k0 + (TK / WK) * wk + 2 * l16;
+   if constexpr (EPI == EPI_NLFORCE) {
+      /* Z_n(G) against the projectors (ccpsdv3/cpsd.c:296-302 with the orbital
+       * sum moved inside): 32 columns at a time staged in LDS, then a wave
+       * per row with a lane per G and the wave's fixed shuffle tree */
+      double (*T)[TK + 2] = reinterpret_cast<double (*)[TK + 2]>(panels);
+      static_assert(32 * (TK + 2) <= 2 * MC * TK + 2 * NT * XP, "staging fits the panels");
 #pragma unroll
-   for (int half = 0; half < WN; ++half) {
-      if (half > 0) __syncthreads();
-      if (wn == half) {
+      for (int half = 0; half < NT / 32; ++half) {
+         __syncthreads();
+         if (wn == half >> 1) {
 #pragma unroll
-         for (int i = 0; i < BI; ++i)
+            for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
-            for (int j = 0; j < BJ; ++j)
+               for (int p = 0; p < BP; ++p)
 #pragma unroll
-               for (int r = 0; r < 4; ++r)
-                  T[16 * j + 4 * ab + q][(TK / WK) * wk + 16 * i + 4 * ((ab + s1 * r) & 3) + bb] =
-                     acc[i][j][r];
-      }
-      __syncthreads();
-      constexpr int EU = EPI == EPI_NLFORCE ? 1 : 2;   /* the force reduction does not unroll */
-#pragma unroll EU
-      for (int nl = wave; nl < 64; nl += 8) {
-         const int n = n0 + 64 * half + nl;
-         if (n >= a.Nc) break;
-         const size_t idx = (size_t)n * a.ldc + k0 + 2 * lane;
-         const double2 v = make_double2(T[nl][2 * lane], T[nl][2 * lane + 1]);
-         if (EPI == EPI_KBAPPLY) {
-            double2 cp = *reinterpret_cast<const double2 *>(a.CP + idx);
-            const double2 c1 = *reinterpret_cast<const double2 *>(a.C1 + idx);
-            cp.x += v.x; cp.y += v.y;
-            *reinterpret_cast<double2 *>(a.C2 + idx) = make_double2(c1.x + a.dte * cp.x, c1.y + a.dte * cp.y);
-            if (a.write_cp) *reinterpret_cast<double2 *>(a.CP + idx) = cp;
-         } else if (EPI == EPI_CONSTRAINT) {
-            double2 c2 = *reinterpret_cast<const double2 *>(a.C2 + idx);
-            c2.x += a.dte * v.x; c2.y += a.dte * v.y;
-            *reinterpret_cast<double2 *>(a.C2 + idx) = c2;
-         } else if (EPI == EPI_STORE) {
-            *reinterpret_cast<double2 *>(a.C2 + idx) = v;
-         } else if (EPI == EPI_PRECOND) {
-            const double2 c1 = *reinterpret_cast<const double2 *>(a.C1 + idx);
-            double2 c2 = *reinterpret_cast<const double2 *>(a.C2 + idx);
-            const double f = a.Kp[(k0 >> 1) + lane];
-            c2.x = c1.x + f * (c2.x - c1.x + a.dte * v.x);
-            c2.y = c1.y + f * (c2.y - c1.y + a.dte * v.y);
-            *reinterpret_cast<double2 *>(a.C2 + idx) = c2;
-         } else {
-            /* lane holds Z_n(G) for G = k0/2 + lane (ccpsdv3/cpsd.c:296-302 with
-             * the orbital sum moved inside) */
-            const size_t g = (k0 >> 1) + lane;
-            const double2 b = a.Bp[(size_t)n * a.ngp + g];
+                  for (int r = 0; r < 4; ++r) {
+                     const int j = 2 * (half & 1) + jj;
+                     *reinterpret_cast<double2 *>(&T[16 * jj + mfma16_row(r, lane)][(TK / WK) * wk + 32 * p + 2 * l16]) =
+                        make_double2(acc[j][p][0][r], acc[j][p][1][r]);
+                  }
+         }
+         __syncthreads();
+         for (int nl = wave; nl < 32; nl += 4) {
+            const int n = n0 + 32 * half + nl;
+            if (n >= a.Nc) break;
+            const double2 v = make_double2(T[nl][2 * lane], T[nl][2 * lane + 1]);
+            const size_t gq = (k0 >> 1) + lane;
+            const double2 b = a.Bp[(size_t)n * a.ngp + gq];
             const double t = a.w[k0 + 2 * lane] * (v.y * b.x - v.x * b.y);
-            const double f0 = wave_sum(a.Gp[g] * t);
-            const double f1 = wave_sum(a.Gp[(size_t)a.ngp + g] * t);
-            const double f2 = wave_sum(a.Gp[2 * (size_t)a.ngp + g] * t);
+            const double f0 = wave_sum(a.Gp[gq] * t);
+            const double f1 = wave_sum(a.Gp[(size_t)a.ngp + gq] * t);
+            const double f2 = wave_sum(a.Gp[2 * (size_t)a.ngp + gq] * t);
             if (lane == 0) {
                double *o = a.fpart + ((size_t)(k0 / TK) * a.Nc + n) * 3;
                o[0] = f0; o[1] = f1; o[2] = f2;
             }
          }
       }
+   } else {
+#pragma unroll
+      for (int p = 0; p < BP; ++p) {
+         const size_t kc = kw + 32 * p;
+         double f = 0.0;
+         if (EPI == EPI_PRECOND) f = a.Kp[kc >> 1];
+#pragma unroll
+         for (int j = 0; j < BJ; ++j) {
+            double2 c2[4], c1[4], cp[4];
+            size_t idx[4];
+            bool in[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+               const int n = n0 + 64 * wn + 16 * j + mfma16_row(r, lane);
+               in[r] = n < a.Nc;
+               idx[r] = (size_t)min(n, a.Nc - 1) * a.ldc + kc;   /* columns past Nc load the last one */
+               if (EPI == EPI_CONSTRAINT || EPI == EPI_PRECOND) c2[r] = *reinterpret_cast<const double2 *>(a.C2 + idx[r]);
+               if (EPI == EPI_KBAPPLY || EPI == EPI_PRECOND) c1[r] = *reinterpret_cast<const double2 *>(a.C1 + idx[r]);
+               if (EPI == EPI_KBAPPLY) cp[r] = *reinterpret_cast<const double2 *>(a.CP + idx[r]);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+               if (!in[r]) continue;
+               const double2 v = make_double2(acc[j][p][0][r], acc[j][p][1][r]);
+               double2 o = v;
+               if (EPI == EPI_KBAPPLY) {
+                  cp[r].x += v.x; cp[r].y += v.y;
+                  o = make_double2(c1[r].x + a.dte * cp[r].x, c1[r].y + a.dte * cp[r].y);
+                  if (a.write_cp) *reinterpret_cast<double2 *>(a.CP + idx[r]) = cp[r];
+               } else if (EPI == EPI_CONSTRAINT) {
+                  o = make_double2(c2[r].x + a.dte * v.x, c2[r].y + a.dte * v.y);
+               } else if (EPI == EPI_PRECOND) {
+                  o.x = c1[r].x + f * (c2[r].x - c1[r].x + a.dte * v.x);
+                  o.y = c1[r].y + f * (c2[r].y - c1[r].y + a.dte * v.y);
+               }
+               *reinterpret_cast<double2 *>(a.C2 + idx[r]) = o;
+            }
+         }
+      }
    }
+}
+
+template<int NT>
+static void gemm_tall_go(int epi, TallArgs &a, hipStream_t s)
+{
+   a.ntn = (a.Nc + NT - 1) / NT;
+   a.blocks = (int)(a.K / TK) * a.ntn;
+   const dim3 g = xcd_grid(a.blocks), t(256);
+   if (epi == EPI_KBAPPLY) hipLaunchKernelGGL((k_gemm_tall<EPI_KBAPPLY, NT>), g, t, 0, s, a);
+   else if (epi == EPI_CONSTRAINT) hipLaunchKernelGGL((k_gemm_tall<EPI_CONSTRAINT, NT>), g, t, 0, s, a);
+   else if (epi == EPI_STORE) hipLaunchKernelGGL((k_gemm_tall<EPI_STORE, NT>), g, t, 0, s, a);
+   else if (epi == EPI_PRECOND) hipLaunchKernelGGL((k_gemm_tall<EPI_PRECOND, NT>), g, t, 0, s, a);
+   else hipLaunchKernelGGL((k_gemm_tall<EPI_NLFORCE, NT>), g, t, 0, s, a);
 }
 
 int launch_gemm_tall(int epi, const TallArgs &args, hipStream_t s)
 {
    if (args.K % TK) { cpsd_set_error("gemm_tall: K=%zu not a multiple of %d", args.K, TK); return -1; }
+   /* 32-bit lane offsets of the MC rows of a chunk */
+   if (args.lda * 8 * MC >= (1ull << 32)) { cpsd_set_error("gemm_tall: rows of %zu doubles", args.lda); return -1; }
    TallArgs a = args;
-   a.ntn = (a.Nc + 63) / 64;
-   const long blocks = (long)(a.K / TK) * a.ntn;
-   a.per = blocks % 8 == 0 ? (int)(blocks / 8) : 0;
-   if (epi == EPI_KBAPPLY) hipLaunchKernelGGL((k_gemm_tall<EPI_KBAPPLY, 64>), dim3((unsigned)blocks), dim3(512), 0, s, a);
-   else if (epi == EPI_CONSTRAINT) hipLaunchKernelGGL((k_gemm_tall<EPI_CONSTRAINT, 64>), dim3((unsigned)blocks), dim3(512), 0, s, a);
-   else if (epi == EPI_STORE) hipLaunchKernelGGL((k_gemm_tall<EPI_STORE, 64>), dim3((unsigned)blocks), dim3(512), 0, s, a);
-   else if (epi == EPI_PRECOND) hipLaunchKernelGGL((k_gemm_tall<EPI_PRECOND, 64>), dim3((unsigned)blocks), dim3(512), 0, s, a);
-   else hipLaunchKernelGGL((k_gemm_tall<EPI_NLFORCE, 64>), dim3((unsigned)blocks), dim3(512), 0, s, a);
+   /* 128 columns per workgroup read A and X half as often as 64; 64 where
+    * they pad less */
+   if ((a.Nc + 127) / 128 * 2 == (a.Nc + 63) / 64) gemm_tall_go<128>(epi, a, s);
+   else gemm_tall_go<64>(epi, a, s);
    CPSD_CHECK(hipGetLastError());
    return 0;
 }

@@ -430,31 +430,24 @@ __global__ void k_precond_lmd(double *__restrict__ lmd, const double *__restrict
 
 /* ------------------------------------------ 16 x 16 tiles on the MFMA */
 
-/* acc += P Q over k in [kb, kb + 4n) for a 16 x 16 tile on the FP64 4x4x4
- * MFMA (mfma64.h); Pr[i][k] = P(i, k) and Qc[j][k] = Q(k, j) in LDS.  The
- * result lands in the rotated layout that tile16_reduce undoes. */
+/* acc += P Q over k in [kb, kb + 4n) for a 16 x 16 tile on the FP64 MFMA
+ * (mfma64.h); Pr[i][k] = P(i, k) and Qc[j][k] = Q(k, j) in LDS */
 template<int LP>
-__device__ __forceinline__ void tile16_mfma(double (*Pr)[LP], double (*Qc)[LP], int kb, int ke, int lane,
-                                            double (&acc)[4])
+__device__ __forceinline__ void tile16_mfma(double (*Pr)[LP], double (*Qc)[LP], int kb, int ke, int lane, mfma_d4 &acc)
 {
    for (int m0 = kb; m0 < ke; m0 += 4) {
       const int m = m0 + (lane >> 4);
-      const double pa = Pr[lane & 15][m];
-      double bq[4];
-      rotations(Qc[lane & 15][m], bq);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) acc[t] = mfma4(pa, bq[t], acc[t]);
+      acc = mfma16(Pr[lane & 15][m], Qc[lane & 15][m], acc);
    }
 }
 
 /* the four waves' partial tiles (each over a quarter of K) added in wave
  * order at element (rl, cl) of the tile; all 256 threads call it */
-__device__ __forceinline__ double tile16_reduce(double (*part)[16][17], const double (&acc)[4], int wave, int lane,
-                                                int s1, int rl, int cl)
+__device__ __forceinline__ double tile16_reduce(double (*part)[16][17], const mfma_d4 &acc, int wave, int lane, int rl,
+                                                int cl)
 {
-   const int q = lane >> 4, ab = (lane >> 2) & 3, bb = lane & 3;
 #pragma unroll
-   for (int t = 0; t < 4; ++t) part[wave][4 * ab + q][4 * ((ab + s1 * t) & 3) + bb] = acc[t];
+   for (int t = 0; t < 4; ++t) part[wave][mfma16_row(t, lane)][lane & 15] = acc[t];
    __syncthreads();
    const double v = ((part[0][rl][cl] + part[1][rl][cl]) + part[2][rl][cl]) + part[3][rl][cl];
    __syncthreads();
@@ -480,7 +473,6 @@ __global__ void __launch_bounds__(256) k_gram_next_w_mf(const double *__restrict
    const int ti = blockIdx.x % nt, tj = blockIdx.x / nt;
    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
    const int kp = (ne + 15) & ~15, kq = kp / 4, kb = wave * kq, ke = kb + kq;
-   const int s1 = rot_step(lane);
    const int n2 = 2 * ne, o1 = c1_second ? ne : 0, o2 = c1_second ? 0 : ne;
    const double *gb = g11c ? g11c : Gm + (size_t)o1 * n2 + o1;
    const size_t gld = g11c ? (size_t)ne : (size_t)n2;
@@ -510,12 +502,12 @@ __global__ void __launch_bounds__(256) k_gram_next_w_mf(const double *__restrict
       if (x % NM < kp) lmc[x / NM][x % NM] = vl[u];
    }
    __syncthreads();
-   double aw[4] = {0.0, 0.0, 0.0, 0.0}, at[4] = {0.0, 0.0, 0.0, 0.0};
+   mfma_d4 aw = {0.0, 0.0, 0.0, 0.0}, at = {0.0, 0.0, 0.0, 0.0};
    tile16_mfma<P>(g11r, lmc, kb, ke, lane, aw);
    tile16_mfma<P>(g21r, lmc, kb, ke, lane, at);
    const int rl = tid % TS, cl = tid / TS, i = ti * TS + rl, b = tj * TS + cl;
-   const double w = tile16_reduce(part, aw, wave, lane, s1, rl, cl);
-   const double t = tile16_reduce(part, at, wave, lane, s1, rl, cl);
+   const double w = tile16_reduce(part, aw, wave, lane, rl, cl);
+   const double t = tile16_reduce(part, at, wave, lane, rl, cl);
    if (i < ne && b < ne) {
       W[(size_t)i * ne + b] = w;
       T1[(size_t)i * ne + b] = t;
@@ -776,11 +768,11 @@ __global__ void __launch_bounds__(256) k_lagrange(LagArgs a)
  * the st1 panel, i.e. two round trips to L2 and two grid barriers per
  * iteration (the general kernel above makes one round trip per 32-wide K
  * chunk of each of its four products).  The tile products run on the FP64
- * 4x4x4 MFMA (mfma64.h): the four waves take a quarter of K each and their
+ * MFMA (mfma64.h): the four waves take a quarter of K each and their
  * 16 x 16 partial tiles are added in wave order, so results do not depend on
  * timing.  Matrices are column-major: M(r, c) = M[r + c*ne]. */
 template<int NM>
-__global__ void __launch_bounds__(256) k_lagrange_res(LagArgs a)
+__global__ void __launch_bounds__(256, 2) k_lagrange_res(LagArgs a)
 {
    constexpr int TS = 16;
    constexpr int P = NM + 2;   /* row pitch: a 64-bit read of 16 rows x 2 k hits distinct banks */
@@ -800,7 +792,6 @@ __global__ void __launch_bounds__(256) k_lagrange_res(LagArgs a)
    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
    /* K padded to whole 4-wide steps for each of the four waves */
    const int kp = (ne + 15) & ~15, kq = kp / 4, kb = wave * kq, ke = kb + kq;
-   const int s1 = rot_step(lane);
    /* this thread's element of the tile */
    const int rl = tid % TS, cl = tid / TS, r = ti * TS + rl, c = tj * TS + cl;
    const bool mine = r < ne && c < ne;
@@ -840,10 +831,10 @@ __global__ void __launch_bounds__(256) k_lagrange_res(LagArgs a)
       }
    };
    /* acc += P Q over this wave's K quarter; the four waves' tiles summed */
-   auto tile = [&](double (*Pr)[P], double (*Qc)[P], double (&acc)[4]) {
+   auto tile = [&](double (*Pr)[P], double (*Qc)[P], mfma_d4 &acc) {
       tile16_mfma<P>(Pr, Qc, kb, ke, lane, acc);
    };
-   auto reduce = [&](const double (&acc)[4]) { return tile16_reduce(part, acc, wave, lane, s1, rl, cl); };
+   auto reduce = [&](const mfma_d4 &acc) { return tile16_reduce(part, acc, wave, lane, rl, cl); };
 
    /* K padding read by the MFMA steps stays zero: the loads write k < ne only */
    for (int x = tid; x < 6 * TS * (kp - ne); x += 256) {
@@ -868,7 +859,7 @@ __global__ void __launch_bounds__(256) k_lagrange_res(LagArgs a)
       load_rows(X, xr);
       __syncthreads();
       /* st1 = s11 X */
-      double acc[4] = {0.0, 0.0, 0.0, 0.0};
+      mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
       tile(s11r, xc, acc);
       const double st = reduce(acc);
       if (mine) a.st1[e] = st;
@@ -876,7 +867,7 @@ __global__ void __launch_bounds__(256) k_lagrange_res(LagArgs a)
       load_cols(a.st1, stc);
       __syncthreads();
       /* X_new = s22 + s21 X + X s12 + X st1 */
-      acc[0] = acc[1] = acc[2] = acc[3] = 0.0;
+      acc = mfma_d4{0.0, 0.0, 0.0, 0.0};
       tile(s21r, xc, acc);
       tile(xr, s12c, acc);
       tile(xr, stc, acc);
@@ -917,16 +908,12 @@ __global__ void __launch_bounds__(256) k_lagrange_res(LagArgs a)
  * which then fall on 16 distinct bank pairs. */
 template<int LP>
 __device__ __forceinline__ void tile16_mfma_swz(double (*Pr)[LP], double (*Qc)[LP], int kb, int ke, int lane,
-                                                double (&acc)[4])
+                                                mfma_d4 &acc)
 {
    const int sw = lane & 15;
    for (int m0 = kb; m0 < ke; m0 += 4) {
       const int m = (m0 + (lane >> 4)) ^ sw;
-      const double pa = Pr[sw][m];
-      double bq[4];
-      rotations(Qc[sw][m], bq);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) acc[t] = mfma4(pa, bq[t], acc[t]);
+      acc = mfma16(Pr[sw][m], Qc[sw][m], acc);
    }
 }
 
@@ -946,7 +933,6 @@ __global__ void __launch_bounds__(256) k_lagrange_str(LagArgs a)
    const size_t nn = (size_t)ne * ne;
    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
    const int kp = (ne + 15) & ~15, kq = kp / 4, kb = wave * kq, ke = kb + kq;
-   const int s1 = rot_step(lane);
    const int rl = tid % TS, cl = tid / TS, r = ti * TS + rl, c = tj * TS + cl;
    const bool mine = r < ne && c < ne;
    const size_t e = r + (size_t)c * ne;
@@ -984,10 +970,10 @@ __global__ void __launch_bounds__(256) k_lagrange_str(LagArgs a)
          if (k < ne) Cp[cc][k ^ cc] = v[u];
       }
    };
-   auto tile = [&](double (*Pr)[NM], double (*Qc)[NM], double (&acc)[4]) {
+   auto tile = [&](double (*Pr)[NM], double (*Qc)[NM], mfma_d4 &acc) {
       tile16_mfma_swz<NM>(Pr, Qc, kb, ke, lane, acc);
    };
-   auto reduce = [&](const double (&acc)[4]) { return tile16_reduce(part, acc, wave, lane, s1, rl, cl); };
+   auto reduce = [&](const mfma_d4 &acc) { return tile16_reduce(part, acc, wave, lane, rl, cl); };
 
    /* the K padding k in [ne, kp) of every slot stays zero (the loads write
     * k < ne only; the swizzle keeps each 16-wide block of k in place) */
@@ -1010,7 +996,7 @@ __global__ void __launch_bounds__(256) k_lagrange_str(LagArgs a)
       load_rows(a.s11, slA);
       load_cols(X, slB);
       __syncthreads();
-      double acc[4] = {0.0, 0.0, 0.0, 0.0};
+      mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
       tile(slA, slB, acc);
       const double st = reduce(acc);
       if (mine) a.st1[e] = st;
@@ -1018,7 +1004,7 @@ __global__ void __launch_bounds__(256) k_lagrange_str(LagArgs a)
       /* X_new = s22 + s21 X + X s12 + X st1 */
       load_rows(a.s21, slA);
       __syncthreads();
-      acc[0] = acc[1] = acc[2] = acc[3] = 0.0;
+      acc = mfma_d4{0.0, 0.0, 0.0, 0.0};
       tile(slA, slB, acc);
       __syncthreads();
       load_rows(X, slA);
