@@ -62,98 +62,228 @@ __device__ __forceinline__ void mlp_forward(const float *P, const float *x, floa
    y = o;
 }
 
-/* One pass over the samples: the loss and its gradient.  Workgroup w takes
- * chunks w, w + grid, ... of TB samples; thread t owns the gradient entries
- * q = t, t + TB, ... and sums them over the workgroup's chunks in order;
- * gpart[w][q] and lpart[w] are the workgroup's partial sums. */
-__global__ void __launch_bounds__(TB) k_mlp_loss_grad(const float *X, const float *A, const float *B, long n,
-                                                      const float *Pg, float *gpart, float *lpart)
+typedef float mfma_f4 __attribute__((ext_vector_type(4)));
+
+/* v_mfma_f32_16x16x4_f32: A lane l = A[l%16][l/16], B lane l = B[l/16][l%16],
+ * D register r of lane l = D[4 (l/16) + r][l%16].  Each element adds its four
+ * products to C by fused multiply-adds in the order of k (measured bit for
+ * bit), so these sums are the sequential fmaf chains over increasing k. */
+__device__ __forceinline__ mfma_f4 mfma_f32(float a, float b, mfma_f4 c)
 {
-   __shared__ float P[MLP_NP];
+   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+#define LP (MLP_NH + 1)   /* pitch of the activation rows */
+
+/* One pass over the samples: the loss and its gradient.  Workgroup w takes
+ * chunks w, w + grid, ... of TB samples; the gradient entries of a chunk are
+ * sums over its samples in order, added to the workgroup's running sums chunk
+ * by chunk; gpart[w][q] and lpart[w] are the workgroup's partial sums.
+ *
+ * The layers, the backward products and the weight gradients (activations
+ * transposed times errors, k = sample) are FP32 MFMA tiles: a wave's 64
+ * samples are four 16-row blocks, its activations stay in the D layout for
+ * the elementwise steps and pass through two LDS arrays (h1, then z1; h2, then
+ * z2) as operands.  36 KB of LDS hold the 1024 workgroups of a full grid at
+ * once, four per CU.  Bound by the 64 tanhf per sample.  At 234980 samples
+ * 44 us per pass; the form with a thread per sample and a thread per
+ * gradient entry (two workgroups of two waves per CU, two LDS reads per FMA)
+ * took 302 us. */
+__global__ void __launch_bounds__(TB, 2) k_mlp_loss_grad(const float *__restrict__ X, const float *__restrict__ A,
+                                                         const float *__restrict__ B, long n,
+                                                         const float *__restrict__ P, float *__restrict__ gpart,
+                                                         float *__restrict__ lpart)
+{
+   __shared__ float s0[TB][LP], s1[TB][LP];
    __shared__ float sx[TB][MLP_NF];
-   __shared__ float sh1[TB][MLP_NH + 1], sh2[TB][MLP_NH + 1];
-   __shared__ float sz1[TB][MLP_NH + 1], sz2[TB][MLP_NH + 1];
    __shared__ float sdy[TB];
    __shared__ float sl[TB];
-   const int t = threadIdx.x;
-   for (int q = t; q < MLP_NP; q += TB) P[q] = Pg[q];
-   constexpr int QPT = (MLP_NP + TB - 1) / TB;
-   float g[QPT];
+   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+   const int l16 = lane & 15, q4 = lane >> 4, r0 = 64 * wv;
+   constexpr int RB = 4, JB = MLP_NH / 16, KS = MLP_NH / 4;
+   /* weights as MFMA operands: W1 and W2 (inputs x outputs), W2 transposed */
+   float w1[JB], b1[JB], b2[JB], w3[JB], w2[JB][KS], w2t[JB][KS];
 #pragma unroll
-   for (int u = 0; u < QPT; ++u) g[u] = 0.f;
-   float lsum = 0.f;
-   __syncthreads();
+   for (int j = 0; j < JB; ++j) {
+      w1[j] = P[OFF_W1 + q4 * MLP_NH + 16 * j + l16];
+      b1[j] = P[OFF_B1 + 16 * j + l16];
+      b2[j] = P[OFF_B2 + 16 * j + l16];
+      w3[j] = P[OFF_W3 + 16 * j + l16];
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+         w2[j][s] = P[OFF_W2 + (4 * s + q4) * MLP_NH + 16 * j + l16];
+         w2t[j][s] = P[OFF_W2 + (16 * j + l16) * MLP_NH + 4 * s + q4];
+      }
+   }
+   /* running sums: W2 rows 16 wv.., W1 and b1 columns 16 wv.., and one of
+    * w3 (wave 0, lanes 0-31), b3 (wave 0, lane 32), b2 (wave 1, lanes 0-31) */
+   mfma_f4 g2[JB], g1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+   for (int j = 0; j < JB; ++j) g2[j] = mfma_f4{0.f, 0.f, 0.f, 0.f};
+   float gv = 0.f, lsum = 0.f;
    const long nchunk = (n + TB - 1) / TB;
    for (long ch = blockIdx.x; ch < nchunk; ch += gridDim.x) {
       const long i = ch * TB + t;
-      float x[MLP_NF], h1[MLP_NH], h2[MLP_NH], y = 0.f;
       float a = 0.f, b = 0.f;
       if (i < n) {
-#pragma unroll
-         for (int f = 0; f < MLP_NF; ++f) x[f] = X[i * MLP_NF + f];
          a = A[i];
          b = B[i];
-      } else {
-#pragma unroll
-         for (int f = 0; f < MLP_NF; ++f) x[f] = 0.f;
       }
-      mlp_forward(P, x, h1, h2, y);
-      const float K = expf(fminf(y, YMAX));
-      /* dL/dy = 2 K (A K - B); zero above YMAX, where K is held constant */
-      float dy = (y < YMAX) ? 2.f * K * (a * K - b) : 0.f;
-      float l = a * K * K - 2.f * b * K;
-      if (i >= n) { dy = 0.f; l = 0.f; }
-      lsum += l;
-      float z2[MLP_NH];
+      /* layer 1 */
+      mfma_f4 h1[RB][JB], h2[RB][JB];
+      float x[RB];
 #pragma unroll
-      for (int j = 0; j < MLP_NH; ++j) z2[j] = dy * P[OFF_W3 + j] * (1.f - h2[j] * h2[j]);
-#pragma unroll
-      for (int i1 = 0; i1 < MLP_NH; ++i1) {
-         float s = 0.f;
-#pragma unroll
-         for (int j = 0; j < MLP_NH; ++j) s = fmaf(z2[j], P[OFF_W2 + i1 * MLP_NH + j], s);
-         sz1[t][i1] = s * (1.f - h1[i1] * h1[i1]);
-         sh1[t][i1] = h1[i1];
-         sh2[t][i1] = h2[i1];
-         sz2[t][i1] = z2[i1];
+      for (int u = 0; u < RB; ++u) {
+         const long ix = ch * TB + r0 + 16 * u + l16;
+         x[u] = ix < n ? X[ix * MLP_NF + q4] : 0.f;
       }
 #pragma unroll
-      for (int f = 0; f < MLP_NF; ++f) sx[t][f] = x[f];
-      sdy[t] = dy;
+      for (int u = 0; u < RB; ++u) {
+         sx[r0 + 16 * u + l16][q4] = x[u];
+#pragma unroll
+         for (int j = 0; j < JB; ++j) {
+            mfma_f4 c = {b1[j], b1[j], b1[j], b1[j]};
+            c = mfma_f32(x[u], w1[j], c);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+               c[r] = tanhf(c[r]);
+               s0[r0 + 16 * u + 4 * q4 + r][16 * j + l16] = c[r];
+            }
+            h1[u][j] = c;
+         }
+      }
       __syncthreads();
-      /* this chunk's contribution to the entries the thread owns */
+      /* layer 2 */
 #pragma unroll
-      for (int u = 0; u < QPT; ++u) {
-         const int q = t + TB * u;
-         if (q >= MLP_NP) break;
+      for (int u = 0; u < RB; ++u) {
+#pragma unroll
+         for (int j = 0; j < JB; ++j) h2[u][j] = mfma_f4{b2[j], b2[j], b2[j], b2[j]};
+#pragma unroll
+         for (int s = 0; s < KS; ++s) {
+            const float h = s0[r0 + 16 * u + l16][4 * s + q4];
+#pragma unroll
+            for (int j = 0; j < JB; ++j) h2[u][j] = mfma_f32(h, w2[j][s], h2[u][j]);
+         }
+#pragma unroll
+         for (int j = 0; j < JB; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+               h2[u][j][r] = tanhf(h2[u][j][r]);
+               s1[r0 + 16 * u + 4 * q4 + r][16 * j + l16] = h2[u][j][r];
+            }
+      }
+      __syncthreads();
+      /* output, loss and its derivative of sample t */
+      float y = P[OFF_B3];
+#pragma unroll
+      for (int j = 0; j < MLP_NH; ++j) y = fmaf(s1[t][j], P[OFF_W3 + j], y);
+      {
+         const float K = expf(fminf(y, YMAX));
+         /* dL/dy = 2 K (A K - B); zero above YMAX, where K is held constant */
+         float dy = (y < YMAX) ? 2.f * K * (a * K - b) : 0.f;
+         float l = a * K * K - 2.f * b * K;
+         if (i >= n) { dy = 0.f; l = 0.f; }
+         lsum += l;
+         sdy[t] = dy;
+      }
+      __syncthreads();
+      /* w3 and b3 */
+      if (wv == 0) {
          float s = 0.f;
-         if (q < OFF_B1) {
-            const int f = q / MLP_NH, j = q % MLP_NH;
-            for (int r = 0; r < TB; ++r) s = fmaf(sx[r][f], sz1[r][j], s);
-         } else if (q < OFF_W2) {
-            const int j = q - OFF_B1;
-            for (int r = 0; r < TB; ++r) s += sz1[r][j];
-         } else if (q < OFF_B2) {
-            const int i1 = (q - OFF_W2) / MLP_NH, j = (q - OFF_W2) % MLP_NH;
-            for (int r = 0; r < TB; ++r) s = fmaf(sh1[r][i1], sz2[r][j], s);
-         } else if (q < OFF_W3) {
-            const int j = q - OFF_B2;
-            for (int r = 0; r < TB; ++r) s += sz2[r][j];
-         } else if (q < OFF_B3) {
-            const int j = q - OFF_W3;
-            for (int r = 0; r < TB; ++r) s = fmaf(sh2[r][j], sdy[r], s);
-         } else {
+         if (lane < MLP_NH) {
+#pragma unroll 16
+            for (int r = 0; r < TB; ++r) s = fmaf(s1[r][lane], sdy[r], s);
+         } else if (lane == MLP_NH) {
+#pragma unroll 16
             for (int r = 0; r < TB; ++r) s += sdy[r];
          }
-         g[u] += s;
+         gv += s;
+      }
+      __syncthreads();
+      /* errors of layer 2, over h2 */
+#pragma unroll
+      for (int u = 0; u < RB; ++u)
+#pragma unroll
+         for (int r = 0; r < 4; ++r) {
+            const float dy = sdy[r0 + 16 * u + 4 * q4 + r];
+#pragma unroll
+            for (int j = 0; j < JB; ++j) {
+               const float hv = h2[u][j][r];
+               s1[r0 + 16 * u + 4 * q4 + r][16 * j + l16] = dy * w3[j] * (1.f - hv * hv);
+            }
+         }
+      __syncthreads();
+      /* W2 rows 16 wv.. (k = sample) */
+      {
+         mfma_f4 s[JB];
+#pragma unroll
+         for (int j = 0; j < JB; ++j) s[j] = mfma_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+         for (int k = 0; k < TB / 4; ++k) {
+            const float h = s0[4 * k + q4][16 * wv + l16];
+#pragma unroll
+            for (int j = 0; j < JB; ++j) s[j] = mfma_f32(h, s1[4 * k + q4][16 * j + l16], s[j]);
+         }
+#pragma unroll
+         for (int j = 0; j < JB; ++j) g2[j] += s[j];
+      }
+      if (wv == 1 && lane < MLP_NH) {
+         float s = 0.f;
+#pragma unroll 16
+         for (int r = 0; r < TB; ++r) s += s1[r][lane];
+         gv += s;
+      }
+      /* errors of layer 1 */
+#pragma unroll
+      for (int u = 0; u < RB; ++u) {
+         mfma_f4 z[JB];
+#pragma unroll
+         for (int j = 0; j < JB; ++j) z[j] = mfma_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+         for (int s = 0; s < KS; ++s) {
+            const float v = s1[r0 + 16 * u + l16][4 * s + q4];
+#pragma unroll
+            for (int j = 0; j < JB; ++j) z[j] = mfma_f32(v, w2t[j][s], z[j]);
+         }
+#pragma unroll
+         for (int j = 0; j < JB; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+               const float hv = h1[u][j][r];
+               h1[u][j][r] = z[j][r] * (1.f - hv * hv);
+            }
+      }
+      __syncthreads();   /* every read of h1 in s0 is done */
+#pragma unroll
+      for (int u = 0; u < RB; ++u)
+#pragma unroll
+         for (int j = 0; j < JB; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s0[r0 + 16 * u + 4 * q4 + r][16 * j + l16] = h1[u][j][r];
+      __syncthreads();
+      /* W1 and b1, columns 16 wv..: rows 0-3 the features, row 4 ones */
+      {
+         mfma_f4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+         for (int k = 0; k < TB / 4; ++k) {
+            const float v = l16 < MLP_NF ? sx[4 * k + q4][l16 & 3] : (l16 == MLP_NF ? 1.f : 0.f);
+            s = mfma_f32(v, s0[4 * k + q4][16 * wv + l16], s);
+         }
+         g1 += s;
       }
       __syncthreads();
    }
+   float *gp = gpart + (size_t)blockIdx.x * MLP_NP;
 #pragma unroll
-   for (int u = 0; u < QPT; ++u) {
-      const int q = t + TB * u;
-      if (q < MLP_NP) gpart[(size_t)blockIdx.x * MLP_NP + q] = g[u];
+   for (int r = 0; r < 4; ++r) {
+#pragma unroll
+      for (int j = 0; j < JB; ++j) gp[OFF_W2 + (16 * wv + 4 * q4 + r) * MLP_NH + 16 * j + l16] = g2[j][r];
+      if (q4 == 0) gp[OFF_W1 + r * MLP_NH + 16 * wv + l16] = g1[r];
    }
+   if (q4 == 1) gp[OFF_B1 + 16 * wv + l16] = g1[0];
+   if (wv == 0 && lane < MLP_NH) gp[OFF_W3 + lane] = gv;
+   if (wv == 0 && lane == MLP_NH) gp[OFF_B3] = gv;
+   if (wv == 1 && lane < MLP_NH) gp[OFF_B2 + lane] = gv;
    /* workgroup loss: fixed tree over the threads */
    sl[t] = lsum;
    __syncthreads();
@@ -164,36 +294,56 @@ __global__ void __launch_bounds__(TB) k_mlp_loss_grad(const float *X, const floa
    if (t == 0) lpart[blockIdx.x] = sl[0];
 }
 
-/* grad[q] = sum over workgroups w (in order) of gpart[w][q]; loss likewise */
-__global__ void k_mlp_reduce(const float *gpart, const float *lpart, int nblk, float *grad, double *loss)
-{
-   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-   if (q < MLP_NP) {
-      float s = 0.f;
-      for (int w = 0; w < nblk; ++w) s += gpart[(size_t)w * MLP_NP + q];
-      grad[q] = s;
-   }
-   if (q == MLP_NP) {
-      double s = 0.0;
-      for (int w = 0; w < nblk; ++w) s += (double)lpart[w];
-      *loss = s;
-   }
-}
+#define RQ 16       /* gradient entries per reduction workgroup */
+#define RROWS 1024  /* workgroups of a full k_mlp_loss_grad grid */
 
-/* Adam (Kingma & Ba 2015) on the whole parameter vector, step t >= 1 */
-__global__ void k_mlp_adam(float *P, const float *g, float *m, float *v, float lr, float b1, float b2, float eps,
-                           int t)
+/* grad[q] = sum over workgroups w (in order) of gpart[w][q]; the loss
+ * likewise (the last workgroup).  The partials of RQ entries come into LDS
+ * with every load in flight at once, then one thread per entry adds them in
+ * order: 13 us for 1024 workgroups, where a thread per entry reading them one
+ * by one took 296.  With P, the Adam step t >= 1 (Kingma & Ba 2015) of the
+ * entry follows. */
+__global__ void __launch_bounds__(256) k_mlp_reduce(const float *__restrict__ gpart, const float *__restrict__ lpart,
+                                                    int nblk, float *__restrict__ grad, double *__restrict__ loss,
+                                                    float *__restrict__ P, float *__restrict__ m,
+                                                    float *__restrict__ v, float lr, float b1, float b2, float eps,
+                                                    int t)
 {
-   const int q = blockIdx.x * blockDim.x + threadIdx.x;
-   if (q >= MLP_NP) return;
-   const float gq = g[q];
-   const float mq = b1 * m[q] + (1.f - b1) * gq;
-   const float vq = b2 * v[q] + (1.f - b2) * gq * gq;
-   m[q] = mq;
-   v[q] = vq;
-   const float mh = mq / (1.f - powf(b1, (float)t));
-   const float vh = vq / (1.f - powf(b2, (float)t));
-   P[q] -= lr * mh / (sqrtf(vh) + eps);
+   __shared__ float rows[RROWS][RQ];
+   const int tid = threadIdx.x, q0 = blockIdx.x * RQ;
+   if (q0 >= MLP_NP) {
+      for (int w = tid; w < nblk; w += 256) rows[w / RQ][w % RQ] = lpart[w];
+      __syncthreads();
+      if (tid == 0) {
+         double s = 0.0;
+         for (int w = 0; w < nblk; ++w) s += (double)rows[w / RQ][w % RQ];
+         *loss = s;
+      }
+      return;
+   }
+   const int c = tid % RQ, q = min(q0 + c, MLP_NP - 1), w0 = tid / RQ;
+   constexpr int U = RROWS / (256 / RQ);
+   float r[U];
+#pragma unroll
+   for (int u = 0; u < U; ++u) r[u] = gpart[(size_t)min(w0 + (256 / RQ) * u, nblk - 1) * MLP_NP + q];
+#pragma unroll
+   for (int u = 0; u < U; ++u) rows[w0 + (256 / RQ) * u][c] = r[u];
+   __syncthreads();
+   if (tid >= RQ || q0 + tid >= MLP_NP) return;
+   float s = 0.f;
+#pragma unroll 16
+   for (int w = 0; w < nblk; ++w) s += rows[w][tid];
+   grad[q] = s;
+   if (P) {
+      const float gq = s;
+      const float mq = b1 * m[q] + (1.f - b1) * gq;
+      const float vq = b2 * v[q] + (1.f - b2) * gq * gq;
+      m[q] = mq;
+      v[q] = vq;
+      const float mh = mq / (1.f - powf(b1, (float)t));
+      const float vh = vq / (1.f - powf(b2, (float)t));
+      P[q] -= lr * mh / (sqrtf(vh) + eps);
+   }
 }
 
 /* y[i] of every sample; with Kout, also Kout[i] = clamp(alpha exp(y), kmin,
@@ -272,21 +422,15 @@ __global__ void k_precond_stats(const double2 *CP, const double2 *Rh, const doub
 
 int mlp_nparam(void) { return MLP_NP; }
 
-int launch_mlp_loss_grad(const float *X, const float *A, const float *B, long n, const float *P, float *gpart,
-                         float *lpart, int nblk, float *grad, double *loss, hipStream_t s)
+/* the loss and gradient at P and, with m and v, the Adam step t of P */
+static int launch_mlp_step(const float *X, const float *A, const float *B, long n, float *P, float *gpart, float *lpart,
+                           int nblk, float *grad, double *loss, float *m, float *v, float lr, int t, hipStream_t s)
 {
+   if (nblk > RROWS) { cpsd_set_error("mlp: %d workgroups, at most %d", nblk, RROWS); return -1; }
    hipLaunchKernelGGL(k_mlp_loss_grad, dim3(nblk), dim3(TB), 0, s, X, A, B, n, P, gpart, lpart);
    CPSD_CHECK(hipGetLastError());
-   hipLaunchKernelGGL(k_mlp_reduce, dim3((MLP_NP + 1 + 255) / 256), dim3(256), 0, s, gpart, lpart, nblk, grad,
-                      loss);
-   CPSD_CHECK(hipGetLastError());
-   return 0;
-}
-
-int launch_mlp_adam(float *P, const float *g, float *m, float *v, float lr, int t, hipStream_t s)
-{
-   hipLaunchKernelGGL(k_mlp_adam, dim3((MLP_NP + 255) / 256), dim3(256), 0, s, P, g, m, v, lr, 0.9f, 0.999f,
-                      1e-8f, t);
+   hipLaunchKernelGGL(k_mlp_reduce, dim3((MLP_NP + RQ - 1) / RQ + 1), dim3(256), 0, s, gpart, lpart, nblk, grad, loss,
+                      m ? P : nullptr, m, v, lr, 0.9f, 0.999f, 1e-8f, t);
    CPSD_CHECK(hipGetLastError());
    return 0;
 }
@@ -360,7 +504,7 @@ static int upload_set(const float *X, const double *A, const double *B, long n, 
 static int grad_blocks(long n)
 {
    const long chunks = (n + TB - 1) / TB;
-   return (int)(chunks < 1024 ? (chunks > 0 ? chunks : 1) : 1024);
+   return (int)(chunks < RROWS ? (chunks > 0 ? chunks : 1) : RROWS);
 }
 
 extern "C" int cpsd_mlp_nparam(void) { return MLP_NP; }
@@ -379,8 +523,8 @@ extern "C" int cpsd_mlp_loss_grad(const float *X, const double *A, const double 
        alloc(gp, (size_t)nblk * MLP_NP * sizeof(float)) || alloc(lp, nblk * sizeof(float)) ||
        alloc(dg, MLP_NP * sizeof(float)) || alloc(dl, sizeof(double)))
       return -1;
-   if (launch_mlp_loss_grad((float *)dX.p, (float *)dA.p, (float *)dB.p, n, (float *)dP.p, (float *)gp.p,
-                            (float *)lp.p, nblk, (float *)dg.p, (double *)dl.p, s) != 0)
+   if (launch_mlp_step((float *)dX.p, (float *)dA.p, (float *)dB.p, n, (float *)dP.p, (float *)gp.p, (float *)lp.p,
+                       nblk, (float *)dg.p, (double *)dl.p, nullptr, nullptr, 0.f, 0, s) != 0)
       return -1;
    CPSD_CHECK(hipMemcpy(grad, dg.p, MLP_NP * sizeof(float), hipMemcpyDeviceToHost));
    CPSD_CHECK(hipMemcpy(loss, dl.p, sizeof(double), hipMemcpyDeviceToHost));
@@ -405,9 +549,8 @@ extern "C" int cpsd_mlp_train(const float *X, const double *A, const double *B, 
    CPSD_CHECK(hipMemsetAsync(dm.p, 0, MLP_NP * sizeof(float), s));
    CPSD_CHECK(hipMemsetAsync(dv.p, 0, MLP_NP * sizeof(float), s));
    for (int it = 0; it < iters; ++it) {
-      if (launch_mlp_loss_grad((float *)dX.p, (float *)dA.p, (float *)dB.p, n, (float *)dP.p, (float *)gp.p,
-                               (float *)lp.p, nblk, (float *)dg.p, (double *)dl.p + it, s) != 0 ||
-          launch_mlp_adam((float *)dP.p, (float *)dg.p, (float *)dm.p, (float *)dv.p, lr, it + 1, s) != 0)
+      if (launch_mlp_step((float *)dX.p, (float *)dA.p, (float *)dB.p, n, (float *)dP.p, (float *)gp.p, (float *)lp.p,
+                          nblk, (float *)dg.p, (double *)dl.p + it, (float *)dm.p, (float *)dv.p, lr, it + 1, s) != 0)
          return -1;
    }
    CPSD_CHECK(hipMemcpy(params, dP.p, MLP_NP * sizeof(float), hipMemcpyDeviceToHost));
