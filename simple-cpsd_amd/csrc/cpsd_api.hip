@@ -580,7 +580,7 @@ static int run_structure(cpsd_dev *c)
    a.n = c->n; a.ng = c->ng; a.ngp = c->ngp; a.nion = c->nion; a.nproj = c->nproj;
    a.kx = c->kx; a.ky = c->ky; a.kz = c->kz;
    a.ex1 = c->ex1; a.ex2 = c->ex2; a.ex3 = c->ex3;
-   a.katm = c->katm; a.lmmax = c->lmmax; a.zv = c->zv; a.vl = c->vl; a.vnl = c->vnl;
+   a.katm = c->katm; a.lmmax = c->lmmax; a.poff = c->poff; a.zv = c->zv; a.vl = c->vl; a.vnl = c->vnl;
    a.s = c->s; a.vall = c->vall; a.B = c->B;
    TRY(sd_structure(a, st));
    c->bf_valid = 0;

@@ -82,47 +82,76 @@ __global__ void __launch_bounds__(256) k_force_nlsum(const double *__restrict__ 
    if (threadIdx.x == 0) nlsum[pd] = v;
 }
 
-/* one thread per ion: add the parts, the real-space Ewald pairs, then move
- * the ion */
-__global__ void k_force_finish(ForceFinishArgs a)
+#define FJ 32   /* ions per pass of k_force_finish */
+#define FL 27   /* images per pass */
+
+/* A workgroup per ion: add the parts and the real-space Ewald pairs, then move
+ * the ion.  The pair terms (a square root, an exponential and divisions per
+ * image) of FJ x FL pairs and images are evaluated at once; the sums over
+ * images and ions then run in order from LDS, so the force is the sequential
+ * one.  At 24 ions 10 us, where a thread per ion took 202. */
+__global__ void __launch_bounds__(256) k_force_finish(ForceFinishArgs a)
 {
-   const int ii = blockIdx.x * blockDim.x + threadIdx.x;
-   if (ii >= a.nion) return;
-   double f[3] = {0.0, 0.0, 0.0};
-   for (int ch = 0; ch < a.nchunk; ++ch)
-      for (int d = 0; d < 3; ++d) f[d] += a.gpart[((size_t)ii * a.nchunk + ch) * 3 + d];
+   __shared__ double4 term[FJ][FL];   /* displacement and factor of a pair image */
+   __shared__ double sum[FJ][3];
+   __shared__ double part[256];
+   const int ii = blockIdx.x, t = threadIdx.x;
    const int ia = a.katm[ii];
-   for (int l = 0; l < a.lmmax[ia]; ++l)
-      for (int d = 0; d < 3; ++d) f[d] -= 4.0 * a.nlsum[(a.poff[ii] + l) * 3 + d];
+   /* thread d < 3 holds component d */
+   double f = 0.0;
+   for (int c0 = 0; c0 < 3 * a.nchunk; c0 += 255) {   /* 85 chunks of 3 */
+      if (t < 255 && c0 + t < 3 * a.nchunk) part[t] = a.gpart[(size_t)ii * a.nchunk * 3 + c0 + t];
+      __syncthreads();
+      if (t < 3)
+         for (int e = t; e < 255 && c0 + e < 3 * a.nchunk; e += 3) f += part[e];
+      __syncthreads();
+   }
+   if (t < 3)
+      for (int l = 0; l < a.lmmax[ia]; ++l) f -= 4.0 * a.nlsum[(a.poff[ii] + l) * 3 + t];
    /* real space, :334-362, with the erfc of :11-17 */
    const double CERFC = 1.128379167;
    const double B1 = 0.0705230784, B2 = 0.0422820123, B3 = 0.0092705272;
    const double B4 = 0.0001520143, B5 = 0.0002765672, B6 = 0.0000430638;
    const double zi = a.zv[ia];
-   for (int jj = 0; jj < a.nion; ++jj) {
-      if (jj == ii) continue;
-      const double dx = a.r1[3 * ii] - a.r1[3 * jj];
-      const double dy = a.r1[3 * ii + 1] - a.r1[3 * jj + 1];
-      const double dz = a.r1[3 * ii + 2] - a.r1[3 * jj + 2];
-      const double zz = zi * a.zv[a.katm[jj]];
-      double s1 = 0.0, s2 = 0.0, s3 = 0.0;
-      for (int l = 0; l < a.nsh; ++l) {
-         const double x = a.rcell[l] + dx, y = a.rcell[l + a.nsh] + dy, z = a.rcell[l + 2 * a.nsh] + dz;
-         const double r = sqrt(x * x + y * y + z * z);
-         const double w = r / a.rcut;
-         double aa = 1.0 + w * (B1 + w * (B2 + w * (B3 + w * (B4 + w * (B5 + w * B6)))));
-         aa *= aa * aa * aa;
-         const double erfc = 1.0 / (aa * aa * aa * aa);
-         const double adiff = zz * (erfc + CERFC * w * exp(-w * w)) / (r * r * r);
-         s1 += x * adiff;
-         s2 += y * adiff;
-         s3 += z * adiff;
+   for (int j0 = 0; j0 < a.nion; j0 += FJ) {
+      const int nj = min(FJ, a.nion - j0);
+      if (t < 3 * FJ) sum[t / 3][t % 3] = 0.0;
+      for (int l0 = 0; l0 < a.nsh; l0 += FL) {
+         const int nl = min(FL, a.nsh - l0);
+         __syncthreads();
+         for (int e = t; e < nj * nl; e += 256) {
+            const int j = e / nl, l = l0 + e % nl, jj = j0 + j;
+            if (jj == ii) continue;
+            const double dx = a.r1[3 * ii] - a.r1[3 * jj];
+            const double dy = a.r1[3 * ii + 1] - a.r1[3 * jj + 1];
+            const double dz = a.r1[3 * ii + 2] - a.r1[3 * jj + 2];
+            const double zz = zi * a.zv[a.katm[jj]];
+            const double x = a.rcell[l] + dx, y = a.rcell[l + a.nsh] + dy, z = a.rcell[l + 2 * a.nsh] + dz;
+            const double r = sqrt(x * x + y * y + z * z);
+            const double w = r / a.rcut;
+            double aa = 1.0 + w * (B1 + w * (B2 + w * (B3 + w * (B4 + w * (B5 + w * B6)))));
+            aa *= aa * aa * aa;
+            const double erfc = 1.0 / (aa * aa * aa * aa);
+            const double adiff = zz * (erfc + CERFC * w * exp(-w * w)) / (r * r * r);
+            term[j][l - l0] = make_double4(x, y, z, adiff);
+         }
+         __syncthreads();
+         if (t < 3 * nj && j0 + t / 3 != ii) {
+            const int j = t / 3, d = t % 3;
+            double s = sum[j][d];
+            for (int l = 0; l < nl; ++l) s += reinterpret_cast<const double *>(&term[j][l])[d] * term[j][l].w;
+            sum[j][d] = s;
+         }
       }
-      f[0] += s1; f[1] += s2; f[2] += s3;
+      __syncthreads();
+      if (t < 3)
+         for (int j = 0; j < nj; ++j)
+            if (j0 + j != ii) f += sum[j][t];
+      __syncthreads();
    }
-   for (int d = 0; d < 3; ++d) {
-      a.fion[3 * ii + d] = f[d];
-      a.r2[3 * ii + d] = a.r1[3 * ii + d] + a.dti[ii] * f[d];
+   if (t < 3) {
+      a.fion[3 * ii + t] = f;
+      a.r2[3 * ii + t] = a.r1[3 * ii + t] + a.dti[ii] * f;
    }
 }
 
@@ -143,7 +172,7 @@ int sd_force_nlsum(const double *nlpart, int kblocks, int nproj, double *nlsum, 
 
 int sd_force_finish(const ForceFinishArgs &a, hipStream_t s)
 {
-   hipLaunchKernelGGL(k_force_finish, dim3((a.nion + 63) / 64), dim3(64), 0, s, a);
+   hipLaunchKernelGGL(k_force_finish, dim3(a.nion), dim3(256), 0, s, a);
    CPSD_CHECK(hipGetLastError());
    return 0;
 }

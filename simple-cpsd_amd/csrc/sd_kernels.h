@@ -7,7 +7,7 @@ struct StructArgs {
    int n, ng, ngp, nion, nproj;
    const int *kx, *ky, *kz;          /* grid coordinates of packed G */
    const double2 *ex1, *ex2, *ex3;   /* phase factors per ion */
-   const int *katm, *lmmax;
+   const int *katm, *lmmax, *poff;   /* poff: first projector of each ion */
    const double *zv;
    const double *vl;                 /* [kind][ngp] */
    const double *vnl;                /* [kind][9][ngp] */

@@ -55,44 +55,60 @@ __global__ void k_pad_real(const double *__restrict__ dense, int n, double *__re
 
 /* ------------------------------------- structure factors and projectors */
 
+/* structure factor of ion ii at packed G (kx, ky, kz) */
+__device__ __forceinline__ double2 ion_phase(const StructArgs &a, int ii, int kx, int ky, int kz)
+{
+   const double2 e1 = a.ex1[ii * (a.n + 2) / 2 + kx];
+   const double2 e2 = a.ex2[ii * a.n + ky];
+   const double2 e3 = a.ex3[ii * a.n + kz];
+   const double2 t = make_double2(e2.x * e3.x - e2.y * e3.y, e2.x * e3.y + e2.y * e3.x);
+   return make_double2(e1.x * t.x - e1.y * t.y, e1.y * t.x + e1.x * t.y);
+}
+
+#define SION 8   /* ions per workgroup of the projector rows */
+
 /* Per packed G: exi_I = ex1[kx] * (ex2[ky] * ex3[kz]) (ccpsdv3/strfac.c:93-123),
  * s = sum_I zv exi_I, vall = sum_I vl exi_I (ccpsdv3/cpsd.c:232-245), and the
  * projector rows beta_{I,l} = exi_I vnl_l (times i for l = 1..3,
- * ccpsdv3/cpsd.c:260-286), ions in input order. */
+ * ccpsdv3/cpsd.c:260-286), ions in input order.
+ * blockIdx.y = 0 sums s and vall over the ions in order; y > 0 writes the
+ * projectors of SION ions (first projector of an ion: poff).  Bound by the
+ * projector writes: 48 projectors at 64^3 28 us with one thread per G writing
+ * them all, 19 us split over the ions. */
 __global__ void k_structure(StructArgs a)
 {
    const int p = blockIdx.x * blockDim.x + threadIdx.x;
    if (p >= a.ngp) return;
-   double2 s = make_double2(0.0, 0.0), vall = make_double2(0.0, 0.0);
-   if (p >= a.ng) {
-      a.s[p] = s; a.vall[p] = vall;
-      for (int m = 0; m < a.nproj; ++m) a.B[(size_t)m * a.ngp + p] = s;
+   const bool pad = p >= a.ng;
+   const int kx = a.kx[p], ky = a.ky[p], kz = a.kz[p];
+   if (blockIdx.y == 0) {
+      double2 s = make_double2(0.0, 0.0), vall = make_double2(0.0, 0.0);
+      for (int ii = 0; ii < a.nion && !pad; ++ii) {
+         const int ia = a.katm[ii];
+         const double2 e = ion_phase(a, ii, kx, ky, kz);
+         const double z = a.zv[ia];
+         s.x += z * e.x; s.y += z * e.y;
+         const double vl = a.vl[(size_t)ia * a.ngp + p];
+         vall.x += e.x * vl; vall.y += e.y * vl;
+      }
+      a.s[p] = s;
+      a.vall[p] = vall;
       return;
    }
-   const int kx = a.kx[p], ky = a.ky[p], kz = a.kz[p];
-   int m = 0;
-   for (int ii = 0; ii < a.nion; ++ii) {
-      const int ia = a.katm[ii];
-      const double2 e1 = a.ex1[ii * (a.n + 2) / 2 + kx];
-      const double2 e2 = a.ex2[ii * a.n + ky];
-      const double2 e3 = a.ex3[ii * a.n + kz];
-      const double2 t = make_double2(e2.x * e3.x - e2.y * e3.y, e2.x * e3.y + e2.y * e3.x);
-      const double2 e = make_double2(e1.x * t.x - e1.y * t.y, e1.y * t.x + e1.x * t.y);
-      const double z = a.zv[ia];
-      s.x += z * e.x; s.y += z * e.y;
-      const double vl = a.vl[(size_t)ia * a.ngp + p];
-      vall.x += e.x * vl; vall.y += e.y * vl;
-      for (int l = 0; l < a.lmmax[ia]; ++l) {
+   const int i0 = (blockIdx.y - 1) * SION, i1 = min(a.nion, i0 + SION);
+   for (int ii = i0; ii < i1; ++ii) {
+      const int ia = a.katm[ii], nl = a.lmmax[ia];
+      if (nl == 0) continue;
+      const double2 e = ion_phase(a, ii, kx, ky, kz);
+      double2 *B = a.B + (size_t)a.poff[ii] * a.ngp + p;
+      for (int l = 0; l < nl; ++l) {
          const double v = a.vnl[((size_t)ia * 9 + l) * a.ngp + p];
          double2 b;
          if (l == 0 || l >= 4) b = make_double2(e.x * v, e.y * v);
          else b = make_double2(-e.y * v, e.x * v);
-         a.B[(size_t)m * a.ngp + p] = b;
-         ++m;
+         B[(size_t)l * a.ngp] = pad ? make_double2(0.0, 0.0) : b;
       }
    }
-   a.s[p] = s;
-   a.vall[p] = vall;
 }
 
 /* Phase factors by repeated complex multiplication (ccpsdv3/strfac.c:10-77):
@@ -1167,7 +1183,8 @@ int sd_pad_real(const double *dense, int n, double *padded, hipStream_t s)
 
 int sd_structure(const StructArgs &a, hipStream_t s)
 {
-   hipLaunchKernelGGL(k_structure, g1(a.ngp), dim3(256), 0, s, a);
+   hipLaunchKernelGGL(k_structure, dim3((a.ngp + 255) / 256, 1 + (a.nproj > 0 ? (a.nion + SION - 1) / SION : 0)), dim3(256), 0,
+                      s, a);
    CPSD_CHECK(hipGetLastError());
    return 0;
 }
