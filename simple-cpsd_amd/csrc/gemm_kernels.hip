@@ -15,7 +15,7 @@
  *                      2*sum - sum_{kx=0} of ccpsdv3/gcdotc.c:25-27) is
  *                      applied to the A operand.
  *   k_gemm_tall      : tall output [ncol][K] = X^T A with a short reduction
- *                      (projectors or orbitals), 128- or 64-column x 128-row
+ *                      (projectors or orbitals), 128-, 64- or 32-column x 128-row
  *                      output tiles over 8 waves, SD epilogues fused; the
  *                      nonlocal force (ccpsdv3/cpsd.c:291-304) reduces its
  *                      output against the projectors instead of storing it.
@@ -58,9 +58,7 @@ __device__ __forceinline__ void sched_mix()
 template<int V> using template_int = std::integral_constant<int, V>;
 
 #define TT 128  /* output tile edge */
-#define KT 16   /* K step */
 #define KC 32   /* K ranges are multiples of this */
-#define KP (KT + 2)  /* LDS row pitch: a 16-byte read of 8 rows covers the banks once */
 
 /* The blocks of a diagonal tile.  Its 36 upper 16 x 16 blocks are split
  * evenly between the four waves: waves 0-2 take 3 x 3 squares on or above the
@@ -74,11 +72,12 @@ __device__ constexpr int dg_tri(int f) { return 3 * (f >> 1) + (f & 1); }
 __device__ constexpr int dg_ta(int b) { return 2 * (b / 3) + (b % 3 == 2); }
 __device__ constexpr int dg_tb(int b) { return 2 * (b / 3) + (b % 3 != 0); }
 
-/* partial[z][m][n] = sum_{k in split z} w[k] A[m][k] B[n][k].  TMR x 128 output
- * tiles (TMR = 128, or 96 when that pads the row count less, e.g. 192
- * projectors), four waves of (TMR/2) x 64, K steps of 16 double-buffered in 72
- * KB of LDS: two workgroups share a CU, so one's barriers and loads overlap
- * the other's MFMAs.  The operands of the next 8 k are read from LDS between
+/* partial[z][m][n] = sum_{k in split z} w[k] A[m][k] B[n][k].  TM x TN output
+ * tiles, four waves of (TM/2) x (TN/2), K steps of KT double-buffered in LDS.
+ * 128 x 128 (or 96 x 128 when that pads the row count less, e.g. 192
+ * projectors) in 72 KB: two workgroups share a CU, so one's barriers and loads
+ * overlap the other's MFMAs.  32 x 32 (35 KB, K steps of 32) where 128 would
+ * leave CUs without work (tn_tile).  The operands of the next 8 k are read from LDS between
  * the MFMAs of the current ones; the weight is applied to the A rows on their
  * way into LDS.  Each sum runs over k in order, one fused multiply-add per
  * term (what the FP64 MFMA does with its four k), so a split's result does
@@ -91,8 +90,8 @@ __device__ constexpr int dg_tb(int b) { return 2 * (b / 3) + (b % 3 != 0); }
  * pairs, i.e. all tiles of the same K range, which then share that XCD's L2.
  *
  * A symmetric product (SYM: A = B, M = N) forms the listed tiles only: tiles
- * above the diagonal in full, diagonal tiles by their upper 36 blocks, nine
- * to a wave against 16 in a full tile.  Split z of a diagonal tile is the
+ * above the diagonal in full, 128 x 128 diagonal tiles by their upper 36
+ * blocks, nine to a wave against 16 in a full tile.  Split z of a diagonal tile is the
  * whole range z of kchunk_dd (tl.halves 1) or half h of range z' (z = 2 z' +
  * h, tl.halves 2).
  *
@@ -101,8 +100,8 @@ __device__ constexpr int dg_tb(int b) { return 2 * (b / 3) + (b % 3 != 0); }
  * <c1|c1> carried 3.68 ms (60); the form with four v_mfma_f64_4x4x4_4b
  * per 16 x 16 block, 8 waves of 64 x 32 and one workgroup per CU took 4.24 and
  * 4.46 ms (51 and 49 TFLOP/s). */
-template<int TMR, bool SYM>
-__global__ void __launch_bounds__(256, 2)
+template<int TM, int TN, int KT, bool SYM>
+__global__ void __launch_bounds__(256, TN == 128 ? 2 : 4)
 k_gemm_tn_splitk(const double *__restrict__ A, size_t lda, int M,
                  const double *__restrict__ B, size_t ldb, int N,
                  const double *__restrict__ w, size_t K, size_t kchunk, size_t kchunk_dd,
@@ -141,42 +140,43 @@ k_gemm_tn_splitk(const double *__restrict__ A, size_t lda, int M,
    /* S[buf][0]: the weighted A rows, S[buf][1]: the B rows (of a diagonal
     * tile the same rows without the weight).  Of each 8 k the pairs (q, q + 4)
     * are adjacent: one 16-byte read hands a lane its slot of two successive
-    * instructions */
-   __shared__ __align__(16) double S[2][2][TT][KP];
+    * instructions.  The pitch lets a 16-byte read of 8 rows cover the banks
+    * once. */
+   constexpr int KP = KT + 2;
+   __shared__ __align__(16) double S[2][2][TM > TN ? TM : TN][KP];
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
    const int wm = wave & 1, wn = wave >> 1;
    const int l16 = lane & 15, lq4 = lane >> 4;
-   constexpr int BI = TMR / 32;   /* 16-row blocks per wave */
+   constexpr int BI = TM / 32, BJ = TN / 32;   /* 16-row and 16-column blocks per wave */
 
    /* Row addresses without branches: rows past M or N repeat the last one
     * (their outputs are not written), so a load is a 32-bit lane offset on a
-    * scalar base that moves along K.  Rows lr + 32 h, 8 lanes to the 128-byte
-    * piece of a row. */
-   const int lr = tid >> 3, lc = tid & 7;
-   const int ar0 = tm * TMR, br0 = tn * TT;
+    * scalar base that moves along K.  PR lanes to the K step of a row. */
+   constexpr int PR = KT / 2, RP = 256 / PR;
+   constexpr int HA = TM / RP, HB = TN / RP;
+   const int lr = tid / PR, lc = tid % PR;
+   const int ar0 = tm * TM, br0 = tn * TN;
    const char *const abase = reinterpret_cast<const char *>(A + (size_t)ar0 * lda);
    const char *const bbase = reinterpret_cast<const char *>(B + (size_t)br0 * ldb);
-   unsigned aoff[4], boff[4];
+   unsigned aoff[HA], boff[HB];
 #pragma unroll
-   for (int h = 0; h < 4; ++h) {
-      aoff[h] = (unsigned)min(lr + 32 * h, M - 1 - ar0) * (unsigned)(lda * 8) + lc * 16;
-      boff[h] = (unsigned)min(lr + 32 * h, N - 1 - br0) * (unsigned)(ldb * 8) + lc * 16;
-   }
+   for (int h = 0; h < HA; ++h) aoff[h] = (unsigned)min(lr + RP * h, M - 1 - ar0) * (unsigned)(lda * 8) + lc * 16;
+#pragma unroll
+   for (int h = 0; h < HB; ++h) boff[h] = (unsigned)min(lr + RP * h, N - 1 - br0) * (unsigned)(ldb * 8) + lc * 16;
    /* K tile t + 1 waits in registers while tile t is multiplied */
-   double2 ra[4], rb[4], rw;
+   double2 ra[HA], rb[HB], rw;
    auto gload = [&](size_t k0) {
       const char *const ak = abase + k0 * 8;
       const char *const bk = bbase + k0 * 8;
 #pragma unroll
-      for (int h = 0; h < 4; ++h)
-         if (32 * h < TMR) ra[h] = load2(ak, aoff[h]);
+      for (int h = 0; h < HA; ++h) ra[h] = load2(ak, aoff[h]);
       if (!SYM || !dd) {
 #pragma unroll
-         for (int h = 0; h < 4; ++h) rb[h] = load2(bk, boff[h]);
+         for (int h = 0; h < HB; ++h) rb[h] = load2(bk, boff[h]);
       }
       rw = load2(reinterpret_cast<const char *>(w + k0), lc * 16);
    };
-   /* k = 2 lc, 2 lc + 1 of rows lr + 32 h */
+   /* k = 2 lc, 2 lc + 1 of rows lr + RP h */
    const int sq = 8 * (lc >> 2) + 4 * (lc & 1) + ((lc >> 1) & 1);
    auto lput = [&](double *row, double2 v) {
       row[sq] = v.x;
@@ -184,9 +184,13 @@ k_gemm_tn_splitk(const double *__restrict__ A, size_t lda, int M,
    };
    auto lstore = [&](int bf) {
 #pragma unroll
-      for (int h = 0; h < 4; ++h) {
-         if (32 * h < TMR) lput(S[bf][0][lr + 32 * h], make_double2(ra[h].x * rw.x, ra[h].y * rw.y));
-         lput(S[bf][1][lr + 32 * h], SYM && dd ? ra[h] : rb[h]);
+      for (int h = 0; h < HA; ++h) lput(S[bf][0][lr + RP * h], make_double2(ra[h].x * rw.x, ra[h].y * rw.y));
+      if (SYM && dd) {
+#pragma unroll
+         for (int h = 0; h < HA; ++h) lput(S[bf][1][lr + RP * h], ra[h]);
+      } else {
+#pragma unroll
+         for (int h = 0; h < HB; ++h) lput(S[bf][1][lr + RP * h], rb[h]);
       }
    };
    /* k = 8 ks + lq4 and 8 ks + 4 + lq4 of a row */
@@ -198,6 +202,7 @@ k_gemm_tn_splitk(const double *__restrict__ A, size_t lda, int M,
     * (ia(b), jb(b)), b < NBLK */
    auto kloop = [&](auto na_, auto nb_, auto nblk_, auto arow, auto brow, auto ia, auto jb, mfma_d4 *acc) {
       constexpr int NA = decltype(na_)::value, NB = decltype(nb_)::value, NBLK = decltype(nblk_)::value;
+      constexpr int NK = KT / 8;
       struct Frag { double2 a[NA], b[NB]; };
       auto fread = [&](Frag &f, int bf, int ks) {
 #pragma unroll
@@ -219,29 +224,34 @@ k_gemm_tn_splitk(const double *__restrict__ A, size_t lda, int M,
       lstore(0);
       gload(kb + (nt > 1 ? KT : 0));
       __syncthreads();
-      Frag f0, f1;
-      fread(f0, 0, 0);
+      Frag f[2];
+      fread(f[0], 0, 0);
       int buf = 0;
       /* branch-free body: one workgroup's MFMA stream has to stay fed from one
        * wave per SIMD, so the LDS reads and writes and the loads of the next
        * tile are spread between the MFMAs (64 cycles each) */
       for (int t = 0; t + 1 < nt; ++t) {
-         fread(f1, buf, 1);
-         mma(f0);
-         lstore(buf ^ 1);
-         sched_mix<0x100, NA + NB, 1>();
-         sched_mix<0x200, TMR / 32 + 4, 1>();
+#pragma unroll
+         for (int ks = 0; ks + 1 < NK; ++ks) {
+            fread(f[(ks + 1) & 1], buf, ks + 1);
+            mma(f[ks & 1]);
+            if (ks + 2 == NK) lstore(buf ^ 1);
+            sched_mix<0x100, NA + NB, 1>();
+            if (ks + 2 == NK) sched_mix<0x200, HA + HB, 1>();
+         }
          __syncthreads();   /* every read of this tile has been issued and has returned */
          buf ^= 1;
-         fread(f0, buf, 0);
+         fread(f[0], buf, 0);
          gload(kb + (size_t)min(t + 2, nt - 1) * KT);
-         mma(f1);
+         mma(f[1]);
          sched_mix<0x100, NA + NB, 1>();
-         sched_mix<0x20, TMR / 32 + 5, 1>();
+         sched_mix<0x20, HA + HB + 1, 1>();
       }
-      fread(f1, buf, 1);
-      mma(f0);
-      mma(f1);
+#pragma unroll
+      for (int ks = 0; ks < NK; ++ks) {
+         if (ks + 1 < NK) fread(f[(ks + 1) & 1], buf, ks + 1);
+         mma(f[ks & 1]);
+      }
    };
    auto store_block = [&](int m0, int n0, const mfma_d4 &v) {
       const int n = n0 + l16;
@@ -251,29 +261,29 @@ k_gemm_tn_splitk(const double *__restrict__ A, size_t lda, int M,
          if (m < M && n < N) partial[((size_t)kz * M + m) * N + n] = v[r];
       }
    };
-   template_int<BI> nbi;
-   template_int<4> n4;
-   if (!SYM || !dd) {
-      mfma_d4 acc[BI * 4];
-      kloop(nbi, n4, template_int<BI * 4>{}, [&](int i) { return BI * wm + i; }, [&](int j) { return 4 * wn + j; },
-            [](int b) { return b % BI; }, [](int b) { return b / BI; }, acc);
+   if (TN != 128 || !SYM || !dd) {
+      /* a diagonal tile of 32 is formed in full */
+      mfma_d4 acc[BI * BJ];
+      kloop(template_int<BI>{}, template_int<BJ>{}, template_int<BI * BJ>{}, [&](int i) { return BI * wm + i; },
+            [&](int j) { return BJ * wn + j; }, [](int b) { return b % BI; }, [](int b) { return b / BI; }, acc);
 #pragma unroll
-      for (int b = 0; b < BI * 4; ++b)
-         store_block(ar0 + 16 * (BI * wm + b % BI), br0 + 16 * (4 * wn + b / BI), acc[b]);
-   } else if (wave < 3) {
+      for (int b = 0; b < BI * BJ; ++b)
+         store_block(ar0 + 16 * (BI * wm + b % BI), br0 + 16 * (BJ * wn + b / BI), acc[b]);
+   } else if constexpr (TN == 128 && TM == 128 && SYM) {
       mfma_d4 acc[9];
-      const int r0 = dg_row(wave), c0 = dg_col(wave);
-      kloop(template_int<3>{}, template_int<3>{}, template_int<9>{}, [&](int i) { return r0 + i; },
-            [&](int j) { return c0 + j; }, [](int b) { return b % 3; }, [](int b) { return b / 3; }, acc);
+      if (wave < 3) {
+         const int r0 = dg_row(wave), c0 = dg_col(wave);
+         kloop(template_int<3>{}, template_int<3>{}, template_int<9>{}, [&](int i) { return r0 + i; },
+               [&](int j) { return c0 + j; }, [](int b) { return b % 3; }, [](int b) { return b / 3; }, acc);
 #pragma unroll
-      for (int b = 0; b < 9; ++b) store_block(ar0 + 16 * (r0 + b % 3), br0 + 16 * (c0 + b / 3), acc[b]);
-   } else {
-      mfma_d4 acc[9];
-      kloop(template_int<6>{}, template_int<6>{}, template_int<9>{}, [](int i) { return dg_tri(i); },
-            [](int j) { return dg_tri(j); }, [](int b) { return dg_ta(b); }, [](int b) { return dg_tb(b); }, acc);
+         for (int b = 0; b < 9; ++b) store_block(ar0 + 16 * (r0 + b % 3), br0 + 16 * (c0 + b / 3), acc[b]);
+      } else {
+         kloop(template_int<6>{}, template_int<6>{}, template_int<9>{}, [](int i) { return dg_tri(i); },
+               [](int j) { return dg_tri(j); }, [](int b) { return dg_ta(b); }, [](int b) { return dg_tb(b); }, acc);
 #pragma unroll
-      for (int b = 0; b < 9; ++b)
-         store_block(ar0 + 16 * dg_tri(dg_ta(b)), br0 + 16 * dg_tri(dg_tb(b)), acc[b]);
+         for (int b = 0; b < 9; ++b)
+            store_block(ar0 + 16 * dg_tri(dg_ta(b)), br0 + 16 * dg_tri(dg_tb(b)), acc[b]);
+      }
    }
 }
 
@@ -336,15 +346,46 @@ static size_t k_chunk(size_t K, int sp)
    return (kc + KC - 1) / KC * KC;
 }
 
+/* The tile edge of a product formed in `splits` K ranges: 32 when 128 x 128
+ * tiles would give a CU less than two workgroups and eight 32 x 32 tiles cover
+ * the output, which then spread each range over several workgroups (more of
+ * them read the rows too often).  The K ranges, hence the results, do not
+ * depend on it.  32 against 128, 256 ranges: Gram of 64 rows at 64^3 26 and
+ * 53 us, of 128 rows (ten tiles) at 80^3 136 and 118; projection 48 x 32 at
+ * 64^3 24 and 60, 96 x 64 at 80^3 103 and 130. */
+static int tn_tile(int M, int N, int splits, int symm)
+{
+   auto tiles = [&](int e) {
+      const long nm = (M + e - 1) / e, nn = (N + e - 1) / e;
+      return symm ? nm * (nm + 1) / 2 : nm * nn;
+   };
+   return tiles(TT) * splits < 512 && tiles(32) <= 8 ? 32 : TT;
+}
+
 /* the listed tiles of the symmetric product A W A^T, so and sd K ranges */
+template<int TE, int KT>
 static int launch_tn_list(const GramTiles &tl, const double *A, size_t lda, int M, const double *w, size_t K, int so,
                           int sd, double *partial, hipStream_t s)
 {
    const long poff = (long)tl.noff * so;
    const long pairs = poff + (long)tl.nd * sd * tl.halves;
-   hipLaunchKernelGGL((k_gemm_tn_splitk<TT, true>), dim3(xcd_grid(poff).x + xcd_grid(pairs - poff).x), dim3(256), 0, s, A, lda,
-                      M, A, lda, M,
-                      w, K, so > 0 ? k_chunk(K, so) : 0, sd > 0 ? k_chunk(K, sd) : 0, 0, 0, poff, pairs, tl, partial);
+   hipLaunchKernelGGL((k_gemm_tn_splitk<TE, TE, KT, true>), dim3(xcd_grid(poff).x + xcd_grid(pairs - poff).x), dim3(256),
+                      0, s, A, lda, M, A, lda, M, w, K, so > 0 ? k_chunk(K, so) : 0, sd > 0 ? k_chunk(K, sd) : 0, 0, 0,
+                      poff, pairs, tl, partial);
+   CPSD_CHECK(hipGetLastError());
+   return 0;
+}
+
+template<int TM, int TN, int KT>
+static int launch_tn_tiles(const double *A, size_t lda, int M, const double *B, size_t ldb, int N, const double *w,
+                           size_t K, int splits, double *partial, hipStream_t s)
+{
+   GramTiles tl;
+   memset(&tl, 0, sizeof tl);
+   const int ntm = (M + TM - 1) / TM, ntile = ntm * ((N + TN - 1) / TN);
+   const long pairs = (long)ntile * splits;
+   hipLaunchKernelGGL((k_gemm_tn_splitk<TM, TN, KT, false>), xcd_grid(pairs), dim3(256), 0, s, A, lda, M, B, ldb, N, w,
+                      K, k_chunk(K, splits), 0, ntm, ntile, 0, pairs, tl, partial);
    CPSD_CHECK(hipGetLastError());
    return 0;
 }
@@ -360,33 +401,30 @@ int launch_gemm_tn_splitk(const double *A, size_t lda, int M, const double *B, s
       cpsd_set_error("gemm_tn: rows of %zu doubles", lda > ldb ? lda : ldb);
       return -1;
    }
-   GramTiles tl;
-   memset(&tl, 0, sizeof tl);
    if (symm) {
-      const int ntm = (M + TT - 1) / TT;
+      int so, sd;
+      gemm_tn_symm_splits(M, K, splits, &so, &sd);
+      /* one 128 x 128 tile or less takes sd ranges throughout; more tiles
+       * than that fill the GPU */
+      const int te = M <= TT ? tn_tile(M, M, sd, 1) : TT;
+      if (M <= TT) so = sd;
+      GramTiles tl;
+      memset(&tl, 0, sizeof tl);
+      const int ntm = (M + te - 1) / te;
       for (int i = 0; i < ntm; ++i) {
          for (int j = i + 1; j < ntm; ++j) { tl.otm[tl.noff] = (unsigned char)i; tl.otn[tl.noff] = (unsigned char)j; ++tl.noff; }
          tl.dt[tl.nd++] = (unsigned char)i;
       }
       tl.halves = 1;
-      int so, sd;
-      gemm_tn_symm_splits(M, K, splits, &so, &sd);
-      return launch_tn_list(tl, A, lda, M, w, K, so, sd, partial, s);
+      if (te == 32) return launch_tn_list<32, 32>(tl, A, lda, M, w, K, so, sd, partial, s);
+      return launch_tn_list<TT, 16>(tl, A, lda, M, w, K, so, sd, partial, s);
    }
+   const int te = tn_tile(M, N, splits, 0);
+   if (te == 32) return launch_tn_tiles<32, 32, 32>(A, lda, M, B, ldb, N, w, K, splits, partial, s);
    /* row tile: 128, or 96 when that leaves fewer padding rows */
    const int pad128 = (M + 127) / 128 * 128 - M, pad96 = (M + 95) / 96 * 96 - M;
-   const int tmr = pad96 < pad128 ? 96 : TT;
-   const int ntm = (M + tmr - 1) / tmr, ntile = gemm_tn_tiles(M, N, 0);
-   const long pairs = (long)ntile * splits;
-   const size_t kchunk = k_chunk(K, splits);
-   if (tmr == 96)
-      hipLaunchKernelGGL((k_gemm_tn_splitk<96, false>), xcd_grid(pairs), dim3(256), 0, s, A, lda, M, B,
-                         ldb, N, w, K, kchunk, 0, ntm, ntile, 0, pairs, tl, partial);
-   else
-      hipLaunchKernelGGL((k_gemm_tn_splitk<TT, false>), xcd_grid(pairs), dim3(256), 0, s, A, lda, M, B,
-                         ldb, N, w, K, kchunk, 0, ntm, ntile, 0, pairs, tl, partial);
-   CPSD_CHECK(hipGetLastError());
-   return 0;
+   if (pad96 < pad128) return launch_tn_tiles<96, 128, 16>(A, lda, M, B, ldb, N, w, K, splits, partial, s);
+   return launch_tn_tiles<128, 128, 16>(A, lda, M, B, ldb, N, w, K, splits, partial, s);
 }
 
 /* the Gram of [C1 C2] (M = 2 ne rows of stride lda, ne a multiple of 128)
@@ -419,7 +457,7 @@ int launch_gram_c2(const double *A, size_t lda, int M, int c2row, const double *
    }
    *sp_off = so;
    *sp_dd = 2 * sd;
-   return launch_tn_list(tl, A, lda, M, w, K, so, sd, partial, s);
+   return launch_tn_list<TT, 16>(tl, A, lda, M, w, K, so, sd, partial, s);
 }
 
 /* out[m][n] = sum_z partial[z][m][n] over the splits that formed (m, n):
@@ -596,8 +634,8 @@ int launch_gemm_tn_small(const double *A, size_t lda, int M, const double *B, si
 template<int EPI, int NT>
 __global__ void __launch_bounds__(256, 2) k_gemm_tall(TallArgs a)
 {
-   constexpr int BJ = 4;                     /* 16-column blocks per wave */
-   constexpr int WN = NT / 64, WK = 4 / WN;  /* waves along the columns and along K */
+   constexpr int BJ = NT < 64 ? NT / 16 : 4;                  /* 16-column blocks per wave */
+   constexpr int WN = NT == 128 ? 2 : 1, WK = 4 / WN;         /* waves along the columns and along K */
    constexpr int BP = TK / WK / 32;          /* block pairs along K per wave */
    constexpr int XP = MC + 2;                /* X pitch: 16-byte reads of 8 rows cover the banks once */
    __shared__ __align__(16) double panels[2 * MC * TK + 2 * NT * XP];
@@ -814,8 +852,11 @@ int launch_gemm_tall(int epi, const TallArgs &args, hipStream_t s)
    if (args.lda * 8 * MC >= (1ull << 32)) { cpsd_set_error("gemm_tall: rows of %zu doubles", args.lda); return -1; }
    TallArgs a = args;
    /* 128 columns per workgroup read A and X half as often as 64; 64 where
-    * they pad less */
-   if ((a.Nc + 127) / 128 * 2 == (a.Nc + 63) / 64) gemm_tall_go<128>(epi, a, s);
+    * they pad less; 32 for small outputs, whose workgroups then hold less and
+    * overlap more of each other's loads (constraint of 32 orbitals at 64^3 30
+    * -> 21 us, nonlocal force of 48 projectors 49 -> 45) */
+   if (a.Nc <= 32 || (epi == EPI_NLFORCE && a.Nc <= 64)) gemm_tall_go<32>(epi, a, s);
+   else if ((a.Nc + 127) / 128 * 2 == (a.Nc + 63) / 64) gemm_tall_go<128>(epi, a, s);
    else gemm_tall_go<64>(epi, a, s);
    CPSD_CHECK(hipGetLastError());
    return 0;
