@@ -89,11 +89,11 @@ static int h2d(T *d, const T *h, size_t n, hipStream_t s)
 }
 
 struct cpsd_dev {
-   int n, nh, ne, nion, nkind, nproj, ng, ngp, nfft3d, n2ft3d, nhc, nsh;
+   int n, nh, ne, nion, nkind, nproj, ng, ngp, nfft3d, n2ft3d, nyq, ncol, nsh;   /* ncol: columns of a plane of T */
    size_t n3;
    hipStream_t stream;
    /* packed-G tables */
-   int *rstart, *rlen, *roff, *frstart, *frlen, *froff, *gidx, *pidx, *kx, *ky, *kz;
+   int *crows, *gmap, *gidx, *pidx, *kx, *ky, *kz;   /* crows, gmap: the columns of T (ColTable) */
    double2 *tw;
    double *w, *tg, *vc, *vg, *vl, *vnl, *pnrm, *zv, *unitg, *r1, *rcell;
    int *katm, *lmmax;
@@ -239,7 +239,7 @@ static int ph_end(cpsd_dev *c, int ph)
 
 static void ctx_free(cpsd_dev *c)
 {
-   void *ptrs[] = {c->rstart, c->rlen, c->roff, c->frstart, c->frlen, c->froff, c->gidx, c->pidx,
+   void *ptrs[] = {c->crows, c->gmap, c->gidx, c->pidx,
                    c->kx, c->ky, c->kz, c->tw, c->w, c->tg, c->vc, c->vg, c->vl, c->vnl, c->pnrm,
                    c->zv, c->unitg, c->r1, c->rcell, c->katm, c->lmmax, c->ex1, c->ex2, c->ex3,
                    c->Cbase, c->CP, c->T, c->Tv, c->dnpart, c->dn, c->xcp, c->xce, c->V, c->dng,
@@ -391,9 +391,9 @@ static int ctx_build(cpsd_dev *c, int nfft, int ne, int nion, const int *katm, c
    for (int i = 0, m = 0; i < nion; ++i) { poff[i] = m; m += lmmax[katm[i]]; }
 
    /* masked rows: each (ky,kz) row must hold one contiguous kx interval */
-   std::vector<int> rs(n * n), rl(n * n), ro(n * n), pidx(c->nfft3d, -1);
+   std::vector<int> clen(n, 0), pidx(c->nfft3d, -1);
    std::vector<int> gidx, kxv, kyv, kzv;
-   int ng = 0, nhc = 0;
+   int ng = 0;
    for (int kz = 0; kz < n; ++kz)
       for (int ky = 0; ky < n; ++ky) {
          const int r = ky + n * kz;
@@ -411,25 +411,33 @@ static int ctx_build(cpsd_dev *c, int nfft, int ne, int nion, const int *katm, c
                last = kx;
             }
          }
-         rs[r] = first < 0 ? 0 : first;
-         rl[r] = first < 0 ? 0 : last - first + 1;
-         ro[r] = ng;
-         for (int kx = rs[r]; kx < rs[r] + rl[r]; ++kx) {
+         if (first < 0) continue;
+         for (int kx = first; kx <= last; ++kx) {
             pidx[kx + nh * r] = ng++;
             gidx.push_back(kx + nh * r);
             kxv.push_back(kx); kyv.push_back(ky); kzv.push_back(kz);
          }
-         if (rs[r] + rl[r] > nhc) nhc = rs[r] + rl[r];
+         if (last + 1 > clen[ky]) clen[ky] = last + 1;
       }
    if (ng == 0) { cpsd_set_error("empty mask"); return -1; }
    c->ng = ng;
    c->ngp = (ng + 63) / 64 * 64;
-   c->nhc = nhc;
+   /* columns of T: row ky holds kx < clen[ky], rows padded to 8 columns */
+   std::vector<int> crows(n);
+   c->ncol = 0;
+   c->nyq = 0;
+   for (int ky = 0; ky < n; ++ky) {
+      crows[ky] = clen[ky] << 16 | c->ncol;
+      c->ncol += (clen[ky] + 7) / 8 * 8;
+      if (clen[ky] == nh) c->nyq = 1;
+   }
+   std::vector<int> gmap((size_t)n * c->ncol, -1);
+   for (int kz = 0; kz < n; ++kz)
+      for (int ky = 0; ky < n; ++ky)
+         for (int kx = 0; kx < clen[ky]; ++kx)
+            gmap[(size_t)kz * c->ncol + (crows[ky] & 0xffff) + kx] = pidx[kx + nh * (ky + n * kz)];
    const int ngp = c->ngp;
    for (int p = ng; p < ngp; ++p) { gidx.push_back(0); kxv.push_back(0); kyv.push_back(0); kzv.push_back(0); }
-
-   std::vector<int> frs(n * n, 0), frl(n * n, nh), fro(n * n);
-   for (int r = 0; r < n * n; ++r) fro[r] = r * nh;
 
    std::vector<double2> tw(n);
    for (int m = 0; m < n; ++m) {
@@ -460,9 +468,7 @@ static int ctx_build(cpsd_dev *c, int nfft, int ne, int nion, const int *katm, c
    CPSD_CHECK(hipHostMalloc((void **)&c->hout, 16 * sizeof(double), hipHostMallocDefault));
    CPSD_CHECK(hipHostMalloc((void **)&c->herr, sizeof(int), hipHostMallocDefault));
    hipStream_t st = c->stream;
-   const size_t nn2 = (size_t)n * n;
-   TRY(dalloc(&c->rstart, nn2)); TRY(dalloc(&c->rlen, nn2)); TRY(dalloc(&c->roff, nn2));
-   TRY(dalloc(&c->frstart, nn2)); TRY(dalloc(&c->frlen, nn2)); TRY(dalloc(&c->froff, nn2));
+   TRY(dalloc(&c->crows, n)); TRY(dalloc(&c->gmap, gmap.size()));
    TRY(dalloc(&c->gidx, ngp)); TRY(dalloc(&c->pidx, c->nfft3d));
    TRY(dalloc(&c->kx, ngp)); TRY(dalloc(&c->ky, ngp)); TRY(dalloc(&c->kz, ngp));
    TRY(dalloc(&c->tw, n)); TRY(dalloc(&c->w, 2 * (size_t)ngp));
@@ -473,10 +479,7 @@ static int ctx_build(cpsd_dev *c, int nfft, int ne, int nion, const int *katm, c
    TRY(dalloc(&c->katm, nion)); TRY(dalloc(&c->lmmax, nkind));
    TRY(dalloc(&c->ex1, (size_t)nion * nh)); TRY(dalloc(&c->ex2, (size_t)nion * n));
    TRY(dalloc(&c->ex3, (size_t)nion * n));
-   TRY(h2d(c->rstart, rs.data(), nn2, st)); TRY(h2d(c->rlen, rl.data(), nn2, st));
-   TRY(h2d(c->roff, ro.data(), nn2, st));
-   TRY(h2d(c->frstart, frs.data(), nn2, st)); TRY(h2d(c->frlen, frl.data(), nn2, st));
-   TRY(h2d(c->froff, fro.data(), nn2, st));
+   TRY(h2d(c->crows, crows.data(), n, st)); TRY(h2d(c->gmap, gmap.data(), gmap.size(), st));
    TRY(h2d(c->gidx, gidx.data(), ngp, st)); TRY(h2d(c->pidx, pidx.data(), c->nfft3d, st));
    TRY(h2d(c->kx, kxv.data(), ngp, st)); TRY(h2d(c->ky, kyv.data(), ngp, st));
    TRY(h2d(c->kz, kzv.data(), ngp, st));
@@ -511,7 +514,7 @@ static int ctx_build(cpsd_dev *c, int nfft, int ne, int nion, const int *katm, c
    TRY(dalloc(&c->Cbase, 2 * orb)); TRY(dalloc(&c->CP, orb));
    CPSD_CHECK(hipMemsetAsync(c->Cbase, 0, 2 * orb * sizeof(double2), st));
    CPSD_CHECK(hipMemsetAsync(c->CP, 0, orb * sizeof(double2), st));
-   const size_t plane = (size_t)n * n * nh;
+   const size_t plane = (size_t)n * c->ncol;
    TRY(dalloc(&c->T, (size_t)ne * plane)); TRY(dalloc(&c->Tv, plane));
    /* launch plan: all orbitals per FFT launch pair by default
     * (CPSD_FFT_BATCH sets fewer, whose z-transformed planes then stay in the
@@ -560,16 +563,29 @@ static int ctx_build(cpsd_dev *c, int nfft, int ne, int nion, const int *katm, c
 
 /* ---------------------------------------------------------- one step */
 
-static int zargs_base(cpsd_dev *c, ZArgs &z, int full)
+static ColTable col_table(const cpsd_dev *c)
 {
+   ColTable t;
+   t.rows = c->crows; t.gmap = c->gmap; t.P = c->ncol; t.nyq = c->nyq;
+   return t;
+}
+
+static ZArgs zargs_base(const cpsd_dev *c)
+{
+   ZArgs z;
    memset(&z, 0, sizeof z);
-   if (full) {
-      z.rows.rstart = c->frstart; z.rows.rlen = c->frlen; z.rows.roff = c->froff; z.rows.nhc = c->nh;
-   } else {
-      z.rows.rstart = c->rstart; z.rows.rlen = c->rlen; z.rows.roff = c->roff; z.rows.nhc = c->nhc;
-   }
+   z.cols = col_table(c);
    z.tw = c->tw;
-   return 0;
+   return z;
+}
+
+static PlaneArgs pargs_base(const cpsd_dev *c)
+{
+   PlaneArgs pa;
+   memset(&pa, 0, sizeof pa);
+   pa.cols = col_table(c);
+   pa.tw = c->tw;
+   return pa;
 }
 
 static int run_structure(cpsd_dev *c)
@@ -662,7 +678,7 @@ static int sd_step(cpsd_dev *c, double dte, int last, int fp64)
 
    ZArgs z;
    PlaneArgs pa;
-   const size_t plane = (size_t)n * n * c->nh;
+   const size_t plane = (size_t)n * c->ncol;
    const int f32 = c->mixed && !last && !fp64;
    /* 2-3: orbitals in batches of fb, so that each batch's z-transformed
     * planes are read by the density pass while they sit in the Infinity
@@ -670,14 +686,14 @@ static int sd_step(cpsd_dev *c, double dte, int last, int fp64)
    for (int b0 = 0; b0 < ne; b0 += c->fb) {
       const int bs = ne - b0 < c->fb ? ne - b0 : c->fb;
       TRY(ph_begin(c, PH_ZG2R));
-      zargs_base(c, z, 0);
+      z = zargs_base(c);
       z.src = C1 + (size_t)b0 * ngp; z.sstride = ngp; z.T = c->T + (size_t)b0 * plane;
       z.fp32 = f32;
-      TRY(launch_zpass_g2r(n, SRC_PACKED, z, bs, st));
+      TRY(launch_zpass_g2r(n, z, bs, st));
       TRY(ph_end(c, PH_ZG2R));
       TRY(ph_begin(c, PH_DENSITY));
-      memset(&pa, 0, sizeof pa);
-      pa.T = c->T + (size_t)b0 * plane; pa.nhload = c->nhc; pa.tw = c->tw; pa.b0 = 0;
+      pa = pargs_base(c);
+      pa.T = c->T + (size_t)b0 * plane;
       pa.nb = c->nob[f32]; pa.nbatch = bs; pa.dnpart = c->dnpart; pa.accumulate = b0 > 0;
       pa.fp32 = f32;
       TRY(launch_plane(n, PM_DENSITY, pa, (bs + c->nob[f32] - 1) / c->nob[f32], st));
@@ -687,14 +703,14 @@ static int sd_step(cpsd_dev *c, double dte, int last, int fp64)
    TRY(ph_begin(c, PH_DNRED));
    TRY(sd_dn_reduce_xc(c->dnpart, c->ndnblk[f32], c->n3, scal2, c->dn, c->xcp, c->xce, st));
    TRY(ph_end(c, PH_DNRED));
-   /* 5 */
+   /* 5, and the z transform of 6 */
    TRY(ph_begin(c, PH_DNG));
-   memset(&pa, 0, sizeof pa);
-   pa.T = c->Tv; pa.tw = c->tw; pa.dn = c->dn; pa.scal1 = scal1; pa.nbatch = 1;
+   pa = pargs_base(c);
+   pa.T = c->Tv; pa.dn = c->dn; pa.scal1 = scal1; pa.nbatch = 1;
    TRY(launch_plane(n, PM_R2C_DN, pa, 1, st));
-   zargs_base(c, z, 0);
-   z.T = c->Tv; z.out = c->dng; z.ostride = ngp;
-   TRY(launch_zpass_r2g(n, DST_DNG, z, 1, st));
+   z = zargs_base(c);
+   z.T = c->Tv; z.out = c->dng; z.ostride = ngp; z.vall = c->vall; z.vc = c->vc; z.scal2 = scal2;
+   TRY(launch_zpass_field(n, z, st));
    TRY(ph_end(c, PH_DNG));
    if (c->move) {
       TRY(ph_begin(c, PH_FORCE));
@@ -708,28 +724,22 @@ static int sd_step(cpsd_dev *c, double dte, int last, int fp64)
    }
    /* 6 */
    TRY(ph_begin(c, PH_VTOT));
-   zargs_base(c, z, 0);
-   z.T = c->Tv; z.vall = c->vall; z.dng = c->dng; z.vc = c->vc; z.scal2 = scal2;
-   TRY(launch_zpass_g2r(n, SRC_VG, z, 1, st));
-   memset(&pa, 0, sizeof pa);
-   pa.T = c->Tv; pa.nhload = c->nhc; pa.tw = c->tw; pa.Vout = c->V; pa.xcp = c->xcp; pa.nbatch = 1;
+   pa = pargs_base(c);
+   pa.T = c->Tv; pa.Vout = c->V; pa.xcp = c->xcp; pa.nbatch = 1;
    TRY(launch_plane(n, PM_VTOT, pa, 1, st));
    TRY(ph_end(c, PH_VTOT));
    /* 7-8, batched the same way: the z pass reads what the plane pass wrote */
    for (int b0 = 0; b0 < ne; b0 += c->fb) {
       const int bs = ne - b0 < c->fb ? ne - b0 : c->fb;
       TRY(ph_begin(c, PH_VPSI));
-      memset(&pa, 0, sizeof pa);
-      pa.T = c->T + (size_t)b0 * plane; pa.nhload = c->nhc; pa.tw = c->tw; pa.V = c->V;
+      pa = pargs_base(c);
+      pa.T = c->T + (size_t)b0 * plane; pa.V = c->V;
       pa.nbatch = bs; pa.fp32 = f32;
-      /* orbitals per workgroup: an FP64 pass that prefetches the next
-       * orbital's plane (plane_prefetch_on) takes up to 4 while the grid
-       * keeps about 4 workgroups per CU (the kernel takes one otherwise) */
-      pa.nb = (f32 || !plane_prefetch_on(n)) ? 1 : (int)std::max(1L, std::min(4L, (long)bs * n / 1024));
+      pa.nb = plane_orbitals(n, (long)bs * n);
       TRY(launch_plane(n, PM_VPSI, pa, (bs + pa.nb - 1) / pa.nb, st));
       TRY(ph_end(c, PH_VPSI));
       TRY(ph_begin(c, PH_ZR2G));
-      zargs_base(c, z, 0);
+      z = zargs_base(c);
       /* -H psi (local part) is kept only on the last step, for the energy
        * tail; the other steps write c1 + dte (local -H psi) straight into c2
        * and the KB apply adds dte times the nonlocal part in place */
@@ -1402,7 +1412,7 @@ static int ctx_clear_state(cpsd_dev *c)
 {
    hipStream_t st = c->stream;
    const size_t orb = (size_t)c->ne * c->ngp, ee = (size_t)c->ne * c->ne;
-   const size_t plane = (size_t)c->n * c->n * c->nh;
+   const size_t plane = (size_t)c->n * c->ncol;
    struct { void *p; size_t bytes; } z[] = {
       {c->Cbase, 2 * orb * sizeof(double2)}, {c->CP, orb * sizeof(double2)},
       {c->T, (size_t)c->ne * plane * sizeof(double2)}, {c->Tv, plane * sizeof(double2)},
@@ -1469,7 +1479,7 @@ static int ctx_get(cpsd_dev *c, double *c1, double *c2, double *cpsi, double *dn
    if (c2) TRY(ctx_get_orb(c, c->Cbase + (size_t)c->cur * orb, c2));
    if (cpsi) TRY(ctx_get_orb(c, c->CP, cpsi));
    if (dn) {
-      TRY(sd_pad_real(c->dn, c->n, c->realbuf, st));
+      TRY(sd_pad_real(c->dn, fft_slots(c->n), 2, c->realbuf, st));
       CPSD_CHECK(hipMemcpyAsync(dn, c->realbuf, (size_t)c->n2ft3d * sizeof(double),
                                 hipMemcpyDeviceToHost, st));
    }
@@ -2015,6 +2025,11 @@ extern "C" long cpsd_dev_debug_fetch(cpsd_dev *h, int what, double *out, long ca
    default: cpsd_set_error("debug_fetch: unknown buffer %d", what); return -1;
    }
    if ((long)nd > cap) { cpsd_set_error("debug_fetch: capacity %ld < %zu", cap, nd); return -1; }
+   if (what == 0 || what == 1 || what == 12) {   /* real-space fields, in natural order */
+      TRY(sd_pad_real(static_cast<const double *>(src), fft_slots(h->n), 0, h->realbuf, h->stream));
+      CPSD_CHECK(hipStreamSynchronize(h->stream));
+      src = h->realbuf;
+   }
    if (hipMemcpy(out, src, nd * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess) {
       cpsd_set_error("debug_fetch: copy failed");
       return -1;
@@ -2194,37 +2209,31 @@ extern "C" void cpsd_rotate(const int ispin, const int *ne, const int n2ft3d, do
 struct FftCtx {
    int n, nbatch;
    hipStream_t stream;
-   int *frs, *frl, *fro;
    double2 *tw, *T, *A;
 };
-static FftCtx g_fft = {0, 0, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+static FftCtx g_fft = {0, 0, nullptr, nullptr, nullptr, nullptr};
 
 static int fft_ctx(int n, int nbatch)
 {
    if (!fft_supported(n)) { cpsd_set_error("FFT grid %d is not supported", n); return -1; }
    if (g_fft.n == n && g_fft.nbatch >= nbatch) return 0;
    if (g_fft.stream) {
-      (void)hipFree(g_fft.frs); (void)hipFree(g_fft.frl); (void)hipFree(g_fft.fro);
       (void)hipFree(g_fft.tw); (void)hipFree(g_fft.T); (void)hipFree(g_fft.A);
    } else {
       CPSD_CHECK(hipStreamCreate(&g_fft.stream));
    }
    const int nh = n / 2 + 1;
-   std::vector<int> frs(n * n, 0), frl(n * n, nh), fro(n * n);
-   for (int r = 0; r < n * n; ++r) fro[r] = r * nh;
    std::vector<double2> tw(n);
    for (int m = 0; m < n; ++m) {
       const double a = 2.0 * M_PI * (double)m / (double)n;
       tw[m] = make_double2(cos(a), sin(a));
    }
    g_fft.n = n; g_fft.nbatch = nbatch;
-   TRY(dalloc(&g_fft.frs, n * n)); TRY(dalloc(&g_fft.frl, n * n)); TRY(dalloc(&g_fft.fro, n * n));
    TRY(dalloc(&g_fft.tw, n));
    TRY(dalloc(&g_fft.T, (size_t)nbatch * n * n * nh));
    TRY(dalloc(&g_fft.A, (size_t)nbatch * n * n * nh));
    hipStream_t st = g_fft.stream;
-   TRY(h2d(g_fft.frs, frs.data(), n * n, st)); TRY(h2d(g_fft.frl, frl.data(), n * n, st));
-   TRY(h2d(g_fft.fro, fro.data(), n * n, st)); TRY(h2d(g_fft.tw, tw.data(), n, st));
+   TRY(h2d(g_fft.tw, tw.data(), n, st));
    CPSD_CHECK(hipStreamSynchronize(st));
    return 0;
 }
@@ -2233,27 +2242,9 @@ static int fft_run(int dir, int n, int nbatch, double *Ah)
 {
    TRY(fft_ctx(n, nbatch));
    hipStream_t st = g_fft.stream;
-   const int nh = n / 2 + 1;
-   const size_t per = (size_t)n * n * nh;  /* complex = (n+2) n n / 2 */
+   const size_t per = (size_t)n * n * (n / 2 + 1);  /* complex = (n+2) n n / 2 */
    CPSD_CHECK(hipMemcpyAsync(g_fft.A, Ah, (size_t)nbatch * per * sizeof(double2), hipMemcpyHostToDevice, st));
-   ZArgs z;
-   memset(&z, 0, sizeof z);
-   z.rows.rstart = g_fft.frs; z.rows.rlen = g_fft.frl; z.rows.roff = g_fft.fro; z.rows.nhc = nh;
-   z.tw = g_fft.tw;
-   PlaneArgs pa;
-   memset(&pa, 0, sizeof pa);
-   pa.T = g_fft.T; pa.nhload = nh; pa.tw = g_fft.tw; pa.nbatch = nbatch;
-   if (dir > 0) {
-      z.src = g_fft.A; z.sstride = per; z.T = g_fft.T;
-      TRY(launch_zpass_g2r(n, SRC_PACKED, z, nbatch, st));
-      pa.rout = reinterpret_cast<double *>(g_fft.A);
-      TRY(launch_plane(n, PM_C2R_OUT, pa, nbatch, st));
-   } else {
-      pa.rin = reinterpret_cast<const double *>(g_fft.A);
-      TRY(launch_plane(n, PM_R2C_IN, pa, nbatch, st));
-      z.T = g_fft.T; z.out = g_fft.A; z.ostride = per;
-      TRY(launch_zpass_r2g(n, DST_FULL, z, nbatch, st));
-   }
+   TRY(launch_fft3d(dir, n, nbatch, g_fft.A, g_fft.T, g_fft.tw, st));
    CPSD_CHECK(hipMemcpyAsync(Ah, g_fft.A, (size_t)nbatch * per * sizeof(double2), hipMemcpyDeviceToHost, st));
    CPSD_CHECK(hipStreamSynchronize(st));
    return 0;

@@ -6,12 +6,12 @@
  *   - orbitals C1, C2, CP: [ne][ngp] complex (interleaved re, im), only the
  *     masked G vectors are stored ("packed"), ordered as the reference's
  *     half-complex grid (kx fastest, then ky, then kz; ccpsdv3/get_g.c:20-34).
- *     Each (ky,kz) row of the grid contributes one contiguous kx interval,
- *     described by rstart/rlen/roff.  ngp = ng rounded up to 64; the tail
- *     is zero and carries weight 0.
- *   - T: z-transformed orbitals [ne][z][ky][kx], kx < N/2+1 (the y/x passes
- *     read one (ky,kx) plane per z).
- *   - real-space fields (dn, V, xcp, xce): dense [z][y][x] of N^3 doubles.
+ *     Each (ky,kz) row of the grid contributes one contiguous kx interval.
+ *     ngp = ng rounded up to 64; the tail is zero and carries weight 0.
+ *   - T: z-transformed orbitals [ne][z][columns], the (ky, kx) columns inside
+ *     the cutoff only (ColTable; the y/x passes read one plane per z).
+ *   - real-space fields (dn, V, xcp, xce): N^3 doubles in the slot order of the
+ *     plane passes (PlaneArgs).
  *   - projectors B: [nproj][ngp] complex, beta_{I,lm}(G) = S_I(G) vnl(G)
  *     (times i for p channels), ions ordered as in the reference loops.
  */
@@ -50,25 +50,32 @@ static inline int dyn_lds_once(const void *k, int bytes, std::atomic<unsigned lo
 
 /* ---- FFT ------------------------------------------------------------ */
 
-enum { SRC_PACKED = 0, SRC_VG = 1 };
 /* DST_SD: out = c1 + dte (-scal1 V psi - tg c1), the SD update before the
  * nonlocal term (used when -H psi itself is not needed afterwards) */
-enum { DST_HPSI = 0, DST_DNG = 1, DST_FULL = 2, DST_SD = 3 };
+enum { DST_HPSI = 0, DST_FULL = 2, DST_SD = 3 };
 enum { PM_DENSITY = 0, PM_VTOT = 1, PM_VPSI = 2, PM_C2R_OUT = 3, PM_R2C_DN = 4, PM_R2C_IN = 5 };
 
-struct RowTable {
-   const int *rstart, *rlen, *roff;  /* N*N rows each */
-   int nhc;                          /* kx columns that can be nonzero */
+/* The z-transformed intermediate T holds, per z, the (ky, kx) columns that can
+ * be nonzero: for the cutoff sphere the disc of its projection, 0.79 of the
+ * N x N/2 grid.  Row ky has kx = 0 .. len(ky) - 1 at offset off(ky), rows
+ * padded to 8 columns; P columns per plane.  The z passes run over the
+ * columns c < P whatever row they belong to. */
+struct ColTable {
+   const int *rows;      /* N entries len << 16 | off, or null: every row holds kx = 0..N/2 at ky (N/2 + 1) */
+   const int *gmap;      /* [N][P]: packed coefficient of (kz, column) or -1; null with rows null, when the
+                          * coefficient is kz N (N/2 + 1) + column of the reference's full grid */
+   int P;                /* columns per plane (N (N/2 + 1) with rows null) */
+   int nyq;              /* some row holds the Nyquist column kx = N/2 */
 };
 
 struct ZArgs {
-   RowTable rows;
+   ColTable cols;
    const double2 *src;   /* packed (or full-grid) input, batch stride sstride */
    size_t sstride;
-   double2 *T;           /* [batch][z][ky][NH] */
+   double2 *T;           /* [batch][z][P] */
    const double2 *tw;    /* exp(+2 pi i m/N), m < N */
-   /* SRC_VG */
-   const double2 *vall, *dng;
+   /* the local potential in G space: vall scal2 + dng vc */
+   const double2 *vall;
    const double *vc;
    double scal2;
    /* r->G outputs */
@@ -78,19 +85,23 @@ struct ZArgs {
    const double *tg;
    double scal1;
    double dte;           /* DST_SD */
-   /* set by the launcher: orbitals per workgroup (blockIdx.z covers
-    * [z*bper, min(nbatch, (z+1)*bper))) */
+   /* set by the launcher: orbitals per workgroup */
    int nbatch, bper;
-   /* FP32 transform (SRC_PACKED, DST_HPSI, DST_SD): T holds float2 at the
-    * same base pointer; inputs and outputs stay FP64 */
+   /* FP32 transform (orbitals): T holds float2 at the same base pointer;
+    * inputs and outputs stay FP64 */
    int fp32;
 };
 
+/* Real-space fields (density partials, dn, xcp, xce, V) are stored in the slot
+ * order the plane passes hold them in: pair (x, x + 1) of point (z, y, x) at
+ * pair index ((z NX1 + k1) NX2 + k2) N + s with x / 2 = k1 + NX1 k2 and y in
+ * slot s, so that every pass reads and writes them along consecutive lanes.
+ * fft_slots() gives the factors. */
 struct PlaneArgs {
-   double2 *T;           /* [batch][z][ky][NH] (in place for PM_VPSI) */
-   int nhload;           /* kx columns loaded (others are zero) */
+   ColTable cols;
+   double2 *T;           /* [batch][z][P] (in place for PM_VPSI) */
    const double2 *tw;
-   int b0, nb;           /* PM_DENSITY: orbitals [b0 + blockIdx.y*nb, ...) */
+   int nb;               /* PM_DENSITY, PM_VPSI: orbitals per workgroup */
    int accumulate;       /* PM_DENSITY: add into dnpart instead of overwriting */
    int nbatch;
    double *dnpart;       /* PM_DENSITY: [blocks][N^3] */
@@ -105,14 +116,20 @@ struct PlaneArgs {
 };
 
 int fft_supported(int n);
-int launch_zpass_g2r(int n, int src, const ZArgs &a, int nbatch, hipStream_t s);
+int launch_zpass_g2r(int n, const ZArgs &a, int nbatch, hipStream_t s);
 int launch_zpass_r2g(int n, int dst, const ZArgs &a, int nbatch, hipStream_t s);
+/* one field in place: T -> out = its G coefficients -> T of vall scal2 + out vc */
+int launch_zpass_field(int n, const ZArgs &a, hipStream_t s);
 int launch_plane(int n, int mode, const PlaneArgs &a, int nblocks, hipStream_t s);
-/* workgroups of the density plane pass one CU holds at once */
+/* nbatch transforms of the reference's full grid in place in A (dir +1:
+ * half-complex to padded real, -1 the reverse); T: as many complex values */
+int launch_fft3d(int dir, int n, int nbatch, double2 *A, double2 *T, const double2 *tw, hipStream_t s);
+/* workgroups per CU that the grouping of the density sum is made for */
 int plane_density_occupancy(int n, int fp32);
-/* the FP64 density and V psi passes at grid n prefetch the next orbital's
- * plane (several orbitals per workgroup pay for it) */
-int plane_prefetch_on(int n);
+/* orbitals per V psi workgroup for `planes` (z plane, orbital) pairs */
+int plane_orbitals(int n, long planes);
+struct FftSlots { int n, ny1, ny2, nx1, nx2; };
+FftSlots fft_slots(int n);
 
 /* ---- GEMM ------------------------------------------------------------- */
 

@@ -7,18 +7,23 @@
  *   DIR = +1 : X_k = sum_n x_n exp(+2 pi i nk/N)   (backward, cr_fft3b)
  * Transforms are unnormalised.
  *
- * A length-N transform with N = N1*N2 runs in place in LDS as two register
- * passes separated by one barrier.  Slot s = N2*a + b holds logical index
- * a + N1*b in the "transposed" order:
- *   lds_fft_nat2tr: natural input  -> transposed output
- *   lds_fft_tr2nat: transposed input -> natural output
- * Every item reads and writes only its own slots inside a pass, so no extra
- * scratch is needed; callers un-permute indices when they move data to or
- * from global memory (tr_index below).
+ * A length-N transform with N = N1*N2 is two register passes with one trip
+ * through LDS between them.  Slot s = N2*a + b holds logical index a + N1*b in
+ * the "transposed" order:
+ *   nat2tr: natural input -> transposed output.  Pass 1, item n2: elements
+ *           N2*n1 + n2, DFT over n1, twiddles; pass 2, item k1: slots
+ *           N2*k1 + n2, DFT over n2, in place.
+ *   tr2nat: transposed input -> natural output.  Pass 1, item n1: slots
+ *           N2*n1 + n2, DFT over n2, twiddles; pass 2, item k2: slots
+ *           N2*n1 + k2, DFT over n1, natural index N2*k1 + k2.
+ * An item reads and writes the same slots, so a pass needs no scratch, and
+ * pass 2 of an inverse transform holds exactly the slots that pass 1 of the
+ * forward transform needs.
  */
 #pragma once
 #include <hip/hip_runtime.h>
 #include "small_twiddles.h"
+#include <type_traits>
 
 /* complex helpers for the FP64 (double2) and FP32 (float2) transforms */
 template<typename V> struct Cx;
@@ -159,15 +164,6 @@ template<int DIR> struct DFT<10, DIR> { template<typename V> static __device__ _
 template<int DIR> struct DFT<12, DIR> { template<typename V> static __device__ __forceinline__ void run(V *v) { dft_composite<4, 3, DIR>(v); } };
 template<int DIR> struct DFT<16, DIR> { template<typename V> static __device__ __forceinline__ void run(V *v) { dft_composite<4, 4, DIR>(v); } };
 
-/* twiddle exp(DIR 2 pi i m / N) from a table of exp(+2 pi i m / N), m < N */
-template<int DIR, typename V>
-__device__ __forceinline__ V twiddle(const V *__restrict__ tw, int m)
-{
-   V w = tw[m];
-   if (DIR < 0) w.y = -w.y;
-   return w;
-}
-
 /* logical index held by slot s in the transposed order of N = N1*N2 */
 template<int N1, int N2>
 __device__ __forceinline__ int tr_index(int s) { return s / N2 + N1 * (s % N2); }
@@ -176,93 +172,105 @@ __device__ __forceinline__ int tr_index(int s) { return s / N2 + N1 * (s % N2); 
 template<int N1, int N2>
 __device__ __forceinline__ int tr_slot(int j) { return N2 * (j % N1) + j / N1; }
 
-/* count transforms; element j of transform f sits at buf[f*fs + j*es].
- * tw: table of exp(+2 pi i m / (N*tws)), twiddle W_N^m read at m*tws.  */
-template<int N1, int N2, int DIR, typename V>
-__device__ __forceinline__ void lds_fft_nat2tr(V *buf, int count, int fs, int es,
-                                               const V *__restrict__ tw, int tws)
+/* a value the compiler may not look through.  The passes below take and leave
+ * their values so: products of one stage are never contracted into the sums of
+ * the next, and which products of a DFT become fused multiply-adds does not
+ * depend on where a kernel loads its inputs from or stores its outputs to, so
+ * every kernel rounds a transform the same way. */
+__device__ __forceinline__ void opaque(double2 &v) { asm("" : "+v"(v.x), "+v"(v.y)); }
+__device__ __forceinline__ void opaque(float2 &v) { asm("" : "+v"(v.x), "+v"(v.y)); }
+template<int L, typename V> __device__ __forceinline__ void opaque_all(V (&v)[L])
 {
-   constexpr int N = N1 * N2;
-   for (int it = threadIdx.x; it < count * N2; it += blockDim.x) {
-      const int f = it % count, n2 = it / count;
-      V *p = buf + f * fs;
-      V v[N1];
 #pragma unroll
-      for (int n1 = 0; n1 < N1; ++n1) v[n1] = p[(N2 * n1 + n2) * es];
-      DFT<N1, DIR>::run(v);
-#pragma unroll
-      for (int k1 = 1; k1 < N1; ++k1) v[k1] = cmul(v[k1], twiddle<DIR>(tw, ((n2 * k1) % N) * tws));
-#pragma unroll
-      for (int k1 = 0; k1 < N1; ++k1) p[(N2 * k1 + n2) * es] = v[k1];
-   }
-   __syncthreads();
-   for (int it = threadIdx.x; it < count * N1; it += blockDim.x) {
-      const int f = it % count, k1 = it / count;
-      V *p = buf + f * fs;
-      V v[N2];
-#pragma unroll
-      for (int n2 = 0; n2 < N2; ++n2) v[n2] = p[(N2 * k1 + n2) * es];
-      DFT<N2, DIR>::run(v);
-#pragma unroll
-      for (int k2 = 0; k2 < N2; ++k2) p[(N2 * k1 + k2) * es] = v[k2];
-   }
-   __syncthreads();
+   for (int i = 0; i < L; ++i) opaque(v[i]);
 }
 
-template<int N1, int N2, int DIR, typename V>
-__device__ __forceinline__ void lds_fft_tr2nat(V *buf, int count, int fs, int es,
-                                               const V *__restrict__ tw, int tws)
+/* DFT of an item's L values */
+template<int L, int DIR, typename V>
+__device__ __forceinline__ void pass_dft(V (&v)[L])
 {
-   constexpr int N = N1 * N2;
-   for (int it = threadIdx.x; it < count * N1; it += blockDim.x) {
-      const int f = it % count, n1 = it / count;
-      V *p = buf + f * fs;
-      V v[N2];
-#pragma unroll
-      for (int n2 = 0; n2 < N2; ++n2) v[n2] = p[(N2 * n1 + n2) * es];
-      DFT<N2, DIR>::run(v);
-#pragma unroll
-      for (int k2 = 1; k2 < N2; ++k2) v[k2] = cmul(v[k2], twiddle<DIR>(tw, ((n1 * k2) % N) * tws));
-#pragma unroll
-      for (int k2 = 0; k2 < N2; ++k2) p[(N2 * n1 + k2) * es] = v[k2];
-   }
-   __syncthreads();
-   for (int it = threadIdx.x; it < count * N2; it += blockDim.x) {
-      const int f = it % count, k2 = it / count;
-      V *p = buf + f * fs;
-      V v[N1];
-#pragma unroll
-      for (int n1 = 0; n1 < N1; ++n1) v[n1] = p[(N2 * n1 + k2) * es];
-      DFT<N1, DIR>::run(v);
-#pragma unroll
-      for (int k1 = 0; k1 < N1; ++k1) p[(N2 * k1 + k2) * es] = v[k1];
-   }
-   __syncthreads();
+   opaque_all(v);
+   DFT<L, DIR>::run(v);
+   opaque_all(v);
 }
+
+/* v W, the products contracted in a fixed way: W = w (DIR = +1) or conj w; for
+ * DIR = +1 the imaginary part adds Re v Im w to the rounded Im v Re w when
+ * vx_first, and the other way round otherwise */
+__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+template<int DIR, typename V>
+__device__ __forceinline__ V twiddle_mul(V v, V w, bool vx_first)
+{
+   using R = typename Cx<V>::R;
+   const R yy = v.y * w.y;
+   if (DIR < 0) return Cx<V>::mk(fma_(v.x, w.x, yy), fma_(v.y, w.x, -(v.x * w.y)));
+   return Cx<V>::mk(fma_(v.x, w.x, -yy), vx_first ? fma_(v.x, w.y, v.y * w.x) : fma_(v.y, w.x, v.x * w.y));
+}
+
+/* DFT of item i's L values with the twiddles after pass 1, v[k] *= W_N^(i k),
+ * from a table of exp(+2 pi i m / (N tws)) read at m tws.  The forms of the
+ * products are those that earlier builds of this library compiled to, kept so
+ * that results stay the same to the bit. */
+template<int N, int L, int DIR, typename V>
+__device__ __forceinline__ void pass_dft_tw(V (&v)[L], int i, const V *__restrict__ tw, int tws)
+{
+   opaque_all(v);
+   DFT<L, DIR>::run(v);
+#pragma unroll
+   for (int k = 1; k < L; ++k)
+      v[k] = twiddle_mul<DIR>(v[k], tw[((i * k) % N) * tws], (L == 3 && k == 1) || (L == 5 && k < 3) || (L == 8 && k == 2));
+   opaque_all(v);
+}
+
+/* element i of an array below 4 GB: the address is a uniform base plus a
+ * 32-bit offset, one register per element instead of two */
+template<typename E> __device__ __forceinline__ E &at(E *base, unsigned i)
+{
+   using B = typename std::conditional<std::is_const<E>::value, const char, char>::type;
+   return *reinterpret_cast<E *>(reinterpret_cast<B *>(base) + (size_t)(unsigned)(i * (unsigned)sizeof(E)));
+}
+
+/* an index whose addresses are recomputed at each use, not held in registers
+ * across the orbital loop */
+__device__ __forceinline__ int fresh(int i)
+{
+   asm volatile("" : "+v"(i));
+   return i;
+}
+
+/* the scheduler finishes one item before it starts the next: the items of an
+ * unrolled loop would otherwise be interleaved and their registers spilled */
+__device__ __forceinline__ void item_end() { __builtin_amdgcn_sched_barrier(0); }
 
 /* ------------------------------------------------ grid configurations */
 
-/* N = NY1*NY2 for the y and z passes, N/2 = NX1*NX2 for the real x pass */
+/* N = NY1*NY2 for the y and z passes, N/2 = NX1*NX2 for the real x pass;
+ * PLANE_THREADS: threads of a plane workgroup, chosen so that the items of
+ * each pass (N/2 NY2, N/2 NY1, N x_units and N NX1 of them) fill whole
+ * rounds */
 template<int N> struct GridCfg;
-/* z pass: KXB kx columns per workgroup of ZT threads; whole kx rows up to
- * N = 96 (no row is split between workgroups), two balanced halves at 128 */
-#define GRID_CFG(n, y1, y2, x1, x2, pt, kxb, zt)                               \
+#define GRID_CFG(n, y1, y2, x1, x2, pt)                                        \
    template<> struct GridCfg<n> {                                              \
       static constexpr int NY1 = y1, NY2 = y2, NX1 = x1, NX2 = x2;             \
-      static constexpr int PLANE_THREADS = pt, KXB = kxb, ZT = zt;             \
+      static constexpr int PLANE_THREADS = pt;                                 \
    };
-GRID_CFG(8,   4,  2, 2, 2, 256, 5,  256)
-GRID_CFG(12,  4,  3, 3, 2, 256, 7,  256)
-GRID_CFG(16,  4,  4, 4, 2, 256, 9,  256)
-GRID_CFG(20,  5,  4, 5, 2, 256, 11, 256)
-GRID_CFG(24,  6,  4, 4, 3, 256, 13, 256)
-GRID_CFG(32,  8,  4, 4, 4, 256, 17, 256)
-GRID_CFG(40,  8,  5, 5, 4, 256, 21, 256)
-GRID_CFG(48,  8,  6, 6, 4, 256, 25, 256)
-GRID_CFG(64,  8,  8, 8, 4, 256, 33, 256)
-GRID_CFG(80,  10, 8, 8, 5, 512, 41, 512)
-GRID_CFG(96,  8, 12, 8, 6, 512, 49, 512)
-GRID_CFG(128, 8, 16, 8, 8, 512, 33, 512)
+GRID_CFG(8,   4,  2, 2, 2, 64)
+GRID_CFG(12,  4,  3, 3, 2, 64)
+GRID_CFG(16,  4,  4, 4, 2, 64)
+GRID_CFG(20,  5,  4, 5, 2, 128)
+GRID_CFG(24,  6,  4, 4, 3, 128)
+GRID_CFG(32,  8,  4, 4, 4, 128)
+GRID_CFG(40,  8,  5, 5, 4, 256)
+GRID_CFG(48,  8,  6, 6, 4, 256)
+GRID_CFG(64,  8,  8, 8, 4, 256)
+GRID_CFG(80,  10, 8, 8, 5, 256)
+GRID_CFG(96,  8, 12, 8, 6, 512)
+GRID_CFG(128, 8, 16, 8, 8, 512)
 #undef GRID_CFG
+
+/* columns and threads of a z-pass workgroup */
+#define ZKB 32
+#define ZT 256
 
 #define CPSD_FOR_EACH_GRID(X) X(8) X(12) X(16) X(20) X(24) X(32) X(40) X(48) X(64) X(80) X(96) X(128)

@@ -8,8 +8,8 @@
  * serving loops, harnesses that forbid hipMalloc) call
  * cpsd_fft3d_batch_noalloc() instead: the grid stays in their own device
  * buffer and is transformed in place, and the two things the transform needs
- * besides it -- the z-transformed intermediate T and the row/twiddle tables
- * of the kernels -- live in `scratch`, a file-scope device array of
+ * besides it -- the z-transformed intermediate T and the twiddle table of the
+ * kernels -- live in `scratch`, a file-scope device array of
  * CPSD_NOALLOC_SCRATCH_BYTES that each GPU holds until the process ends.
  *
  * The kernels are the ones cpsd_fft3d_batch() launches (z pass and fused
@@ -19,7 +19,6 @@
 #include "../../include/cpsd_abi.h"
 
 #include <math.h>
-#include <string.h>
 #include <mutex>
 
 static __device__ __align__(256) unsigned char scratch[CPSD_NOALLOC_SCRATCH_BYTES];
@@ -53,9 +52,11 @@ static int scratch_on_current_device(unsigned char **out)
    return 0;
 }
 
-/* byte offsets of the pieces of the scratch array for grid n */
+/* byte offsets of the pieces of the scratch array for grid n.  The room of the
+ * three N^2 index tables ahead of the twiddles is unused; it is kept because
+ * it is part of how many transforms of a grid fit, which callers ask for. */
 struct NoallocLayout {
-   size_t frs, frl, fro, tw, T, end;
+   size_t tw, T, end;
 };
 
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -64,27 +65,17 @@ static NoallocLayout noalloc_layout(int n, int nbatch)
 {
    const size_t rows = (size_t)n * n * sizeof(int);
    NoallocLayout L;
-   L.frs = 0;
-   L.frl = align256(L.frs + rows);
-   L.fro = align256(L.frl + rows);
-   L.tw = align256(L.fro + rows);
+   L.tw = align256(align256(align256(rows) + rows) + rows);
    L.T = align256(L.tw + (size_t)n * sizeof(double2));
    L.end = L.T + (size_t)nbatch * n * n * (n / 2 + 1) * sizeof(double2);
    return L;
 }
 
-/* the full-grid row table (every (ky,kz) row holds kx = 0..N/2) and the
- * twiddles exp(+2 pi i m/N), written on the device on every call, so a call
- * never depends on what an earlier call on another grid left there */
-__global__ void k_noalloc_tables(int n, int *frs, int *frl, int *fro, double2 *tw)
+/* the twiddles exp(+2 pi i m/N), written on the device on every call, so a
+ * call never depends on what an earlier call on another grid left there */
+__global__ void k_noalloc_twiddles(int n, double2 *tw)
 {
-   const int nh = n / 2 + 1;
-   const int r = blockIdx.x * blockDim.x + threadIdx.x;
-   if (r < n * n) {
-      frs[r] = 0;
-      frl[r] = nh;
-      fro[r] = r * nh;
-   }
+   const int r = threadIdx.x;
    if (r < n) {
       double s, c;
       sincospi(2.0 * (double)r / (double)n, &s, &c);
@@ -125,36 +116,11 @@ extern "C" int cpsd_fft3d_batch_noalloc(int dir, int nfft, int nbatch, double *A
    unsigned char *base = nullptr;
    if (scratch_on_current_device(&base) != 0) return -1;
    const NoallocLayout L = noalloc_layout(nfft, nbatch);
-   int *frs = reinterpret_cast<int *>(base + L.frs);
-   int *frl = reinterpret_cast<int *>(base + L.frl);
-   int *fro = reinterpret_cast<int *>(base + L.fro);
    double2 *tw = reinterpret_cast<double2 *>(base + L.tw);
    double2 *T = reinterpret_cast<double2 *>(base + L.T);
    hipStream_t st = static_cast<hipStream_t>(stream);
 
-   const int n = nfft, nh = n / 2 + 1;
-   hipLaunchKernelGGL(k_noalloc_tables, dim3((n * n + 255) / 256), dim3(256), 0, st, n, frs, frl, fro, tw);
+   hipLaunchKernelGGL(k_noalloc_twiddles, dim3(1), dim3(128), 0, st, nfft, tw);
    CPSD_CHECK(hipGetLastError());
-
-   const size_t per = (size_t)n * n * nh;  /* complex values per transform */
-   double2 *Ac = reinterpret_cast<double2 *>(A);
-   ZArgs z;
-   memset(&z, 0, sizeof z);
-   z.rows.rstart = frs; z.rows.rlen = frl; z.rows.roff = fro; z.rows.nhc = nh;
-   z.tw = tw;
-   PlaneArgs pa;
-   memset(&pa, 0, sizeof pa);
-   pa.T = T; pa.nhload = nh; pa.tw = tw; pa.nbatch = nbatch;
-   if (dir > 0) {
-      z.src = Ac; z.sstride = per; z.T = T;
-      if (launch_zpass_g2r(n, SRC_PACKED, z, nbatch, st) != 0) return -1;
-      pa.rout = A;
-      if (launch_plane(n, PM_C2R_OUT, pa, nbatch, st) != 0) return -1;
-   } else {
-      pa.rin = A;
-      if (launch_plane(n, PM_R2C_IN, pa, nbatch, st) != 0) return -1;
-      z.T = T; z.out = Ac; z.ostride = per;
-      if (launch_zpass_r2g(n, DST_FULL, z, nbatch, st) != 0) return -1;
-   }
-   return 0;
+   return launch_fft3d(dir, nfft, nbatch, reinterpret_cast<double2 *>(A), T, tw, st);
 }

@@ -42,15 +42,19 @@ __global__ void k_unpack(const double2 *__restrict__ packed, size_t pstride, con
    full[i * fstride + g] = (p >= 0) ? packed[i * pstride + p] : make_double2(0.0, 0.0);
 }
 
-/* dense N^3 real field -> padded (N+2) rows with zeroed pads */
-__global__ void k_pad_real(const double *__restrict__ dense, int n, double *__restrict__ padded)
+/* slot-ordered real field -> rows [z][y][x] with `pad` zeroed reals each */
+__global__ void k_pad_real(const double *__restrict__ field, FftSlots f, int pad, double *__restrict__ out)
 {
    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-   const size_t rows = (size_t)n * n;
-   if (idx >= rows * (n + 2)) return;
-   const size_t r = idx / (n + 2);
-   const int x = (int)(idx % (n + 2));
-   padded[idx] = (x < n) ? dense[r * n + x] : 0.0;
+   const int n = f.n, ld = n + pad;
+   if (idx >= (size_t)n * n * ld) return;
+   const int x = (int)(idx % ld), y = (int)(idx / ld % n), z = (int)(idx / ((size_t)ld * n));
+   double v = 0.0;
+   if (x < n) {
+      const int j = x >> 1, s = f.ny2 * (y % f.ny1) + y / f.ny1;
+      v = field[2 * (((size_t)(z * f.nx1 + j % f.nx1) * f.nx2 + j / f.nx1) * n + s) + (x & 1)];
+   }
+   out[idx] = v;
 }
 
 /* ------------------------------------- structure factors and projectors */
@@ -1173,10 +1177,10 @@ int sd_unpack(const double2 *packed, size_t pstride, const int *pidx, int nfft3d
    return 0;
 }
 
-int sd_pad_real(const double *dense, int n, double *padded, hipStream_t s)
+int sd_pad_real(const double *field, const FftSlots &f, int pad, double *out, hipStream_t s)
 {
-   const size_t tot = (size_t)n * n * (n + 2);
-   hipLaunchKernelGGL(k_pad_real, g1(tot), dim3(256), 0, s, dense, n, padded);
+   const size_t tot = (size_t)f.n * f.n * (f.n + pad);
+   hipLaunchKernelGGL(k_pad_real, g1(tot), dim3(256), 0, s, field, f, pad, out);
    CPSD_CHECK(hipGetLastError());
    return 0;
 }
