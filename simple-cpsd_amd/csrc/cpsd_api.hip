@@ -865,6 +865,7 @@ static int sd_step(cpsd_dev *c, double dte, int last, int fp64)
     * forms the products of its step d = c2 - c1 only */
    const int dgram = sb && c->g11_valid;
    const int carry = c->g11_valid && (dgram || !c->g11_drift);
+   const int one = !pstep && lagrange_one(ne);   /* the Lagrange kernel forms the s matrices itself */
    TRY(ph_begin(c, PH_GRAM));
    if (dgram) {
       int sp = 0;
@@ -877,7 +878,7 @@ static int sd_step(cpsd_dev *c, double dte, int last, int fp64)
       if (pstep)
          TRY(sd_smat_precond(c->Gm, c->g11c[c->g11_idx], ne, c->cur, dte, c->DP, c->s11, c->s12, c->s21, c->s22,
                              c->bar, st));
-      else
+      else if (!one)
          TRY(sd_smat(c->Gm, c->g11c[c->g11_idx], ne, c->cur, dte, c->s11, c->s12, c->s21, c->s22, c->bar, st));
       TRY(ph_end(c, PH_GRAMRED));
    } else {
@@ -902,7 +903,7 @@ static int sd_step(cpsd_dev *c, double dte, int last, int fp64)
       if (pstep)
          TRY(sd_smat_precond(c->Gm, carry ? c->g11c[c->g11_idx] : nullptr, ne, c->cur, dte, c->DP, c->s11,
                              c->s12, c->s21, c->s22, c->bar, st));
-      else
+      else if (!one)
          TRY(sd_smat(c->Gm, carry ? c->g11c[c->g11_idx] : nullptr, ne, c->cur, dte, c->s11, c->s12, c->s21,
                      c->s22, c->bar, st));
       TRY(ph_end(c, PH_GRAMRED));
@@ -914,6 +915,9 @@ static int sd_step(cpsd_dev *c, double dte, int last, int fp64)
       l.ne = ne; l.s11 = c->s11; l.s12 = c->s12; l.s21 = c->s21; l.s22 = c->s22;
       l.X = c->LX; l.st1 = c->st1; l.lmd = c->lmd; l.wgmax = c->wgmax; l.info = c->info;
       l.bar = c->bar; l.err = c->err;
+      if (one) {
+         l.Gm = c->Gm; l.g11c = carry ? c->g11c[c->g11_idx] : nullptr; l.c1_second = c->cur; l.dte = dte;
+      }
       l.itmax = 30;
       c->lag_itmax = l.itmax;
       TRY(sd_lagrange(l, st));

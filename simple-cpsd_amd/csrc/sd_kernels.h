@@ -16,7 +16,8 @@ struct StructArgs {
 
 struct LagArgs {
    int ne;
-   const double *s11, *s12, *s21, *s22;
+   double *s11;
+   const double *s12, *s21, *s22;
    double *X;        /* 2 ne^2 */
    double *st1;      /* ne^2 */
    double *lmd;
@@ -24,6 +25,11 @@ struct LagArgs {
    double *info;     /* [iterations, last max|dX|] */
    unsigned *bar;    /* grid-barrier counter, zero at launch (sd_smat clears it) */
    int *err;
+   /* lagrange_one(ne) only: the s matrices are formed from the Gram matrix (as
+    * sd_smat does; s11 is written) instead of read where Gm is set */
+   const double *Gm = nullptr, *g11c = nullptr;
+   int c1_second = 0;
+   double dte = 0.0;
    int itmax = 30;   /* the reference's ITERLMD (ccpsdv3/cpsd.c:19) */
 };
 
@@ -79,6 +85,8 @@ int sd_precond_lmd(double *lmd, const double *DP, int ne, double dte, hipStream_
 int sd_gram_next(const double *Gm, const double *g11, int ne, int c1_second, const double *lmd, double dte,
                  double *work, double *out, hipStream_t s);
 int sd_kbcoef(const double *P, int nproj, int ne, const double *pnrm, double scal2, double *X, hipStream_t s);
+/* the orbital count is solved by one workgroup, without grid barriers */
+int lagrange_one(int ne);
 int sd_lagrange(const LagArgs &a, hipStream_t s);
 int sd_energy(const EnergyArgs &a, hipStream_t s);
 int sd_hml(const double *M, int ne, double *hml, hipStream_t s);

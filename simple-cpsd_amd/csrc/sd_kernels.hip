@@ -346,17 +346,13 @@ __global__ void k_erfc_as(const double *__restrict__ w, int n, double *__restric
 /* ------------------------------------------- overlaps -> s matrices */
 
 /* Gram matrix Gm (2ne x 2ne, row-major) of the two orbital blocks (C1 first
- * unless c1_second) -> the four ne x ne
- * matrices of ccpsdv3/cpsd.c:415-437 (column-major).  s21 and s12 are each
- * filled from one triangle and mirrored, as the reference does. */
-__global__ void k_smat(const double *__restrict__ Gm, const double *__restrict__ g11c, int ne, int c1_second,
-                       double dte, double *__restrict__ s11, double *__restrict__ s12, double *__restrict__ s21,
-                       double *__restrict__ s22, unsigned *__restrict__ bar)
+ * unless c1_second) -> element (r, c) of the four ne x ne matrices of
+ * ccpsdv3/cpsd.c:415-437.  s21 and s12 are each filled from one triangle and
+ * mirrored, as the reference does. */
+struct SElem { double s11, s12, s21, s22; };
+__device__ __forceinline__ SElem s_elem(const double *__restrict__ Gm, const double *__restrict__ g11c, int ne,
+                                        int c1_second, double dte, int r, int c)
 {
-   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-   if (bar && idx == 0) *bar = 0u;
-   if (idx >= ne * ne) return;
-   const int r = idx % ne, c = idx / ne;   /* element (r, c) at r + c*ne */
    const int i = min(r, c), j = max(r, c);
    const int n2 = 2 * ne;
    const int o1 = c1_second ? ne : 0, o2 = c1_second ? 0 : ne;   /* row offsets of C1, C2 */
@@ -364,17 +360,34 @@ __global__ void k_smat(const double *__restrict__ Gm, const double *__restrict__
    const double g22 = Gm[(size_t)(o2 + i) * n2 + o2 + j];
    const double g21 = Gm[(size_t)(o2 + i) * n2 + o1 + j];      /* <c2_i|c1_j> */
    const double g12 = Gm[(size_t)(o1 + i) * n2 + o2 + j];      /* <c1_i|c2_j> */
+   SElem s;
    if (i == j) {
-      s22[idx] = (1.0 - g22) * 0.5 / dte;
-      s21[idx] = (1.0 - g21) * 0.5;
-      s12[idx] = s21[idx];
-      s11[idx] = -g11 * 0.5 * dte;
+      s.s22 = (1.0 - g22) * 0.5 / dte;
+      s.s21 = (1.0 - g21) * 0.5;
+      s.s12 = s.s21;
+      s.s11 = -g11 * 0.5 * dte;
    } else {
-      s22[idx] = -g22 * 0.5 / dte;
-      s21[idx] = -g21 * 0.5;
-      s12[idx] = -g12 * 0.5;
-      s11[idx] = -g11 * 0.5 * dte;
+      s.s22 = -g22 * 0.5 / dte;
+      s.s21 = -g21 * 0.5;
+      s.s12 = -g12 * 0.5;
+      s.s11 = -g11 * 0.5 * dte;
    }
+   return s;
+}
+
+/* the four matrices, column-major */
+__global__ void k_smat(const double *__restrict__ Gm, const double *__restrict__ g11c, int ne, int c1_second,
+                       double dte, double *__restrict__ s11, double *__restrict__ s12, double *__restrict__ s21,
+                       double *__restrict__ s22, unsigned *__restrict__ bar)
+{
+   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+   if (bar && idx == 0) *bar = 0u;
+   if (idx >= ne * ne) return;
+   const SElem s = s_elem(Gm, g11c, ne, c1_second, dte, idx % ne, idx / ne);
+   s22[idx] = s.s22;
+   s21[idx] = s.s21;
+   s12[idx] = s.s12;
+   s11[idx] = s.s11;
 }
 
 /* The preconditioned step's overlaps.  K o R is not orthogonal to c1 where
@@ -917,6 +930,126 @@ __global__ void __launch_bounds__(256, 2) k_lagrange_res(LagArgs a)
    }
 }
 
+/* ne <= 16 NT, NT <= 3: the whole fixed point in one workgroup, one wave per
+ * 16 x 16 tile.  A wave keeps the fragments of its rows of s11 and s21 and
+ * its columns of s12 in registers; X and st1 pass between waves through LDS,
+ * two workgroup barriers per iteration and no grid barrier, whose two round
+ * trips to L2 made up most of an iteration.  The K quarters that the
+ * kernel above spreads over four waves are four independent accumulators of
+ * one wave, added in the same order, so both give the same bits.  A
+ * latency-bound chain.  The s matrices are formed here from the Gram matrix
+ * (a.Gm), which saves a launch, unless the caller has them formed (the
+ * preconditioned step).  Per step, with the s matrices: 4 orbitals 21.6 -> 8.3
+ * us, 32 orbitals 40 -> 16.7.  At three tiles a side the SIMD that holds three
+ * of the nine waves takes 1.9 us of MFMA per iteration; four would need 3.4,
+ * no less than the kernel above. */
+template<int NT>
+__global__ void __launch_bounds__(NT * NT * 64) k_lagrange_one(LagArgs a)
+{
+   constexpr int N = 16 * NT, P = N + 2, KS = 4 * NT;   /* KS MFMA steps of 4 along K, NT per quarter */
+   __shared__ double X[N][P], st1[N][P], s12[N][P];
+   __shared__ double wmax[2][NT * NT];
+   const int ne = a.ne, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+   const int r0 = wave % NT * 16, c0 = wave / NT * 16, li = lane & 15, lk = lane >> 4;
+   auto elem = [&](int r, int c) {
+      SElem s = {0.0, 0.0, 0.0, 0.0};
+      if (r < ne && c < ne) {
+         const int e = r + c * ne;
+         if (a.Gm) s = s_elem(a.Gm, a.g11c, ne, a.c1_second, a.dte, r, c);
+         else s = SElem{a.s11[e], a.s12[e], a.s21[e], a.s22[e]};
+      }
+      return s;
+   };
+   double s11a[KS], s21a[KS], s22v[4], x[4];
+#pragma unroll
+   for (int m = 0; m < KS; ++m) {
+      const SElem s = elem(r0 + li, 4 * m + lk);
+      s11a[m] = s.s11;
+      s21a[m] = s.s21;
+   }
+#pragma unroll
+   for (int t = 0; t < 4; ++t) {
+      const int r = r0 + mfma16_row(t, lane), c = c0 + li;
+      const SElem s = elem(r, c);
+      s12[r][c] = s.s12;
+      s22v[t] = x[t] = s.s22;
+      X[r][c] = s.s22;
+      if (a.Gm && r < ne && c < ne) a.s11[r + c * ne] = s.s11;
+   }
+   __syncthreads();
+   int it = 0;
+   double gmax = 0.0;
+   while (it < a.itmax) {
+      ++it;
+      double xa[KS], xb[KS];
+#pragma unroll
+      for (int m = 0; m < KS; ++m) {
+         xb[m] = X[4 * m + lk][c0 + li];
+         xa[m] = X[r0 + li][4 * m + lk];
+      }
+      /* st1 = s11 X */
+      mfma_d4 acc[4];
+#pragma unroll
+      for (int w = 0; w < 4; ++w) acc[w] = mfma_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < NT; ++s)
+#pragma unroll
+         for (int w = 0; w < 4; ++w) acc[w] = mfma16(s11a[NT * w + s], xb[NT * w + s], acc[w]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+         st1[r0 + mfma16_row(t, lane)][c0 + li] = ((acc[0][t] + acc[1][t]) + acc[2][t]) + acc[3][t];
+      /* X_new = s22 + s21 X + X s12 + X st1 */
+#pragma unroll
+      for (int w = 0; w < 4; ++w) acc[w] = mfma_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < NT; ++s)
+#pragma unroll
+         for (int w = 0; w < 4; ++w) acc[w] = mfma16(s21a[NT * w + s], xb[NT * w + s], acc[w]);
+#pragma unroll
+      for (int s = 0; s < NT; ++s)
+#pragma unroll
+         for (int w = 0; w < 4; ++w) {
+            const int m = NT * w + s;
+            acc[w] = mfma16(xa[m], s12[4 * m + lk][c0 + li], acc[w]);
+         }
+      __syncthreads();   /* st1 is written, and every wave holds its fragments of X */
+#pragma unroll
+      for (int s = 0; s < NT; ++s)
+#pragma unroll
+         for (int w = 0; w < 4; ++w) {
+            const int m = NT * w + s;
+            acc[w] = mfma16(xa[m], st1[4 * m + lk][c0 + li], acc[w]);
+         }
+      double lmax = 0.0;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+         const int r = r0 + mfma16_row(t, lane), c = c0 + li;
+         const double v = s22v[t] + (((acc[0][t] + acc[1][t]) + acc[2][t]) + acc[3][t]);
+         if (r < ne && c < ne) {
+            lmax = fmax(lmax, fabs(v - x[t]));
+            x[t] = v;
+            X[r][c] = v;
+         }
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) lmax = fmax(lmax, __shfl_xor(lmax, o));
+      if (lane == 0) wmax[it & 1][wave] = lmax;
+      __syncthreads();
+      gmax = 0.0;
+#pragma unroll
+      for (int w = 0; w < NT * NT; ++w) gmax = fmax(gmax, wmax[it & 1][w]);
+      if (gmax < 1e-15) break;
+   }
+#pragma unroll
+   for (int t = 0; t < 4; ++t) {
+      const int r = r0 + mfma16_row(t, lane), c = c0 + li;
+      if (r < ne && c < ne) a.lmd[r + c * ne] = x[t];
+   }
+   if (tid == 0) {
+      a.info[0] = (double)it;
+      a.info[1] = gmax;
+   }
+}
 
 /* 128 < ne <= NM: the kernel above, with the panels streamed through three
  * LDS slots instead of kept (six resident panels of 256 would need 198 KB).
@@ -1325,10 +1458,19 @@ static int lagrange_grid_fits(const void *k, int grid, int lds)
    return 0;
 }
 
+/* up to 48 orbitals: see k_lagrange_one */
+int lagrange_one(int ne) { return ne <= 48; }
+
 int sd_lagrange(const LagArgs &a, hipStream_t s)
 {
    static std::atomic<int> checked[3] = {0, 0, 0};   /* largest grid shown to fit, per kernel */
-   if (a.ne <= 128) {
+   if (a.ne <= 16) {
+      hipLaunchKernelGGL(k_lagrange_one<1>, dim3(1), dim3(64), 0, s, a);
+   } else if (a.ne <= 32) {
+      hipLaunchKernelGGL(k_lagrange_one<2>, dim3(1), dim3(256), 0, s, a);
+   } else if (lagrange_one(a.ne)) {
+      hipLaunchKernelGGL(k_lagrange_one<3>, dim3(1), dim3(576), 0, s, a);
+   } else if (a.ne <= 128) {
       const int nt = (a.ne + 15) / 16;
       const int lds = 6 * 16 * (128 + 2) * (int)sizeof(double);
       static std::atomic<unsigned long long> attr{0};
