@@ -29,6 +29,8 @@
 #include <string>
 #include <map>
 #include <mutex>
+#include <condition_variable>
+#include <thread>
 #include <algorithm>
 
 #include "cpsd_internal.h"
@@ -181,6 +183,8 @@ struct cpsd_dev {
    int ngsum_parts, nxc_parts, norb_parts;
    double2 *fullbuf;      /* ne * nfft3d staging of the reference layout */
    double *realbuf;       /* n2ft3d staging */
+   char *stage;           /* pinned ring of HostCopier, made when first needed */
+   hipEvent_t stage_ev[8];
    double omega, cewald, rcut;
    int have_run;
    /* moving ions (move = 1): positions r2 after the step, forces, packed
@@ -256,6 +260,10 @@ static void ctx_free(cpsd_dev *c)
    free(c->gidx_h);
    free(c->Gp_h);
    for (int i = 0; i < c->ngc; ++i) (void)hipGraphExecDestroy(c->gcache[i].exec);
+   if (c->stage) {
+      for (hipEvent_t e : c->stage_ev) (void)hipEventDestroy(e);
+      (void)hipHostFree(c->stage);
+   }
    if (c->hout) (void)hipHostFree(c->hout);
    if (c->herr) (void)hipHostFree(c->herr);
    if (c->pool) {
@@ -1436,13 +1444,159 @@ static int ctx_clear_state(cpsd_dev *c)
    return 0;
 }
 
+/* Copies between the caller's (pageable) arrays and the device.  The runtime's
+ * own path moves pageable memory through one thread, about 9 GB/s each way;
+ * here a ring of pinned chunks is filled or emptied by a few threads while the
+ * DMA engine works on the others.  The threads live for one call of ctx_get /
+ * ctx_set_orbitals, the ring (16 MB) as long as its context.  Arrays below
+ * 4 MB, and every copy if threads or pinned memory cannot be had, take the
+ * plain path. */
+class HostCopier {
+   enum { SLOTS = 8, THREADS = 4 };
+   static constexpr size_t CHUNK = (size_t)2 << 20, LEAST = (size_t)4 << 20;
+   struct Job { int slot; char *host; size_t n; bool fill; };
+   cpsd_dev *c;
+   int dev = 0;
+   bool on = false, stop = false;
+   long issued = 0;                      /* chunks given a slot so far */
+   int failed = 0;
+   std::mutex mu;
+   std::condition_variable cv;
+   Job jobs[SLOTS];                      /* queued jobs [head, tail): at most one per slot */
+   long head = 0, tail = 0;
+   long done[SLOTS] = {0};               /* jobs finished on a slot */
+   std::thread th[THREADS];
+
+   void work()
+   {
+      int bad = hipSetDevice(dev) != hipSuccess;
+      std::unique_lock<std::mutex> lk(mu);
+      for (;;) {
+         cv.wait(lk, [&] { return stop || head < tail; });
+         if (head == tail) return;
+         const Job j = jobs[head++ % SLOTS];
+         lk.unlock();
+         char *pin = c->stage + (size_t)j.slot * CHUNK;
+         /* emptying: the chunk has arrived; filling: its last use has left */
+         if (hipEventSynchronize(c->stage_ev[j.slot]) != hipSuccess) bad = 1;
+         if (j.fill) memcpy(pin, j.host, j.n);
+         else memcpy(j.host, pin, j.n);
+         lk.lock();
+         done[j.slot]++;
+         if (bad) failed = 1;
+         cv.notify_all();
+      }
+   }
+   void push(const Job &j)
+   {
+      std::lock_guard<std::mutex> lk(mu);
+      jobs[tail++ % SLOTS] = j;
+      cv.notify_all();
+   }
+   void await(int slot, long count)
+   {
+      std::unique_lock<std::mutex> lk(mu);
+      cv.wait(lk, [&] { return done[slot] >= count; });
+   }
+   static bool ring(cpsd_dev *c)
+   {
+      if (c->stage) return true;
+      int n = 0;
+      for (; n < SLOTS; ++n)
+         if (hipEventCreateWithFlags(&c->stage_ev[n], hipEventDisableTiming) != hipSuccess) break;
+      void *p = nullptr;
+      if (n == SLOTS && hipHostMalloc(&p, SLOTS * CHUNK, hipHostMallocDefault) == hipSuccess) {
+         c->stage = static_cast<char *>(p);
+         return true;
+      }
+      while (n > 0) (void)hipEventDestroy(c->stage_ev[--n]);
+      (void)hipGetLastError();
+      return false;
+   }
+
+public:
+   /* total: bytes the call is going to move */
+   HostCopier(cpsd_dev *ctx, size_t total) : c(ctx)
+   {
+      if (total < LEAST || hipGetDevice(&dev) != hipSuccess || !ring(c)) return;
+      int n = 0;
+      try {
+         for (; n < THREADS; ++n) th[n] = std::thread([this] { work(); });
+      } catch (...) {
+      }
+      on = n > 0;
+   }
+   ~HostCopier()
+   {
+      {
+         std::lock_guard<std::mutex> lk(mu);
+         stop = true;
+         cv.notify_all();
+      }
+      for (std::thread &t : th)
+         if (t.joinable()) t.join();
+   }
+   /* device -> host after what is on the stream; the data is there after finish() */
+   int get(void *host, const void *d, size_t n)
+   {
+      if (!on || n < LEAST) {
+         CPSD_CHECK(hipMemcpyAsync(host, d, n, hipMemcpyDeviceToHost, c->stream));
+         return 0;
+      }
+      for (size_t o = 0; o < n; o += CHUNK, ++issued) {
+         const int slot = (int)(issued % SLOTS);
+         const size_t m = std::min(CHUNK, n - o);
+         await(slot, issued / SLOTS);
+         CPSD_CHECK(hipMemcpyAsync(c->stage + (size_t)slot * CHUNK, static_cast<const char *>(d) + o, m,
+                                   hipMemcpyDeviceToHost, c->stream));
+         CPSD_CHECK(hipEventRecord(c->stage_ev[slot], c->stream));
+         push(Job{slot, static_cast<char *>(host) + o, m, false});
+      }
+      return 0;
+   }
+   /* host -> device on the stream; the host array may change after it */
+   int put(void *d, const void *host, size_t n)
+   {
+      if (!on || n < LEAST) {
+         CPSD_CHECK(hipMemcpyAsync(d, host, n, hipMemcpyHostToDevice, c->stream));
+         return 0;
+      }
+      const long first = issued, count = (long)((n + CHUNK - 1) / CHUNK);
+      long pushed = 0;
+      for (long j = 0; j < count; ++j, ++issued) {
+         for (; pushed < count && pushed < j + SLOTS; ++pushed) {
+            const int slot = (int)((first + pushed) % SLOTS);
+            const size_t o = (size_t)pushed * CHUNK;
+            push(Job{slot, static_cast<char *>(const_cast<void *>(host)) + o, std::min(CHUNK, n - o), true});
+         }
+         const int slot = (int)(issued % SLOTS);
+         const size_t o = (size_t)j * CHUNK;
+         await(slot, issued / SLOTS + 1);
+         CPSD_CHECK(hipMemcpyAsync(static_cast<char *>(d) + o, c->stage + (size_t)slot * CHUNK, std::min(CHUNK, n - o),
+                                   hipMemcpyHostToDevice, c->stream));
+         CPSD_CHECK(hipEventRecord(c->stage_ev[slot], c->stream));
+      }
+      return 0;
+   }
+   /* everything is where it belongs */
+   int finish()
+   {
+      CPSD_CHECK(hipStreamSynchronize(c->stream));
+      if (!on) return 0;
+      for (long j = std::max(0L, issued - SLOTS); j < issued; ++j) await((int)(j % SLOTS), j / SLOTS + 1);
+      if (failed) { cpsd_set_error("copy to or from the host failed"); return -1; }
+      return 0;
+   }
+};
+
 static int ctx_set_orbitals(cpsd_dev *c, const double *cin)
 {
    hipStream_t st = c->stream;
    if (c->poisoned) TRY(ctx_clear_state(c));
    const size_t fstride = c->nfft3d;
-   CPSD_CHECK(hipMemcpyAsync(c->fullbuf, cin, (size_t)c->ne * c->n2ft3d * sizeof(double),
-                             hipMemcpyHostToDevice, st));
+   const size_t bytes = (size_t)c->ne * c->n2ft3d * sizeof(double);
+   HostCopier hc(c, bytes);
+   TRY(hc.put(c->fullbuf, cin, bytes));
    CPSD_CHECK(hipMemsetAsync(c->flag, 0, sizeof(int), st));
    /* a timed-out Lagrange barrier of an earlier run does not outlive it */
    CPSD_CHECK(hipMemsetAsync(c->err, 0, sizeof(int), st));
@@ -1455,7 +1609,7 @@ static int ctx_set_orbitals(cpsd_dev *c, const double *cin)
    TRY(sd_pack(c->fullbuf, fstride, c->gidx, c->ng, c->ngp, c->Cbase, c->ngp, c->ne, st));
    int flag = 0;
    CPSD_CHECK(hipMemcpyAsync(&flag, c->flag, sizeof(int), hipMemcpyDeviceToHost, st));
-   CPSD_CHECK(hipStreamSynchronize(st));
+   TRY(hc.finish());
    if (flag) {
       cpsd_set_error("orbital coefficients outside the cutoff mask are nonzero; the GPU path "
                      "stores masked coefficients only");
@@ -1464,24 +1618,19 @@ static int ctx_set_orbitals(cpsd_dev *c, const double *cin)
    return 0;
 }
 
-static int ctx_get_orb(cpsd_dev *c, const double2 *packed, double *host)
-{
-   hipStream_t st = c->stream;
-   TRY(sd_unpack(packed, c->ngp, c->pidx, c->nfft3d, c->fullbuf, c->nfft3d, c->ne, st));
-   CPSD_CHECK(hipMemcpyAsync(host, c->fullbuf, (size_t)c->ne * c->n2ft3d * sizeof(double),
-                             hipMemcpyDeviceToHost, st));
-   CPSD_CHECK(hipStreamSynchronize(st));
-   return 0;
-}
-
 static int ctx_get(cpsd_dev *c, double *c1, double *c2, double *cpsi, double *dn, double *hml,
                    double *lmd)
 {
-   const size_t orb = (size_t)c->ne * c->ngp;
+   const size_t orb = (size_t)c->ne * c->ngp, bytes = (size_t)c->ne * c->n2ft3d * sizeof(double);
    hipStream_t st = c->stream;
-   if (c1) TRY(ctx_get_orb(c, c->Cbase + (size_t)(c->cur ^ 1) * orb, c1));
-   if (c2) TRY(ctx_get_orb(c, c->Cbase + (size_t)c->cur * orb, c2));
-   if (cpsi) TRY(ctx_get_orb(c, c->CP, cpsi));
+   HostCopier hc(c, ((c1 != nullptr) + (c2 != nullptr) + (cpsi != nullptr)) * bytes);
+   auto get_orb = [&](const double2 *packed, double *host) {
+      TRY(sd_unpack(packed, c->ngp, c->pidx, c->nfft3d, c->fullbuf, c->nfft3d, c->ne, st));
+      return hc.get(host, c->fullbuf, bytes);
+   };
+   if (c1) TRY(get_orb(c->Cbase + (size_t)(c->cur ^ 1) * orb, c1));
+   if (c2) TRY(get_orb(c->Cbase + (size_t)c->cur * orb, c2));
+   if (cpsi) TRY(get_orb(c->CP, cpsi));
    if (dn) {
       TRY(sd_pad_real(c->dn, fft_slots(c->n), 2, c->realbuf, st));
       CPSD_CHECK(hipMemcpyAsync(dn, c->realbuf, (size_t)c->n2ft3d * sizeof(double),
@@ -1490,8 +1639,7 @@ static int ctx_get(cpsd_dev *c, double *c1, double *c2, double *cpsi, double *dn
    const size_t ee = (size_t)c->ne * c->ne;
    if (hml) CPSD_CHECK(hipMemcpyAsync(hml, c->hml, ee * sizeof(double), hipMemcpyDeviceToHost, st));
    if (lmd) CPSD_CHECK(hipMemcpyAsync(lmd, c->lmd, ee * sizeof(double), hipMemcpyDeviceToHost, st));
-   CPSD_CHECK(hipStreamSynchronize(st));
-   return 0;
+   return hc.finish();
 }
 
 /* The run epilogue of ccpsdv3/main.c:451-484 on the resident state:
@@ -2062,7 +2210,10 @@ static std::vector<double> g_r2;
 static int g_ctx_reusable = 0;
 
 /* 64-bit hash of a byte range: 8-byte words mixed with the splitmix64
- * finaliser (tail bytes zero-padded), chained through h */
+ * finaliser (tail bytes zero-padded), chained through h.  Whole 64-byte blocks
+ * run through eight chains, folded into one at their end: one chain waits for
+ * its own two multiplications at every word (3 ms for the tables of two kinds
+ * at 48^3, 0.5 with eight). */
 static uint64_t hash_bytes(uint64_t h, const void *p, size_t n)
 {
    const unsigned char *b = static_cast<const unsigned char *>(p);
@@ -2071,16 +2222,27 @@ static uint64_t hash_bytes(uint64_t h, const void *p, size_t n)
       z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
       return z ^ (z >> 31);
    };
+   const uint64_t step = 0x9e3779b97f4a7c15ull;
    size_t i = 0;
+   if (n >= 64) {
+      uint64_t l[8];
+      for (int q = 0; q < 8; ++q) l[q] = mix(h + (uint64_t)(q + 1) * step);
+      for (; i + 64 <= n; i += 64) {
+         uint64_t w[8];
+         memcpy(w, b + i, 64);
+         for (int q = 0; q < 8; ++q) l[q] = mix(l[q] ^ (w[q] + step));
+      }
+      for (int q = 0; q < 8; ++q) h = mix(h ^ (l[q] + step));
+   }
    for (; i + 8 <= n; i += 8) {
       uint64_t w;
       memcpy(&w, b + i, 8);
-      h = mix(h ^ (w + 0x9e3779b97f4a7c15ull));
+      h = mix(h ^ (w + step));
    }
    if (i < n) {
       uint64_t w = 0;
       memcpy(&w, b + i, n - i);
-      h = mix(h ^ (w + 0x9e3779b97f4a7c15ull));
+      h = mix(h ^ (w + step));
    }
    return mix(h ^ n);
 }
