@@ -771,7 +771,7 @@ static int sd_step(cpsd_dev *c, double dte, int last, int fp64)
       if (sb) TRY(ensure_bs(c));
       if (small) {
          TRY(launch_gemm_tn_small(reinterpret_cast<const double *>(c->B), K, c->nproj, A2, K, ne, c->w, K, 0,
-                                  c->P, st));
+                                  c->P, c->pnrm, scal2, c->Xkb, st));
       } else if (sb) {
          TRY(launch_kbproj_dbf16(c->BsH, c->BsL, c->nproj, A2, ne, c->w, K, sp, c->partial, c->partial_cap, st));
       } else if (f32 && c->mixed == 2) {
@@ -785,7 +785,6 @@ static int sd_step(cpsd_dev *c, double dte, int last, int fp64)
       TRY(ph_end(c, PH_KBPROJ));
       TRY(ph_begin(c, PH_KBRED));
       if (!small) TRY(launch_reduce_partials_kb(c->partial, sp, c->nproj, ne, c->P, c->pnrm, scal2, c->Xkb, st));
-      else TRY(sd_kbcoef(c->P, c->nproj, ne, c->pnrm, scal2, c->Xkb, st));
       TRY(ph_end(c, PH_KBRED));
    }
    if (c->move) {
@@ -898,7 +897,7 @@ static int sd_step(cpsd_dev *c, double dte, int last, int fp64)
          TRY(launch_gram_c2(Cb, K, 2 * ne, (c->cur ^ 1) * ne, c->w, K, c->gram_wgs, c->partial, c->partial_cap,
                             &so, &sdd, st));
       } else if (small) {
-         TRY(launch_gemm_tn_small(Cb, K, 2 * ne, Cb, K, 2 * ne, c->w, K, 1, c->Gm, st));
+         TRY(launch_gemm_tn_small(Cb, K, 2 * ne, Cb, K, 2 * ne, c->w, K, 1, c->Gm, nullptr, 0.0, nullptr, st));
       } else {
          TRY(launch_gemm_tn_splitk(Cb, K, 2 * ne, Cb, K, 2 * ne, c->w, K, sp, 1, c->partial, st));
       }
@@ -972,7 +971,8 @@ static int energy_tail(cpsd_dev *c, int inner, double dt, double dte)
       const int sp = splits_for(c, ne, ne, K, 0);
       if (gemm_tn_small_ok(ne, ne)) {
          TRY(launch_gemm_tn_small(reinterpret_cast<const double *>(C1), K, ne,
-                                  reinterpret_cast<const double *>(c->CP), K, ne, c->w, K, 0, c->Mh, st));
+                                  reinterpret_cast<const double *>(c->CP), K, ne, c->w, K, 0, c->Mh,
+                                  nullptr, 0.0, nullptr, st));
       } else {
          TRY(launch_gemm_tn_splitk(reinterpret_cast<const double *>(C1), K, ne,
                                    reinterpret_cast<const double *>(c->CP), K, ne, c->w, K, sp, 0,
@@ -1666,7 +1666,7 @@ static int ctx_epilogue(cpsd_dev *c, double *ortho, double *eig, double *V)
       }
       const double *c1r = reinterpret_cast<const double *>(C1);
       if (gemm_tn_small_ok(ne, ne)) {
-         TRY(launch_gemm_tn_small(c1r, K, ne, c1r, K, ne, c->w, K, 1, c->Gm, st));
+         TRY(launch_gemm_tn_small(c1r, K, ne, c1r, K, ne, c->w, K, 1, c->Gm, nullptr, 0.0, nullptr, st));
       } else {
          TRY(launch_gemm_tn_splitk(c1r, K, ne, c1r, K, ne, c->w, K, sp, 1, c->partial, st));
          TRY(launch_reduce_partials_symm(c->partial, ne, K, sp, c->Gm, st));

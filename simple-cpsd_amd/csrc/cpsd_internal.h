@@ -138,10 +138,13 @@ FftSlots fft_slots(int n);
  * symm (A == B, M == N): only the 16 x 16 blocks on or above the diagonal
  * are formed.                                                             */
 /* out[m][n] = sum_k w[k] A[m][k] B[n][k] directly (no partials) for the
- * small products gemm_tn_small_ok() admits; symm: out is written in full */
+ * small products gemm_tn_small_ok() admits; symm: out is written in full; X, if
+ * set, takes the KB apply coefficients X[m + n M] = -out[m][n] scal2 / pnrm[m]
+ * (ccpsdv3/cpsd.c:289) */
 int gemm_tn_small_ok(int M, int N);
 int launch_gemm_tn_small(const double *A, size_t lda, int M, const double *B, size_t ldb, int N,
-                         const double *w, size_t K, int symm, double *out, hipStream_t s);
+                         const double *w, size_t K, int symm, double *out, const double *pnrm, double scal2, double *X,
+                         hipStream_t s);
 /* tile list of a symmetric product restricted to some tiles (k_gemm_tn_splitk) */
 struct GramTiles {
    int noff, nd, halves;

@@ -84,7 +84,6 @@ int sd_smat_precond(const double *Gm, const double *g11, int ne, int c1_second, 
 int sd_precond_lmd(double *lmd, const double *DP, int ne, double dte, hipStream_t s);
 int sd_gram_next(const double *Gm, const double *g11, int ne, int c1_second, const double *lmd, double dte,
                  double *work, double *out, hipStream_t s);
-int sd_kbcoef(const double *P, int nproj, int ne, const double *pnrm, double scal2, double *X, hipStream_t s);
 /* the orbital count is solved by one workgroup, without grid barriers */
 int lagrange_one(int ne);
 int sd_lagrange(const LagArgs &a, hipStream_t s);

@@ -617,17 +617,6 @@ __global__ void __launch_bounds__(256) k_gram_next(const double *__restrict__ Gm
    }
 }
 
-/* P (nproj x ne, row-major, P[m][n] = gcdotc(beta_m, c1_n)) -> the apply
- * coefficients X[m + n*nproj] = -P scal2 / vnlnrm_m (ccpsdv3/cpsd.c:289) */
-__global__ void k_kbcoef(const double *__restrict__ P, int nproj, int ne, const double *__restrict__ pnrm,
-                         double scal2, double *__restrict__ X)
-{
-   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-   if (idx >= nproj * ne) return;
-   const int m = idx % nproj, n = idx / nproj;
-   X[idx] = -P[(size_t)m * ne + n] * scal2 / pnrm[m];
-}
-
 /* ---------------------------------------- Lagrange multiplier fixed point */
 
 /* thread 0 publishes the workgroup's writes (agent-scope release), arrives,
@@ -1428,13 +1417,6 @@ int sd_gram_next(const double *Gm, const double *g11, int ne, int c1_second, con
    }
    CPSD_CHECK(hipGetLastError());
    hipLaunchKernelGGL(k_gram_next, grid, dim3(256), 0, s, Gm, ne, c1_second, lmd, dte, W, T1, out);
-   CPSD_CHECK(hipGetLastError());
-   return 0;
-}
-
-int sd_kbcoef(const double *P, int nproj, int ne, const double *pnrm, double scal2, double *X, hipStream_t s)
-{
-   hipLaunchKernelGGL(k_kbcoef, g1((size_t)nproj * ne), dim3(256), 0, s, P, nproj, ne, pnrm, scal2, X);
    CPSD_CHECK(hipGetLastError());
    return 0;
 }
