@@ -52,19 +52,26 @@ __device__ __forceinline__ f4 mfma16(float a, float b, f4 c)
 
 #define PK 32           /* K step */
 #define PP (PK + 4)     /* row pitch (floats): a 16-byte read of 16 rows at one k hits distinct banks */
-#define PN 128          /* output columns (orbitals) per tile */
-
-/* 8 waves as 2 (rows) x 4 (columns), each (TM/2) x 32 of the TM x 128 tile;
- * one workgroup per (tile, K split), blocks assigned to the 8 XCDs so that
- * the workgroups one XCD runs together hold consecutive (tile, split)
- * pairs: the tiles of one K range then share that XCD's L2 */
-template<int TM>
-__global__ void __launch_bounds__(512, 4)
+/* The waves are 2 along the rows (projectors), TM / 2 each, times the columns
+ * (orbitals) of a tile: 4 of 32 (PN = 128), 4 of 16 (64) or 2 of 16 (32); one
+ * workgroup per (tile, K split), blocks assigned to the 8 XCDs so that the
+ * workgroups one XCD runs together hold consecutive (tile, split) pairs: the
+ * tiles of one K range then share that XCD's L2.  The K splits are about one a
+ * CU, so a workgroup of small products waits for its loads alone: DEPTH K
+ * tiles are on their way in registers.  An output's sum runs over k in order
+ * whatever the tile, so the results are the same.  Against 96 x 128 tiles with
+ * one K tile ahead: 42 x 28 at 64^3 28.0 -> 12.1 us, 96 x 64 at 80^3 77.6 -> 61.9. */
+template<int TM, int PN>
+__global__ void __launch_bounds__(PN == 32 ? 256 : 512, PN == 32 ? 2 : 4)
 k_kbproj_f32(const float *__restrict__ Bf, size_t ldb, int M, const double *__restrict__ C, size_t ldc,
              int N, const double *__restrict__ w, size_t K, size_t kchunk, int ntm, int ntile, int per,
              double *__restrict__ partial)
 {
-   constexpr int BI = TM / 32;   /* 16-row blocks per wave, and A loader rows per thread / 32 */
+   constexpr int NTH = PN == 32 ? 256 : 512, LR = NTH / 16;   /* threads; loader rows per pass */
+   constexpr int BI = TM / 32, BJ = PN == 128 ? 2 : 1;        /* 16-row and 16-column blocks per wave */
+   constexpr int AQ = TM / LR, CQ = PN / LR;                  /* A and B loader rows per thread */
+   constexpr int DEPTH = PN == 128 ? 1 : 3;
+   static_assert(TM % LR == 0 && PN % LR == 0, "whole loader passes");
    __shared__ float As[2][TM][PP];
    __shared__ float Bs[2][PN][PP];
    const int bid = blockIdx.x;
@@ -76,81 +83,88 @@ k_kbproj_f32(const float *__restrict__ Bf, size_t ldb, int M, const double *__re
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
    const int wm = wave & 1, wn = wave >> 1;
    const int q = lane >> 4, rr = lane & 15;
-   /* loader: rows lr + 32 h, k pair lq; 16 lanes cover one row's 32 k */
+   /* loader: rows lr + LR h, k pair lq; 16 lanes cover one row's 32 k */
    const int lr = tid >> 4, lq = (tid & 15) * 2;
 
-   f4 acc[BI][2];
+   f4 acc[BI][BJ];
 #pragma unroll
    for (int i = 0; i < BI; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < BJ; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
 
-   float2 ra[BI];
-   double2 rb[4], rw;
-   auto gload = [&](size_t k0) {
+   float2 ra[DEPTH][AQ];
+   double2 rb[DEPTH][CQ], rw[DEPTH];
+   auto gload = [&](int d, size_t k0) {
 #pragma unroll
-      for (int h = 0; h < BI; ++h) {
-         const int am = tm * TM + lr + 32 * h;
-         ra[h] = am < M ? *reinterpret_cast<const float2 *>(Bf + (size_t)am * ldb + k0 + lq)
-                        : make_float2(0.f, 0.f);
+      for (int h = 0; h < AQ; ++h) {
+         const int am = tm * TM + lr + LR * h;
+         ra[d][h] = am < M ? *reinterpret_cast<const float2 *>(Bf + (size_t)am * ldb + k0 + lq)
+                           : make_float2(0.f, 0.f);
       }
 #pragma unroll
-      for (int h = 0; h < 4; ++h) {
-         const int bn = tn * PN + lr + 32 * h;
-         rb[h] = bn < N ? *reinterpret_cast<const double2 *>(C + (size_t)bn * ldc + k0 + lq)
-                        : make_double2(0.0, 0.0);
+      for (int h = 0; h < CQ; ++h) {
+         const int bn = tn * PN + lr + LR * h;
+         rb[d][h] = bn < N ? *reinterpret_cast<const double2 *>(C + (size_t)bn * ldc + k0 + lq)
+                           : make_double2(0.0, 0.0);
       }
-      rw = *reinterpret_cast<const double2 *>(w + k0 + lq);
+      rw[d] = *reinterpret_cast<const double2 *>(w + k0 + lq);
    };
-   auto lstore = [&](int bf) {
+   auto lstore = [&](int d, int bf) {
 #pragma unroll
-      for (int h = 0; h < BI; ++h) *reinterpret_cast<float2 *>(&As[bf][lr + 32 * h][lq]) = ra[h];
+      for (int h = 0; h < AQ; ++h) *reinterpret_cast<float2 *>(&As[bf][lr + LR * h][lq]) = ra[d][h];
       /* the G-space weight (1 or 2, 0 on the padded tail) is exact in FP32 */
 #pragma unroll
-      for (int h = 0; h < 4; ++h)
-         *reinterpret_cast<float2 *>(&Bs[bf][lr + 32 * h][lq]) =
-            make_float2((float)(rb[h].x * rw.x), (float)(rb[h].y * rw.y));
+      for (int h = 0; h < CQ; ++h)
+         *reinterpret_cast<float2 *>(&Bs[bf][lr + LR * h][lq]) =
+            make_float2((float)(rb[d][h].x * rw[d].x), (float)(rb[d][h].y * rw[d].y));
    };
    auto mma = [&](int bf, int hk) {
-      f4 a[BI], b[2];
+      f4 a[BI], b[BJ];
 #pragma unroll
       for (int i = 0; i < BI; ++i) a[i] = *reinterpret_cast<const f4 *>(&As[bf][(TM / 2) * wm + 16 * i + rr][16 * hk + 4 * q]);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) b[j] = *reinterpret_cast<const f4 *>(&Bs[bf][32 * wn + 16 * j + rr][16 * hk + 4 * q]);
+      for (int j = 0; j < BJ; ++j) b[j] = *reinterpret_cast<const f4 *>(&Bs[bf][16 * BJ * wn + 16 * j + rr][16 * hk + 4 * q]);
 #pragma unroll
       for (int c = 0; c < 4; ++c)
 #pragma unroll
          for (int i = 0; i < BI; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = mfma16(a[i][c], b[j][c], acc[i][j]);
+            for (int j = 0; j < BJ; ++j) acc[i][j] = mfma16(a[i][c], b[j][c], acc[i][j]);
    };
 
-   /* K tile k+1 waits in registers while tile k is multiplied and goes to
-    * the other LDS buffer halfway through; one barrier per tile */
-   if (kb < ke) {
-      gload(kb);
-      lstore(0);
+   /* K tiles k + 1 .. k + DEPTH wait in registers while tile k is multiplied;
+    * the first of them goes to the other LDS buffer halfway through; one
+    * barrier per tile */
+   const int nt = kb < ke ? (int)((ke - kb + PK - 1) / PK) : 0;
+   if (nt > 0) {
+      gload(0, kb);
+      lstore(0, 0);
    }
    __syncthreads();
-   if (kb + PK < ke) gload(kb + PK);
-   int buf = 0;
-   for (size_t k0 = kb; k0 < ke; k0 += PK) {
-      mma(buf, 0);
-      if (k0 + PK < ke) {
-         lstore(buf ^ 1);
-         if (k0 + 2 * PK < ke) gload(k0 + 2 * PK);
+#pragma unroll
+   for (int d = 0; d < DEPTH; ++d)
+      if (1 + d < nt) gload(d, kb + (size_t)(1 + d) * PK);
+   for (int u = 0; u < nt; u += DEPTH) {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+         const int v = u + d;   /* the tile in LDS buffer v & 1; tile v + 1 is in register set d */
+         if (v >= nt) break;
+         mma(v & 1, 0);
+         if (v + 1 < nt) {
+            lstore(d, (v + 1) & 1);
+            if (v + 1 + DEPTH < nt) gload(d, kb + (size_t)(v + 1 + DEPTH) * PK);
+         }
+         mma(v & 1, 1);
+         __syncthreads();
       }
-      mma(buf, 1);
-      __syncthreads();
-      buf ^= 1;
    }
 
    /* 16 lanes hold 16 consecutive columns of one row: 128-byte segments */
 #pragma unroll
    for (int i = 0; i < BI; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-         const int n = tn * PN + 32 * wn + 16 * j + rr;
+      for (int j = 0; j < BJ; ++j) {
+         const int n = tn * PN + 16 * BJ * wn + 16 * j + rr;
 #pragma unroll
          for (int r = 0; r < 4; ++r) {
             const int p = tm * TM + (TM / 2) * wm + 16 * i + 4 * q + r;
@@ -167,19 +181,29 @@ int launch_kbproj_f32(const float *Bf, int M, const double *C, int N, const doub
       cpsd_set_error("kbproj_f32: %d splits of %d x %d do not fit the partial buffer", splits, M, N);
       return -1;
    }
+   /* rows: 64 where they hold all projectors, else the one of 96 and 128 that
+    * pads less; columns: 32 or 64 where they hold all orbitals */
    const int pad128 = (M + 127) / 128 * 128 - M, pad96 = (M + 95) / 96 * 96 - M;
-   const int tm = pad96 < pad128 ? 96 : 128;
-   const int ntm = (M + tm - 1) / tm, ntile = ntm * ((N + PN - 1) / PN);
+   const int tm = M <= 64 ? 64 : pad96 < pad128 ? 96 : 128, pn = N <= 32 ? 32 : N <= 64 ? 64 : 128;
+   const int ntm = (M + tm - 1) / tm, ntile = ntm * ((N + pn - 1) / pn);
    size_t kchunk = (K + splits - 1) / splits;
    kchunk = (kchunk + PK - 1) / PK * PK;
    const long pairs = (long)ntile * splits;
    const int per = pairs % 8 == 0 ? (int)(pairs / 8) : 0;
-   if (tm == 96)
-      hipLaunchKernelGGL((k_kbproj_f32<96>), dim3((unsigned)pairs), dim3(512), 0, s, Bf, K, M, C, K, N, w, K,
-                         kchunk, ntm, ntile, per, partial);
-   else
-      hipLaunchKernelGGL((k_kbproj_f32<128>), dim3((unsigned)pairs), dim3(512), 0, s, Bf, K, M, C, K, N, w, K,
-                         kchunk, ntm, ntile, per, partial);
+#define KBPROJ(TM_, PN_)                                                                                     \
+   if (tm == TM_ && pn == PN_)                                                                               \
+   hipLaunchKernelGGL((k_kbproj_f32<TM_, PN_>), dim3((unsigned)pairs), dim3(PN_ == 32 ? 256 : 512), 0, s, Bf, K, M, C, K, N, w, \
+                      K, kchunk, ntm, ntile, per, partial)
+   KBPROJ(64, 32);
+   KBPROJ(96, 32);
+   KBPROJ(128, 32);
+   KBPROJ(64, 64);
+   KBPROJ(96, 64);
+   KBPROJ(128, 64);
+   KBPROJ(64, 128);
+   KBPROJ(96, 128);
+   KBPROJ(128, 128);
+#undef KBPROJ
    CPSD_CHECK(hipGetLastError());
    return 0;
 }
@@ -187,19 +211,21 @@ int launch_kbproj_f32(const float *Bf, int M, const double *C, int N, const doub
 /* ----------------------------------------------------------- apply */
 
 #define AM 16           /* projectors per step */
-#define AN 128          /* output columns (orbitals) per workgroup */
+#define AKT 128         /* output reals per workgroup */
 #define XP (AM + 4)     /* Xs row pitch: a 16-byte read of 16 rows hits distinct banks */
 
-/* AKT output reals (k) per workgroup, 8 waves as 2 (columns) x 4 (k), each
- * 64 columns x AKT/4 k = 4 x AKT/64 blocks; the Bs row pitch AKT + 4 puts the
- * 4 rows 4 apart that one read touches 16 banks apart.  WAVES: waves per
- * SIMD the registers are sized for.
+/* AKT = 128 output reals (k) x AN columns (orbitals) per workgroup.  The waves
+ * are 4 along k, 32 reals each, times AN / 64 along the columns (one for AN =
+ * 32): up to 4 x 2 blocks a wave.  The Bs row pitch AKT + 4 puts the 4 rows 4
+ * apart that one read touches 16 banks apart.  WAVES: waves per SIMD the
+ * registers are sized for.  The column order of the sums does not depend on AN,
+ * so neither do the results.
  * TA = float: the KB apply, rows of Bf; C2 += dte result.
  * TA = double: the preconditioned step of the FP32 steps (PRE), rows of the
  * FP64 orbitals C1 rounded to FP32 as they are staged, X = hml:
  * C2 = C1 + Kp o (C2 - C1 + dte result), the update in FP64. */
-template<int AKT, int WAVES, typename TA, int PRE>
-__global__ void __launch_bounds__(512, WAVES)
+template<int AN, int WAVES, typename TA, int PRE>
+__global__ void __launch_bounds__(AN == 128 ? 512 : 256, WAVES)
 k_kbapply_f32(const TA *__restrict__ Bf, size_t ldb, int Mr, const double *__restrict__ X, int xsm, int ldx,
               int Nc, size_t K, double *__restrict__ C2, size_t ldc, double dte, int ntn, int per,
               const double *__restrict__ Kp, const double *__restrict__ C1, int Mr2,
@@ -212,10 +238,12 @@ k_kbapply_f32(const TA *__restrict__ Bf, size_t ldb, int Mr, const double *__res
     * epilogue is PRE's with result = B X + C1 hml. */
    const int Mr1 = PRE == 2 ? (Mr + AM - 1) / AM * AM : Mr;
    const int Mtot = PRE == 2 ? Mr1 + Mr2 : Mr;
-   constexpr int BP = AKT + 4, JB = AKT / 64, WKE = AKT / 4, BH = AKT / 128;
-   /* main loop: Bs[2][AM][BP] and Xs[2][AN][XP]; epilogue: T[64][BP], one
-    * 64-column half of the output tile at a time */
-   constexpr int BSZ = 2 * AM * BP, XSZ = 2 * AN * XP, TSZ = 64 * BP;
+   constexpr int NTH = AN == 128 ? 512 : 256, WN = AN == 128 ? 2 : 1;   /* threads; waves along the columns */
+   constexpr int CB = AN / WN / 16, JB = 2, BP = AKT + 4;               /* blocks per wave along the columns and k */
+   constexpr int BR = NTH / 32, BQ = AM / BR;                           /* Bs rows per pass of the loader */
+   /* main loop: Bs[2][AM][BP] and Xs[2][AN][XP]; epilogue: T[AN / WN][BP], the
+    * columns of one wave at a time */
+   constexpr int BSZ = 2 * AM * BP, XSZ = 2 * AN * XP, TSZ = AN / WN * BP;
    __shared__ float lds[BSZ + XSZ > TSZ ? BSZ + XSZ : TSZ];
    float (*Bs)[AM][BP] = reinterpret_cast<float (*)[AM][BP]>(lds);
    float (*Xs)[AN][XP] = reinterpret_cast<float (*)[AN][XP]>(lds + BSZ);
@@ -224,28 +252,28 @@ k_kbapply_f32(const TA *__restrict__ Bf, size_t ldb, int Mr, const double *__res
    const size_t k0 = (size_t)(g / ntn) * AKT;
    const int n0 = (g % ntn) * AN;
    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-   const int wn = wave & 1, wk = wave >> 1;
+   const int wn = wave % WN, wk = wave / WN;
    const int q = lane >> 4, rr = lane & 15;
-   /* loaders: Bs row br, BH 16-byte pieces from bc (32 lanes per row); Xs
-    * column xn, 4 projectors at xp */
-   const int br = tid >> 5, bc = (tid & 31) * 4 * BH;
+   /* loaders: Bs rows br + BR h at bc (32 lanes per row); Xs column xn, 4
+    * projectors at xp (AN = 32: half the threads) */
+   const int br = tid >> 5, bc = (tid & 31) * 4;
    const int xn = tid >> 2, xp = (tid & 3) * 4;
 
-   f4 acc[4][JB];   /* [column block][k block] */
+   f4 acc[CB][JB];   /* [column block][k block] */
 #pragma unroll
-   for (int i = 0; i < 4; ++i)
+   for (int i = 0; i < CB; ++i)
 #pragma unroll
       for (int j = 0; j < JB; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
 
-   float4 rb[BH];
+   float4 rb[BQ];
    double rx[4];
    auto gload = [&](int m0) {
       if (PRE == 2 && m0 >= Mr1) {
          /* orbital segment: rows of C1, X2 = hml */
-         const int m = m0 - Mr1 + br;
+         const size_t k = k0 + bc;
 #pragma unroll
-         for (int h = 0; h < BH; ++h) {
-            const size_t k = k0 + bc + 4 * h;
+         for (int h = 0; h < BQ; ++h) {
+            const int m = m0 - Mr1 + br + BR * h;
             rb[h] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (m < Mr2 && k < K) {
                const double2 u = *reinterpret_cast<const double2 *>(C1 + (size_t)m * ldc + k);
@@ -253,7 +281,7 @@ k_kbapply_f32(const TA *__restrict__ Bf, size_t ldb, int Mr, const double *__res
                rb[h] = make_float4((float)u.x, (float)u.y, (float)v.x, (float)v.y);
             }
          }
-         const int n = n0 + xn;
+         const int n = xn < AN ? n0 + xn : Nc;
 #pragma unroll
          for (int c = 0; c < 4; ++c) {
             const int mm = m0 - Mr1 + xp + c;
@@ -261,10 +289,10 @@ k_kbapply_f32(const TA *__restrict__ Bf, size_t ldb, int Mr, const double *__res
          }
          return;
       }
-      const int m = m0 + br;
+      const size_t k = k0 + bc;
 #pragma unroll
-      for (int h = 0; h < BH; ++h) {
-         const size_t k = k0 + bc + 4 * h;
+      for (int h = 0; h < BQ; ++h) {
+         const int m = m0 + br + BR * h;
          if constexpr (sizeof(TA) == 4) {
             rb[h] = (m < Mr && k < K) ? *reinterpret_cast<const float4 *>(Bf + (size_t)m * ldb + k)
                                       : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -277,7 +305,7 @@ k_kbapply_f32(const TA *__restrict__ Bf, size_t ldb, int Mr, const double *__res
             }
          }
       }
-      const int n = n0 + xn;
+      const int n = xn < AN ? n0 + xn : Nc;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
          const int mm = m0 + xp + c;
@@ -286,22 +314,23 @@ k_kbapply_f32(const TA *__restrict__ Bf, size_t ldb, int Mr, const double *__res
    };
    auto lstore = [&](int bf) {
 #pragma unroll
-      for (int h = 0; h < BH; ++h) *reinterpret_cast<float4 *>(&Bs[bf][br][bc + 4 * h]) = rb[h];
-      *reinterpret_cast<float4 *>(&Xs[bf][xn][xp]) =
-         make_float4((float)rx[0], (float)rx[1], (float)rx[2], (float)rx[3]);
+      for (int h = 0; h < BQ; ++h) *reinterpret_cast<float4 *>(&Bs[bf][br + BR * h][bc]) = rb[h];
+      if (xn < AN)
+         *reinterpret_cast<float4 *>(&Xs[bf][xn][xp]) =
+            make_float4((float)rx[0], (float)rx[1], (float)rx[2], (float)rx[3]);
    };
    /* slot q of instruction c takes projector 4q + c */
    auto mma = [&](int bf) {
-      f4 x[4];
+      f4 x[CB];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = *reinterpret_cast<const f4 *>(&Xs[bf][64 * wn + 16 * i + rr][4 * q]);
+      for (int i = 0; i < CB; ++i) x[i] = *reinterpret_cast<const f4 *>(&Xs[bf][16 * CB * wn + 16 * i + rr][4 * q]);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
          float b[JB];
 #pragma unroll
-         for (int j = 0; j < JB; ++j) b[j] = Bs[bf][4 * q + c][WKE * wk + 16 * j + rr];
+         for (int j = 0; j < JB; ++j) b[j] = Bs[bf][4 * q + c][32 * wk + 16 * j + rr];
 #pragma unroll
-         for (int i = 0; i < 4; ++i)
+         for (int i = 0; i < CB; ++i)
 #pragma unroll
             for (int j = 0; j < JB; ++j) acc[i][j] = mfma16(x[i][c], b[j], acc[i][j]);
       }
@@ -320,37 +349,29 @@ k_kbapply_f32(const TA *__restrict__ Bf, size_t ldb, int Mr, const double *__res
       buf ^= 1;
    }
 
-   /* epilogue per 64-column half: the half's waves stage their sums in LDS
-    * (lane (rr, q), register r holds column 16 i + 4 q + r, k = 16 j + rr
-    * of the wave's range), then every wave updates whole rows of C2, AKT/64
-    * reals per lane */
+   /* epilogue per wave column: its waves stage their sums in LDS (lane (rr,
+    * q), register r holds column 16 i + 4 q + r, k = 16 j + rr of the wave's
+    * range), then every wave updates whole rows of C2, two reals per lane */
    float (*T)[BP] = reinterpret_cast<float (*)[BP]>(lds);
 #pragma unroll
-   for (int half = 0; half < 2; ++half) {
+   for (int half = 0; half < WN; ++half) {
       if (half > 0) __syncthreads();
       if (wn == half) {
 #pragma unroll
-         for (int i = 0; i < 4; ++i)
+         for (int i = 0; i < CB; ++i)
 #pragma unroll
             for (int j = 0; j < JB; ++j)
 #pragma unroll
-               for (int r = 0; r < 4; ++r) T[16 * i + 4 * q + r][WKE * wk + 16 * j + rr] = acc[i][j][r];
+               for (int r = 0; r < 4; ++r) T[16 * i + 4 * q + r][32 * wk + 16 * j + rr] = acc[i][j][r];
       }
       __syncthreads();
       const size_t k = k0 + JB * lane;
 #pragma unroll 4
-      for (int nl = wave; nl < 64; nl += 8) {
-         const int n = n0 + 64 * half + nl;
+      for (int nl = wave; nl < 16 * CB; nl += NTH / 64) {
+         const int n = n0 + 16 * CB * half + nl;
          if (n < Nc && k < K) {
             double2 *p = reinterpret_cast<double2 *>(C2 + (size_t)n * ldc + k);
-            if constexpr (JB == 4) {
-               const float4 v = *reinterpret_cast<const float4 *>(&T[nl][4 * lane]);
-               double2 a = p[0], b = p[1];
-               a.x += dte * v.x; a.y += dte * v.y;
-               b.x += dte * v.z; b.y += dte * v.w;
-               p[0] = a;
-               p[1] = b;
-            } else if constexpr (PRE) {
+            if constexpr (PRE) {
                /* one complex coefficient per lane: k = 2 (k / 2) */
                const float2 v = *reinterpret_cast<const float2 *>(&T[nl][2 * lane]);
                const double *c1p = PRE == 2 ? C1 : reinterpret_cast<const double *>(Bf);
@@ -371,20 +392,28 @@ k_kbapply_f32(const TA *__restrict__ Bf, size_t ldb, int Mr, const double *__res
    }
 }
 
-/* 128 reals per workgroup: 32 accumulator registers per lane and 37 KB of
- * LDS let three workgroups share a CU (measured 14% faster than 256 reals
- * at two per CU on the 32-water cell: the C2 update of one workgroup
- * overlaps the products of the others) */
+/* columns of a workgroup: all orbitals up to 32 and 64 (no products of padding,
+ * and more, smaller workgroups a CU), tiles of 128 above: their 32
+ * accumulator registers per lane and 37 KB of LDS let three share a CU, so
+ * that the C2 update of one overlaps the products of the others.  Against
+ * tiles of 128: 28 orbitals at 64^3 30.4 -> 16.5 us, 64 orbitals at 80^3 with
+ * the preconditioned update 176 -> 135. */
+static int apply_f32_cols(int ne) { return ne <= 32 ? 32 : ne <= 64 ? 64 : 128; }
+
 int launch_kbapply_f32(const float *Bf, int Mr, const double *X, int xsm, int ldx, int Nc, size_t K,
                        double *C2, size_t ldc, double dte, hipStream_t s)
 {
-   constexpr int AKT = 128;
    if (K % 8) { cpsd_set_error("kbapply_f32: K=%zu not a multiple of 8", K); return -1; }
-   const int ntn = (Nc + AN - 1) / AN;
+   const int an = apply_f32_cols(Nc), ntn = (Nc + an - 1) / an;
    const long blocks = (long)((K + AKT - 1) / AKT) * ntn;
    const int per = blocks % 8 == 0 ? (int)(blocks / 8) : 0;
-   hipLaunchKernelGGL((k_kbapply_f32<AKT, KBAPPLY_WAVES, float, 0>), dim3((unsigned)blocks), dim3(512), 0, s, Bf, K,
-                      Mr, X, xsm, ldx, Nc, K, C2, ldc, dte, ntn, per, nullptr, nullptr, 0, nullptr, 0);
+#define KBAPPLY(AN_)                                                                                                  \
+   hipLaunchKernelGGL((k_kbapply_f32<AN_, AN_ == 64 ? 4 : KBAPPLY_WAVES, float, 0>), dim3((unsigned)blocks), dim3(AN_ == 128 ? 512 : 256), 0, \
+                      s, Bf, K, Mr, X, xsm, ldx, Nc, K, C2, ldc, dte, ntn, per, nullptr, nullptr, 0, nullptr, 0)
+   if (an == 32) KBAPPLY(32);
+   else if (an == 64) KBAPPLY(64);
+   else KBAPPLY(128);
+#undef KBAPPLY
    CPSD_CHECK(hipGetLastError());
    return 0;
 }
@@ -395,13 +424,17 @@ int launch_kbapply_f32(const float *Bf, int Mr, const double *X, int xsm, int ld
 int launch_precond_f32(const double *C1, int ne, const double *H, size_t K, double *C2, double dte,
                        const double *Kp, hipStream_t s)
 {
-   constexpr int AKT = 128;
    if (K % AKT) { cpsd_set_error("precond_f32: K=%zu not a multiple of %d", K, AKT); return -1; }
-   const int ntn = (ne + AN - 1) / AN;
+   const int an = apply_f32_cols(ne), ntn = (ne + an - 1) / an;
    const long blocks = (long)(K / AKT) * ntn;
    const int per = blocks % 8 == 0 ? (int)(blocks / 8) : 0;
-   hipLaunchKernelGGL((k_kbapply_f32<AKT, KBAPPLY_WAVES, double, 1>), dim3((unsigned)blocks), dim3(512), 0, s, C1,
-                      K, ne, H, 1, ne, ne, K, C2, K, dte, ntn, per, Kp, nullptr, 0, nullptr, 0);
+#define PRECOND(AN_)                                                                                                   \
+   hipLaunchKernelGGL((k_kbapply_f32<AN_, AN_ == 64 ? 4 : KBAPPLY_WAVES, double, 1>), dim3((unsigned)blocks), dim3(AN_ == 128 ? 512 : 256), 0, \
+                      s, C1, K, ne, H, 1, ne, ne, K, C2, K, dte, ntn, per, Kp, nullptr, 0, nullptr, 0)
+   if (an == 32) PRECOND(32);
+   else if (an == 64) PRECOND(64);
+   else PRECOND(128);
+#undef PRECOND
    CPSD_CHECK(hipGetLastError());
    return 0;
 }
@@ -415,18 +448,24 @@ int launch_kbapply_precond_f32(const float *Bf, int nproj, const double *X, cons
                                const double *H, size_t K, double *C2, double dte, const double *Kp,
                                hipStream_t s)
 {
-   constexpr int AKT = 128;
    if (K % AKT) { cpsd_set_error("kbapply_precond_f32: K=%zu not a multiple of %d", K, AKT); return -1; }
-   const int ntn = (ne + AN - 1) / AN;
+   const int an = apply_f32_cols(ne), ntn = (ne + an - 1) / an;
    const long blocks = (long)(K / AKT) * ntn;
    const int per = blocks % 8 == 0 ? (int)(blocks / 8) : 0;
-   hipLaunchKernelGGL((k_kbapply_f32<AKT, KBAPPLY_PRE_WAVES, float, 2>), dim3((unsigned)blocks), dim3(512), 0, s, Bf,
-                      K, nproj, X, 1, nproj, ne, K, C2, K, dte, ntn, per, Kp, C1, ne, H, ne);
+#define KBAPPLY_PRE(AN_)                                                                                                   \
+   hipLaunchKernelGGL((k_kbapply_f32<AN_, KBAPPLY_PRE_WAVES, float, 2>), dim3((unsigned)blocks), dim3(AN_ == 128 ? 512 : 256), 0, \
+                      s, Bf, K, nproj, X, 1, nproj, ne, K, C2, K, dte, ntn, per, Kp, C1, ne, H, ne)
+   if (an == 32) KBAPPLY_PRE(32);
+   else if (an == 64) KBAPPLY_PRE(64);
+   else KBAPPLY_PRE(128);
+#undef KBAPPLY_PRE
    CPSD_CHECK(hipGetLastError());
    return 0;
 }
 
 /* ------------------------------------------------ BF16-input projection */
+
+#define PN 128          /* output columns (orbitals) per tile */
 
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
