@@ -50,6 +50,7 @@ int sd_check_unmasked(const double2 *full, size_t fstride, const int *pidx, int 
                       int *flag, hipStream_t s);
 int sd_unpack(const double2 *packed, size_t pstride, const int *pidx, int nfft3d, double2 *full,
               size_t fstride, int ne, hipStream_t s);
+int sd_gmap(int n, const int *rows, const int *pidx, int ncol, int *gmap, hipStream_t s);
 int sd_pad_real(const double *field, const FftSlots &f, int pad, double *out, hipStream_t s);
 int sd_structure(const StructArgs &a, hipStream_t s);
 int sd_phafac(int n, const double *unitg, int nion, const double *r1, double2 *ex1, double2 *ex2,

@@ -42,6 +42,24 @@ __global__ void k_unpack(const double2 *__restrict__ packed, size_t pstride, con
    full[i * fstride + g] = (p >= 0) ? packed[i * pstride + p] : make_double2(0.0, 0.0);
 }
 
+/* gmap[kz][column] of ColTable from the packed index of the full grid; one
+ * thread per row (ky, kz) */
+__global__ void k_gmap(int n, const int *__restrict__ rows, const int *__restrict__ pidx, int ncol, int *__restrict__ gmap)
+{
+   const int r = blockIdx.x * blockDim.x + threadIdx.x, ky = r % n, kz = r / n, nh = n / 2 + 1;
+   if (r >= n * n) return;
+   const int len = rows[ky] >> 16;
+   int *g = gmap + (size_t)kz * ncol + (rows[ky] & 0xffff);
+   for (int kx = 0; kx < (len + 7) / 8 * 8; ++kx) g[kx] = kx < len ? pidx[kx + nh * r] : -1;
+}
+
+int sd_gmap(int n, const int *rows, const int *pidx, int ncol, int *gmap, hipStream_t s)
+{
+   hipLaunchKernelGGL(k_gmap, dim3((n * n + 63) / 64), dim3(64), 0, s, n, rows, pidx, ncol, gmap);
+   CPSD_CHECK(hipGetLastError());
+   return 0;
+}
+
 /* slot-ordered real field -> rows [z][y][x] with `pad` zeroed reals each */
 __global__ void k_pad_real(const double *__restrict__ field, FftSlots f, int pad, double *__restrict__ out)
 {
