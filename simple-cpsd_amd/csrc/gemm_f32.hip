@@ -467,6 +467,7 @@ int launch_kbapply_precond_f32(const float *Bf, int nproj, const double *X, cons
 
 #define PN 128          /* output columns (orbitals) per tile */
 
+typedef unsigned u4v __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ f4 mfma_bf16(bf8 a, bf8 b, f4 c)
@@ -1150,42 +1151,42 @@ k_apply_dbf16(const __bf16 *__restrict__ BtH, const __bf16 *__restrict__ BtL, in
 #pragma unroll
       for (int j = 0; j < BJ; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
 
-   uint4 rxh, rxl, rv[PU];
-   double2 rc[2 * CU];
+   u4v rxh, rxl, rv[PU];
+   d2v rc[2 * CU];
    auto gload = [&](int p0) {
       {
          const int n = tid >> 2, pc = (tid & 3) * 8;
-         rxh = *reinterpret_cast<const uint4 *>(XTh + (size_t)n * P + p0 + pc);
-         rxl = *reinterpret_cast<const uint4 *>(XTl + (size_t)n * P + p0 + pc);
+         rxh = *reinterpret_cast<const u4v *>(XTh + (size_t)n * P + p0 + pc);
+         rxl = *reinterpret_cast<const u4v *>(XTl + (size_t)n * P + p0 + pc);
       }
       if (p0 < npad) {
 #pragma unroll
          for (int u = 0; u < PU; ++u) {
             const int c = tid + NTH * u, cc = c & 511;
             const __bf16 *src = c < 512 ? BtH : BtL;
-            rv[u] = *reinterpret_cast<const uint4 *>(src + (kt + (cc >> 2)) * npad + p0 + (cc & 3) * 8);
+            rv[u] = *reinterpret_cast<const u4v *>(src + (kt + (cc >> 2)) * npad + p0 + (cc & 3) * 8);
          }
       } else {
          const int m = p0 - npad + 2 * orr;
 #pragma unroll
          for (int u = 0; u < CU; ++u) {
             const size_t k = kt + 2 * (4 * (wave + NWV * u) + okp);
-            rc[2 * u] = *reinterpret_cast<const double2 *>(C1 + (size_t)m * K + k);
-            rc[2 * u + 1] = *reinterpret_cast<const double2 *>(C1 + (size_t)(m + 1) * K + k);
+            rc[2 * u] = *reinterpret_cast<const d2v *>(C1 + (size_t)m * K + k);
+            rc[2 * u + 1] = *reinterpret_cast<const d2v *>(C1 + (size_t)(m + 1) * K + k);
          }
       }
    };
    auto lstore = [&](int bf, int p0) {
       {
          const int n = tid >> 2, pc = (tid & 3) * 8;
-         *reinterpret_cast<uint4 *>(Xat(bf, 0) + swz(n, pc)) = rxh;
-         *reinterpret_cast<uint4 *>(Xat(bf, 1) + swz(n, pc)) = rxl;
+         *reinterpret_cast<u4v *>(Xat(bf, 0) + swz(n, pc)) = rxh;
+         *reinterpret_cast<u4v *>(Xat(bf, 1) + swz(n, pc)) = rxl;
       }
       if (p0 < npad) {
 #pragma unroll
          for (int u = 0; u < PU; ++u) {
             const int c = tid + NTH * u, cc = c & 511;
-            *reinterpret_cast<uint4 *>(Vat(bf, c >> 9) + swz(cc >> 2, (cc & 3) * 8)) = rv[u];
+            *reinterpret_cast<u4v *>(Vat(bf, c >> 9) + swz(cc >> 2, (cc & 3) * 8)) = rv[u];
          }
       } else {
 #pragma unroll
@@ -1237,50 +1238,64 @@ k_apply_dbf16(const __bf16 *__restrict__ BtH, const __bf16 *__restrict__ BtL, in
       buf ^= 1;
    }
 
-   /* epilogue by halves of NO/2 orbitals: the waves of the half stage their
-    * sums in LDS ([n][VK + 4] FP32), then every wave updates whole 1 KB row
-    * pieces, lane l the complex coefficient at reals 2l, 2l + 1, with the
-    * loads of its HN / NWV rows issued before their stores (C2 is read and
-    * written) */
-   constexpr int HN = NO / 2, TP = VK + 4, ER = HN / NWV;
-   float (*T)[TP] = reinterpret_cast<float (*)[TP]>(alds);
+   /* epilogue by quarters of NO/4 orbitals: the waves of a quarter stage its
+    * sums in LDS ([n][VK + 4] FP32, two buffers), then every wave updates whole
+    * 1 KB row pieces, lane l the complex coefficient at reals 2l, 2l + 1.  The
+    * rows of C2 (and C1) of NS quarters are on their way at a time, the first
+    * before any sum is staged (one quarter where two would spill): 256 orbitals
+    * leave one workgroup on a CU, so nothing else hides their latency.  At 128
+    * orbitals and 96^3 0.28 ms, 0.41 with the update (0.49 while a loader array
+    * lay in scratch); at 256 and 128^3 1.51 and 2.45 ms, 4.5 and 4.4 TB/s with
+    * C1's second read */
+   constexpr int QN = NO / 4, TP = VK + 4, ER = QN / NWV, NS = NO == 256 && PRE ? 1 : 2;
+   float (*T)[QN][TP] = reinterpret_cast<float (*)[QN][TP]>(alds);
    const size_t kl = kt + 2 * lane;
-   double f = 0.0;
-   if (PRE) f = Kp[kl >> 1];
-#pragma unroll
-   for (int half = 0; half < 2; ++half) {
-      if (half > 0) __syncthreads();
-      if ((64 * wnn) / HN == half) {
-#pragma unroll
-         for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < BJ; ++j)
-#pragma unroll
-               for (int r = 0; r < 4; ++r)
-                  T[64 * wnn - HN * half + 16 * i + 4 * q + r][KW * wk + 16 * j + rr] = acc[i][j][r];
-      }
-      __syncthreads();
-      double2 c2v[ER], c1v[ER];
+   d2v c2v[NS][ER], c1v[NS][ER];
+   auto eload = [&](int qt) {
 #pragma unroll
       for (int u = 0; u < ER; ++u) {
-         const size_t o = (size_t)(HN * half + wave + NWV * u) * K + kl;
-         c2v[u] = *reinterpret_cast<const double2 *>(C2 + o);
-         if (PRE) c1v[u] = *reinterpret_cast<const double2 *>(C1 + o);
+         const size_t o = (size_t)(QN * qt + wave + NWV * u) * K + kl;
+         c2v[qt % NS][u] = *reinterpret_cast<const d2v *>(C2 + o);
+         if (PRE) c1v[qt % NS][u] = *reinterpret_cast<const d2v *>(C1 + o);
       }
+   };
+   auto stage = [&](int qt) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+         const int nb = 64 * wnn + 16 * i - QN * qt;
+         if (nb < 0 || nb >= QN) continue;
+#pragma unroll
+         for (int j = 0; j < BJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) T[qt & 1][nb + 4 * q + r][KW * wk + 16 * j + rr] = acc[i][j][r];
+      }
+   };
+   double f = 0.0;
+   if (PRE) f = Kp[kl >> 1];
+   eload(0);
+   if (NS == 2) eload(1);
+   stage(0);
+   __syncthreads();
+#pragma unroll
+   for (int qt = 0; qt < 4; ++qt) {
+      if (qt < 3) stage(qt + 1);
 #pragma unroll
       for (int u = 0; u < ER; ++u) {
          const int nl = wave + NWV * u;
-         const float2 v = *reinterpret_cast<const float2 *>(&T[nl][2 * lane]);
-         double2 a = c2v[u];
+         const float2 v = *reinterpret_cast<const float2 *>(&T[qt & 1][nl][2 * lane]);
+         d2v a = c2v[qt % NS][u];
          if (PRE) {
-            a.x = c1v[u].x + f * (a.x - c1v[u].x + dte * (double)v.x);
-            a.y = c1v[u].y + f * (a.y - c1v[u].y + dte * (double)v.y);
+            const d2v c = c1v[qt % NS][u];
+            a.x = c.x + f * (a.x - c.x + dte * (double)v.x);
+            a.y = c.y + f * (a.y - c.y + dte * (double)v.y);
          } else {
             a.x += dte * (double)v.x;
             a.y += dte * (double)v.y;
          }
-         *reinterpret_cast<double2 *>(C2 + (size_t)(HN * half + nl) * K + kl) = a;
+         *reinterpret_cast<d2v *>(C2 + (size_t)(QN * qt + nl) * K + kl) = a;
       }
+      if (qt + NS < 4) eload(qt + NS);
+      if (qt < 3) __syncthreads();
    }
 }
 

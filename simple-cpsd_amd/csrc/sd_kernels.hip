@@ -431,6 +431,7 @@ __global__ void __launch_bounds__(256) k_precond_dpq(const double *__restrict__ 
    const size_t s11 = g11c ? (size_t)ne : (size_t)n2;
    const double *a12 = Gm + (size_t)o1 * n2 + o2;      /* A12(k, c) = a12[k n2 + c] */
    double p = 0.0, q = 0.0;
+#pragma unroll 8
    for (int k = 0; k < ne; ++k) {
       const double dkj = a12[(size_t)k * n2 + j] - (k == j ? 1.0 : 0.0);
       const double dki = a12[(size_t)k * n2 + i] - (k == i ? 1.0 : 0.0);
@@ -460,6 +461,7 @@ __global__ void __launch_bounds__(256) k_precond_smat(const double *__restrict__
    const double *a12 = Gm + (size_t)o1 * n2 + o2;
    const double *pj = P + (size_t)j * ne;
    double r = 0.0;
+#pragma unroll 8
    for (int k = 0; k < ne; ++k) r += (a12[(size_t)k * n2 + i] - (k == i ? 1.0 : 0.0)) * pj[k];
    const double a22 = Gm[(size_t)(o2 + i) * n2 + o2 + j] - Q[idx] - Q[(size_t)i * ne + j] + r;
    const double a12p = a12[(size_t)i * n2 + j] - P[idx];
