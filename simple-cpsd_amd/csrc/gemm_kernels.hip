@@ -633,8 +633,8 @@ int launch_gemm_tn_small(const double *A, size_t lda, int M, const double *B, si
  * straight from the accumulators.  At most 256 VGPRs and 70 KB of LDS: two
  * workgroups share a CU and one's epilogue traffic overlaps the other's MFMA
  * stream.  Bound by the MFMA issue and, for short reductions, by the C2
- * update: at 64 waters the KB apply takes 3.4 ms (64
- * TFLOP/s) and the constraint 2.5 (4.28 and 2.93 ms with v_mfma_f64_4x4x4_4b
+ * update: at 64 waters the KB apply takes 3.35 ms (65
+ * TFLOP/s) and the constraint 2.45 (4.28 and 2.93 ms with v_mfma_f64_4x4x4_4b
  * and DPP-rotated operands). */
 template<int EPI, int NT>
 __global__ void __launch_bounds__(256, 2) k_gemm_tall(TallArgs a)
@@ -796,42 +796,54 @@ __global__ void __launch_bounds__(256, 2) k_gemm_tall(TallArgs a)
          }
       }
    } else {
+      /* column blocks whose rows are fetched together: the operands' registers
+       * are free now, and the compiler may not move a load over a store (one
+       * block at a time: constraint of 64 orbitals at 80^3 93 -> 85 us, KB apply
+       * and constraint of 256 at 128^3 2.98 -> 2.92 ms on average; four at 128
+       * columns spill, 3.00) */
+      constexpr int EJ = BJ < 2 || (EPI == EPI_CONSTRAINT && NT < 128) ? BJ : 2;
 #pragma unroll
       for (int p = 0; p < BP; ++p) {
          const size_t kc = kw + 32 * p;
          double f = 0.0;
          if (EPI == EPI_PRECOND) f = a.Kp[kc >> 1];
 #pragma unroll
-         for (int j = 0; j < BJ; ++j) {
-            double2 c2[4], c1[4], cp[4];
-            size_t idx[4];
-            bool in[4];
+         for (int j0 = 0; j0 < BJ; j0 += EJ) {
+            double2 c2[EJ][4], c1[EJ][4], cp[EJ][4];
+            auto at = [&](int j, int r) {   /* columns past Nc load the last one */
+               return (size_t)min(n0 + 64 * wn + 16 * j + mfma16_row(r, lane), a.Nc - 1) * a.ldc + kc;
+            };
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-               const int n = n0 + 64 * wn + 16 * j + mfma16_row(r, lane);
-               in[r] = n < a.Nc;
-               idx[r] = (size_t)min(n, a.Nc - 1) * a.ldc + kc;   /* columns past Nc load the last one */
-               if (EPI == EPI_CONSTRAINT || EPI == EPI_PRECOND) c2[r] = *reinterpret_cast<const double2 *>(a.C2 + idx[r]);
-               if (EPI == EPI_KBAPPLY || EPI == EPI_PRECOND) c1[r] = *reinterpret_cast<const double2 *>(a.C1 + idx[r]);
-               if (EPI == EPI_KBAPPLY) cp[r] = *reinterpret_cast<const double2 *>(a.CP + idx[r]);
-            }
+            for (int j = j0; j < j0 + EJ; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-               if (!in[r]) continue;
-               const double2 v = make_double2(acc[j][p][0][r], acc[j][p][1][r]);
-               double2 o = v;
-               if (EPI == EPI_KBAPPLY) {
-                  cp[r].x += v.x; cp[r].y += v.y;
-                  o = make_double2(c1[r].x + a.dte * cp[r].x, c1[r].y + a.dte * cp[r].y);
-                  if (a.write_cp) *reinterpret_cast<double2 *>(a.CP + idx[r]) = cp[r];
-               } else if (EPI == EPI_CONSTRAINT) {
-                  o = make_double2(c2[r].x + a.dte * v.x, c2[r].y + a.dte * v.y);
-               } else if (EPI == EPI_PRECOND) {
-                  o.x = c1[r].x + f * (c2[r].x - c1[r].x + a.dte * v.x);
-                  o.y = c1[r].y + f * (c2[r].y - c1[r].y + a.dte * v.y);
+               for (int r = 0; r < 4; ++r) {
+                  const size_t o = at(j, r);
+                  if (EPI == EPI_CONSTRAINT || EPI == EPI_PRECOND) c2[j - j0][r] = *reinterpret_cast<const double2 *>(a.C2 + o);
+                  if (EPI == EPI_KBAPPLY || EPI == EPI_PRECOND) c1[j - j0][r] = *reinterpret_cast<const double2 *>(a.C1 + o);
+                  if (EPI == EPI_KBAPPLY) cp[j - j0][r] = *reinterpret_cast<const double2 *>(a.CP + o);
                }
-               *reinterpret_cast<double2 *>(a.C2 + idx[r]) = o;
-            }
+#pragma unroll
+            for (int j = j0; j < j0 + EJ; ++j)
+#pragma unroll
+               for (int r = 0; r < 4; ++r) {
+                  if (n0 + 64 * wn + 16 * j + mfma16_row(r, lane) >= a.Nc) continue;
+                  const double2 v = make_double2(acc[j][p][0][r], acc[j][p][1][r]);
+                  const double2 d2 = c2[j - j0][r], d1 = c1[j - j0][r];
+                  const size_t e = at(j, r);
+                  double2 o = v;
+                  if (EPI == EPI_KBAPPLY) {
+                     double2 h = cp[j - j0][r];
+                     h.x += v.x; h.y += v.y;
+                     o = make_double2(d1.x + a.dte * h.x, d1.y + a.dte * h.y);
+                     if (a.write_cp) *reinterpret_cast<double2 *>(a.CP + e) = h;
+                  } else if (EPI == EPI_CONSTRAINT) {
+                     o = make_double2(d2.x + a.dte * v.x, d2.y + a.dte * v.y);
+                  } else if (EPI == EPI_PRECOND) {
+                     o.x = d1.x + f * (d2.x - d1.x + a.dte * v.x);
+                     o.y = d1.y + f * (d2.y - d1.y + a.dte * v.y);
+                  }
+                  *reinterpret_cast<double2 *>(a.C2 + e) = o;
+               }
          }
       }
    }
