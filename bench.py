@@ -77,15 +77,14 @@ def measured_traffic(workload):
     return out
 
 
-def algorithmic(phase, w, ng, nproj, ndnblk):
+def algorithmic(phase, w, ng, nproj, ndnblk, cols):
     """(kind, amount per SD step) of the algorithmic work of one phase:
     kind 'flop' for MFMA contractions (flops over the masked G vectors,
     complex coefficients as 2 reals), 'byte' for FFT / elementwise passes
     (compulsory traffic of the pass: its inputs read once, outputs written
-    once)."""
+    once; cols: (ky, kx) columns inside the cutoff)."""
     n, ne = w["nfft"], w["ne"]
-    nh = n // 2 + 1
-    plane = n * n * nh * 16            # one orbital's z-transformed array
+    plane = n * cols * 16              # one orbital's z-transformed array
     packed = ng * 16                   # one orbital's masked coefficients
     n3 = n ** 3 * 8
     if phase == "kb_projection":
@@ -261,6 +260,8 @@ def run(args):
     ms = elapsed * 1000.0 / args.steps
     value = args.steps / elapsed
     ndnblk = min(8, w["ne"])
+    n = w["nfft"]
+    cols = int(cell.masker[0::2].reshape(n, n, n // 2 + 1).any(axis=0).sum())
     phases = {}
     for name, (tms, calls) in prof.items():
         if calls == 0:
@@ -272,7 +273,7 @@ def run(args):
     roofline = None
     traffic = measured_traffic(args.workload)
     for name in sorted(phases, key=lambda n: -phases[n]["ms_per_step"]):
-        kind, amount = algorithmic(name, w, sizes["ng"], sizes["nproj"], ndnblk)
+        kind, amount = algorithmic(name, w, sizes["ng"], sizes["nproj"], ndnblk, cols)
         if kind is None:
             continue
         sec = phases[name]["ms_per_step"] / 1000.0
@@ -290,7 +291,7 @@ def run(args):
                             algorithmic_per_launch=per_launch)
         break
     for name in phases:
-        kind, amount = algorithmic(name, w, sizes["ng"], sizes["nproj"], ndnblk)
+        kind, amount = algorithmic(name, w, sizes["ng"], sizes["nproj"], ndnblk, cols)
         if kind is not None:
             sec = phases[name]["ms_per_step"] / 1000.0
             phases[name]["achieved"] = round(amount / sec / (1e12 if kind == "flop" else 1e9), 3)

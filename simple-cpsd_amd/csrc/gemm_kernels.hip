@@ -633,8 +633,8 @@ int launch_gemm_tn_small(const double *A, size_t lda, int M, const double *B, si
  * straight from the accumulators.  At most 256 VGPRs and 70 KB of LDS: two
  * workgroups share a CU and one's epilogue traffic overlaps the other's MFMA
  * stream.  Bound by the MFMA issue and, for short reductions, by the C2
- * update: at 64 waters the KB apply takes 3.35 ms (65
- * TFLOP/s) and the constraint 2.45 (4.28 and 2.93 ms with v_mfma_f64_4x4x4_4b
+ * update: at 64 waters the KB apply takes 3.6 ms (60
+ * TFLOP/s) and the constraint 2.5 (4.28 and 2.93 ms with v_mfma_f64_4x4x4_4b
  * and DPP-rotated operands). */
 template<int EPI, int NT>
 __global__ void __launch_bounds__(256, 2) k_gemm_tall(TallArgs a)
