@@ -16,8 +16,7 @@ struct StructArgs {
 
 struct LagArgs {
    int ne;
-   double *s11;
-   const double *s12, *s21, *s22;
+   double *s11, *s12, *s21, *s22;
    double *X;        /* 2 ne^2 */
    double *st1;      /* ne^2 */
    double *lmd;
@@ -26,7 +25,7 @@ struct LagArgs {
    unsigned *bar;    /* grid-barrier counter, zero at launch (sd_smat clears it) */
    int *err;
    /* lagrange_one(ne) only: the s matrices are formed from the Gram matrix (as
-    * sd_smat does; s11 is written) instead of read where Gm is set */
+    * sd_smat does, and stored) instead of read where Gm is set */
    const double *Gm = nullptr, *g11c = nullptr;
    int c1_second = 0;
    double dte = 0.0;

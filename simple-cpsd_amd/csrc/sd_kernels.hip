@@ -947,8 +947,8 @@ __global__ void __launch_bounds__(256, 2) k_lagrange_res(LagArgs a)
  * kernel above spreads over four waves are four independent accumulators of
  * one wave, added in the same order, so both give the same bits.  A
  * latency-bound chain.  The s matrices are formed here from the Gram matrix
- * (a.Gm), which saves a launch, unless the caller has them formed (the
- * preconditioned step).  Per step, with the s matrices: 4 orbitals 21.6 -> 8.3
+ * (a.Gm) and stored, which saves a launch, unless the caller has them formed
+ * (the preconditioned step).  Per step, with the s matrices: 4 orbitals 21.6 -> 8.3
  * us, 32 orbitals 40 -> 16.7.  At three tiles a side the SIMD that holds three
  * of the nine waves takes 1.9 us of MFMA per iteration; four would need 3.4,
  * no less than the kernel above. */
@@ -983,7 +983,6 @@ __global__ void __launch_bounds__(NT * NT * 64) k_lagrange_one(LagArgs a)
       s12[r][c] = s.s12;
       s22v[t] = x[t] = s.s22;
       X[r][c] = s.s22;
-      if (a.Gm && r < ne && c < ne) a.s11[r + c * ne] = s.s11;
    }
    __syncthreads();
    int it = 0;
@@ -1052,7 +1051,23 @@ __global__ void __launch_bounds__(NT * NT * 64) k_lagrange_one(LagArgs a)
 #pragma unroll
    for (int t = 0; t < 4; ++t) {
       const int r = r0 + mfma16_row(t, lane), c = c0 + li;
-      if (r < ne && c < ne) a.lmd[r + c * ne] = x[t];
+      if (r >= ne || c >= ne) continue;
+      a.lmd[r + c * ne] = x[t];
+      if (a.Gm) {
+         a.s12[r + c * ne] = s12[r][c];
+         a.s22[r + c * ne] = s22v[t];
+      }
+   }
+   /* not before the iterations, whose first barrier would wait for the stores */
+   if (a.Gm && c0 == 0) {
+#pragma unroll
+      for (int m = 0; m < KS; ++m) {
+         const int r = r0 + li, c = 4 * m + lk;
+         if (r < ne && c < ne) {
+            a.s11[r + c * ne] = s11a[m];
+            a.s21[r + c * ne] = s21a[m];
+         }
+      }
    }
    if (tid == 0) {
       a.info[0] = (double)it;
