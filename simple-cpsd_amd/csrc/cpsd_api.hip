@@ -1462,6 +1462,7 @@ class HostCopier {
    long head = 0, tail = 0;
    long done[SLOTS] = {0};               /* jobs finished on a slot */
    std::thread th[THREADS];
+   uintptr_t lo = UINTPTR_MAX, hi = 0;   /* the host addresses of the arrays so far */
 
    void work()
    {
@@ -1490,6 +1491,11 @@ class HostCopier {
    {
       std::unique_lock<std::mutex> lk(mu);
       cv.wait(lk, [&] { return done[slot] >= count; });
+   }
+   /* every chunk issued so far is in its array */
+   void drain()
+   {
+      for (long j = std::max(0L, issued - SLOTS); j < issued; ++j) await((int)(j % SLOTS), j / SLOTS + 1);
    }
    static bool ring(cpsd_dev *c)
    {
@@ -1529,10 +1535,17 @@ public:
       for (std::thread &t : th)
          if (t.joinable()) t.join();
    }
-   /* after what is on the stream; the data is there after finish() */
-   int get(void *host, const void *d, size_t n)
+   /* after what is on the stream; the data is there after finish().  Where a
+    * caller passes the same memory for several arrays, the last one stays in
+    * it: such an array waits for the chunks of those before it.  staged: the
+    * array may go through the ring */
+   int get(void *host, const void *d, size_t n, bool staged)
    {
-      if (!on || n < LEAST) {
+      const uintptr_t h = reinterpret_cast<uintptr_t>(host);
+      if (h < hi && h + n > lo) drain();
+      lo = std::min(lo, h);
+      hi = std::max(hi, h + n);
+      if (!on || !staged || n < LEAST) {
          CPSD_CHECK(hipMemcpyAsync(host, d, n, hipMemcpyDeviceToHost, c->stream));
          return 0;
       }
@@ -1551,8 +1564,7 @@ public:
    int finish()
    {
       CPSD_CHECK(hipStreamSynchronize(c->stream));
-      if (!on) return 0;
-      for (long j = std::max(0L, issued - SLOTS); j < issued; ++j) await((int)(j % SLOTS), j / SLOTS + 1);
+      drain();
       if (failed) { cpsd_set_error("copy to the host failed"); return -1; }
       return 0;
    }
@@ -1594,19 +1606,18 @@ static int ctx_get(cpsd_dev *c, double *c1, double *c2, double *cpsi, double *dn
    HostCopier hc(c, ((c1 != nullptr) + (c2 != nullptr) + (cpsi != nullptr)) * bytes);
    auto get_orb = [&](const double2 *packed, double *host) {
       TRY(sd_unpack(packed, c->ngp, c->pidx, c->nfft3d, c->fullbuf, c->nfft3d, c->ne, st));
-      return hc.get(host, c->fullbuf, bytes);
+      return hc.get(host, c->fullbuf, bytes, true);
    };
    if (c1) TRY(get_orb(c->Cbase + (size_t)(c->cur ^ 1) * orb, c1));
    if (c2) TRY(get_orb(c->Cbase + (size_t)c->cur * orb, c2));
    if (cpsi) TRY(get_orb(c->CP, cpsi));
    if (dn) {
       TRY(sd_pad_real(c->dn, fft_slots(c->n), 2, c->realbuf, st));
-      CPSD_CHECK(hipMemcpyAsync(dn, c->realbuf, (size_t)c->n2ft3d * sizeof(double),
-                                hipMemcpyDeviceToHost, st));
+      TRY(hc.get(dn, c->realbuf, (size_t)c->n2ft3d * sizeof(double), false));
    }
    const size_t ee = (size_t)c->ne * c->ne;
-   if (hml) CPSD_CHECK(hipMemcpyAsync(hml, c->hml, ee * sizeof(double), hipMemcpyDeviceToHost, st));
-   if (lmd) CPSD_CHECK(hipMemcpyAsync(lmd, c->lmd, ee * sizeof(double), hipMemcpyDeviceToHost, st));
+   if (hml) TRY(hc.get(hml, c->hml, ee * sizeof(double), false));
+   if (lmd) TRY(hc.get(lmd, c->lmd, ee * sizeof(double), false));
    return hc.finish();
 }
 
