@@ -183,8 +183,7 @@ struct cpsd_dev {
    int ngsum_parts, nxc_parts, norb_parts;
    double2 *fullbuf;      /* ne * nfft3d staging of the reference layout */
    double *realbuf;       /* n2ft3d staging */
-   char *stage;           /* pinned ring of HostCopier, made when first needed */
-   hipEvent_t stage_ev[4];
+   int stager;            /* counted among the users of StageRings */
    double omega, cewald, rcut;
    int have_run;
    /* moving ions (move = 1): positions r2 after the step, forces, packed
@@ -241,6 +240,78 @@ static int ph_end(cpsd_dev *c, int ph)
    return 0;
 }
 
+/* Pinned rings that the read-backs of all contexts share, one to a call at a
+ * time: at most RINGS of 8 MB, and when the last context that has used one goes
+ * they are given back but one.  That one stays because a ring takes up to 1.1 ms
+ * to pin: made by each context's first call, a call of 11 MB took 1.5 ms where
+ * the plain copy takes 0.7 and the ring 0.45. */
+class StageRings {
+public:
+   enum { SLOTS = 4, RINGS = 4 };
+   static constexpr size_t CHUNK = (size_t)2 << 20;
+   struct Ring { char *mem; hipEvent_t ev[SLOTS]; int dev, busy; };
+
+   static void join()
+   {
+      std::lock_guard<std::mutex> lk(mu);
+      ++users;
+   }
+   static void leave()
+   {
+      std::lock_guard<std::mutex> lk(mu);
+      if (--users > 0) return;
+      bool kept = false;
+      for (Ring &r : rings) {
+         if (!r.mem) continue;
+         if (!kept) { kept = true; continue; }
+         for (hipEvent_t e : r.ev) (void)hipEventDestroy(e);
+         (void)hipHostFree(r.mem);
+         r.mem = nullptr;
+      }
+   }
+   /* a ring for the device, or null */
+   static Ring *take(int dev)
+   {
+      std::lock_guard<std::mutex> lk(mu);
+      Ring *none = nullptr;
+      for (Ring &r : rings) {
+         if (r.mem && r.dev == dev && !r.busy) { r.busy = 1; return &r; }
+         if (!r.mem && !none) none = &r;
+      }
+      if (!none || !make(none, dev)) return nullptr;
+      none->busy = 1;
+      return none;
+   }
+   static void give(Ring *r)
+   {
+      std::lock_guard<std::mutex> lk(mu);
+      r->busy = 0;
+   }
+
+private:
+   static bool make(Ring *r, int dev)
+   {
+      int n = 0;
+      for (; n < SLOTS; ++n)
+         if (hipEventCreateWithFlags(&r->ev[n], hipEventDisableTiming) != hipSuccess) break;
+      void *p = nullptr;
+      if (n == SLOTS && hipHostMalloc(&p, SLOTS * CHUNK, hipHostMallocPortable) == hipSuccess) {
+         r->mem = static_cast<char *>(p);
+         r->dev = dev;
+         return true;
+      }
+      while (n > 0) (void)hipEventDestroy(r->ev[--n]);
+      (void)hipGetLastError();
+      return false;
+   }
+   static std::mutex mu;
+   static Ring rings[RINGS];
+   static int users;
+};
+std::mutex StageRings::mu;
+StageRings::Ring StageRings::rings[StageRings::RINGS];
+int StageRings::users = 0;
+
 static void ctx_free(cpsd_dev *c)
 {
    void *ptrs[] = {c->crows, c->gmap, c->gidx, c->pidx,
@@ -260,10 +331,7 @@ static void ctx_free(cpsd_dev *c)
    free(c->gidx_h);
    free(c->Gp_h);
    for (int i = 0; i < c->ngc; ++i) (void)hipGraphExecDestroy(c->gcache[i].exec);
-   if (c->stage) {
-      for (hipEvent_t e : c->stage_ev) (void)hipEventDestroy(e);
-      (void)hipHostFree(c->stage);
-   }
+   if (c->stager) StageRings::leave();
    if (c->hout) (void)hipHostFree(c->hout);
    if (c->herr) (void)hipHostFree(c->herr);
    if (c->pool) {
@@ -1443,18 +1511,20 @@ static int ctx_clear_state(cpsd_dev *c)
 /* Copies from the device to the caller's (pageable) arrays.  The runtime's own
  * path empties its staging with one thread, about 9 GB/s; here a ring of
  * pinned chunks is emptied by a few threads while the DMA engine fills the
- * others (28 orbitals at 64^3, 59 MB: 6.2 -> 2.1 ms, 3.6 with the ring to
- * make; uploads run at 27 GB/s either way).  The threads live for one call of ctx_get, the ring (8 MB) as
- * long as its context.  Calls below 8 MB, arrays below 4, arrays in pinned
- * memory (59 MB: 1.07 ms, 1.60 through the ring), and every copy if threads or
- * pinned memory cannot be had, take the plain path. */
+ * others (59 MB: 3.4 -> 1.6 ms, into fresh pages 6.2 -> 2.1; uploads run at
+ * 27 GB/s either way).  The threads live for one call of ctx_get.  Calls below
+ * 8 MB, arrays below 4, arrays in pinned memory (59 MB: 1.07 ms, 1.60 through
+ * the ring), and every copy if no ring or threads can be had, take the plain
+ * path. */
 class HostCopier {
-   enum { SLOTS = 4, THREADS = 4 };
-   static constexpr size_t CHUNK = (size_t)2 << 20, LEAST = (size_t)4 << 20;
+   enum { SLOTS = StageRings::SLOTS, THREADS = 4 };
+   static constexpr size_t CHUNK = StageRings::CHUNK, LEAST = (size_t)4 << 20;
    struct Job { int slot; char *host; size_t n; };
    cpsd_dev *c;
+   StageRings::Ring *ring = nullptr;
    int dev = 0;
    bool on = false, tried, stop = false;   /* the ring and its threads: there; there or not to be had */
+   bool finished = false;
    long issued = 0;                      /* chunks given a slot so far */
    int failed = 0;
    std::mutex mu;
@@ -1474,8 +1544,8 @@ class HostCopier {
          if (head == tail) return;
          const Job j = jobs[head++ % SLOTS];
          lk.unlock();
-         if (hipEventSynchronize(c->stage_ev[j.slot]) != hipSuccess) bad = 1;   /* the chunk has arrived */
-         memcpy(j.host, c->stage + (size_t)j.slot * CHUNK, j.n);
+         if (hipEventSynchronize(ring->ev[j.slot]) != hipSuccess) bad = 1;   /* the chunk has arrived */
+         memcpy(j.host, ring->mem + (size_t)j.slot * CHUNK, j.n);
          lk.lock();
          done[j.slot]++;
          if (bad) failed = 1;
@@ -1507,28 +1577,15 @@ class HostCopier {
       (void)hipGetLastError();
       return ok;
    }
-   static bool ring(cpsd_dev *c)
-   {
-      if (c->stage) return true;
-      int n = 0;
-      for (; n < SLOTS; ++n)
-         if (hipEventCreateWithFlags(&c->stage_ev[n], hipEventDisableTiming) != hipSuccess) break;
-      void *p = nullptr;
-      if (n == SLOTS && hipHostMalloc(&p, SLOTS * CHUNK, hipHostMallocDefault) == hipSuccess) {
-         c->stage = static_cast<char *>(p);
-         return true;
-      }
-      while (n > 0) (void)hipEventDestroy(c->stage_ev[--n]);
-      (void)hipGetLastError();
-      return false;
-   }
-
    /* the ring and its threads, when the first array needs them */
    bool start()
    {
       if (tried) return on;
       tried = true;
-      if (hipGetDevice(&dev) != hipSuccess || !ring(c)) return false;
+      if (hipGetDevice(&dev) != hipSuccess) return false;
+      if (!c->stager) { StageRings::join(); c->stager = 1; }
+      ring = StageRings::take(dev);
+      if (!ring) return false;
       int n = 0;
       try {
          for (; n < THREADS; ++n) th[n] = std::thread([this] { work(); });
@@ -1549,6 +1606,11 @@ public:
       }
       for (std::thread &t : th)
          if (t.joinable()) t.join();
+      if (ring) {
+         /* a call that failed may have chunks on their way */
+         if (!finished) (void)hipStreamSynchronize(c->stream);
+         StageRings::give(ring);
+      }
    }
    /* after what is on the stream; the data is there after finish().  Where a
     * caller passes the same memory for several arrays, the last one stays in
@@ -1568,9 +1630,9 @@ public:
          const int slot = (int)(issued % SLOTS);
          const size_t m = std::min(CHUNK, n - o);
          await(slot, issued / SLOTS);
-         CPSD_CHECK(hipMemcpyAsync(c->stage + (size_t)slot * CHUNK, static_cast<const char *>(d) + o, m,
+         CPSD_CHECK(hipMemcpyAsync(ring->mem + (size_t)slot * CHUNK, static_cast<const char *>(d) + o, m,
                                    hipMemcpyDeviceToHost, c->stream));
-         CPSD_CHECK(hipEventRecord(c->stage_ev[slot], c->stream));
+         CPSD_CHECK(hipEventRecord(ring->ev[slot], c->stream));
          push(Job{slot, static_cast<char *>(host) + o, m});
       }
       return 0;
@@ -1580,6 +1642,7 @@ public:
    {
       CPSD_CHECK(hipStreamSynchronize(c->stream));
       drain();
+      finished = true;
       if (failed) { cpsd_set_error("copy to the host failed"); return -1; }
       return 0;
    }

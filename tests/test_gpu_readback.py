@@ -1,5 +1,6 @@
 """cpsd_dev_get into host arrays of the caller's choosing."""
 import ctypes as C
+import threading
 import time
 
 import numpy as np
@@ -102,3 +103,87 @@ def test_pinned_arrays_take_the_direct_copy(gpu):
     dev.close()
     hip.ok(hip.L.hipFree(pd), "hipFree")
     hip.ok(hip.L.hipHostFree(ph), "hipHostFree")
+
+
+def fill(dev, ne, names):
+    return {k: np.full(ne * dev.cell.n2ft3d, np.nan) for k in names}
+
+
+# one array on either side of the 8 MB from which a call is staged (9 and 10
+# orbitals are 8.3 and 9.2 MB, the line lies at 8.4), of more than the ring, and
+# with a last chunk that is not whole; three arrays of 3.7 MB (a staged call whose
+# arrays are each below 4 MB), of 4.6 (each staged) and of 14.7.
+@pytest.mark.parametrize("ne,names", [(9, ("c2",)), (10, ("c2",)), (18, ("c2",)), (41, ("c2",)),
+                                      (4, ("c1", "c2", "cpsi")), (5, ("c1", "c2", "cpsi")), (16, ("c1", "c2", "cpsi")),
+                                      (5, ("c1", "cpsi"))])
+def test_read_back_by_size(gpu, ne, names):
+    print("[gpu-readback] %d orbitals at 48^3, %s" % (ne, " ".join(names)), flush=True)
+    dev = resident(ne)
+    dev.run(3)
+    blocks = dev.fetch(11).reshape(2, -1)   # the packed G coefficients; after 5 steps c1's are the first
+    packed = dict(c1=blocks[0], c2=blocks[1], cpsi=dev.fetch(3))
+    mask = dev.cell.masker.reshape(-1, 2)[:, 0] != 0
+    ngp = dev.sizes()["ngp"]
+    for _ in range(2):
+        out = fill(dev, ne, names)
+        get(dev, **out)
+        for k in names:
+            full = out[k].reshape(ne, -1, 2)
+            want = packed[k].reshape(ne, ngp, 2)[:, :mask.sum()]
+            assert np.array_equal(full[:, mask], want), k
+            assert not np.any(full[:, ~mask]), k
+    dev.close()
+
+
+def test_read_back_in_more_threads_than_rings(gpu):
+    """six contexts read back at once (four rings at most, one kept between the
+    contexts), freed and made again"""
+    print("[gpu-readback] six contexts, six threads", flush=True)
+    bad = []
+
+    def one(seed):
+        try:
+            for rep in range(2):
+                cell = cpsd_amd.water_cell(1, 14.0, 48, seed=1)
+                dev = cpsd_amd.DeviceSD(cell, 20)
+                for k in (1.0, 2.0, 3.0, 4.0):
+                    psi = k * cell.random_orbitals(20, seed=seed, decay=0.05)
+                    dev.set_orbitals(psi)
+                    assert np.array_equal(dev.get(c2=True)["c2"], psi.ravel())
+                dev.close()
+        except BaseException as e:   # noqa: BLE001
+            bad.append(e)
+    th = [threading.Thread(target=one, args=(s,)) for s in range(6)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not bad
+
+
+def pinned_rings():
+    """mappings of this process of a ring's size on the GPU's device file"""
+    n = 0
+    with open("/proc/self/maps") as f:
+        for line in f:
+            lo, hi = line.split()[0].split("-")
+            n += "/dev/dri/" in line and int(hi, 16) - int(lo, 16) == 8 << 20
+    return n
+
+
+def test_contexts_share_the_ring(gpu):
+    """read-backs one after the other leave as many 8 MB pinned as the first,
+    whatever the number of contexts, and a context that goes takes none away
+    from those that stay"""
+    devs = [resident(12) for _ in range(6)]
+    want = devs[0].get(c2=True)["c2"]
+    first = pinned_rings()
+    for d in devs[1:]:
+        assert np.array_equal(d.get(c2=True)["c2"], want)
+    print("[gpu-readback] 8 MB mappings after the first read-back %d, after six contexts' %d"
+          % (first, pinned_rings()), flush=True)
+    assert pinned_rings() == first
+    for d in devs[:-1]:
+        d.close()
+    assert np.array_equal(devs[-1].get(c2=True)["c2"], want)
+    devs[-1].close()
