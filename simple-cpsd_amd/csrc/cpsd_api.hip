@@ -364,8 +364,10 @@ static int splits_for(const cpsd_dev *c, int M, int N, size_t K, int symm)
 }
 
 /* The launch plan of a context: orbitals per FFT launch pair (fb), orbitals
- * per density partial plane of the FP64 and FP32 passes (nob; 0: the
- * fewest that fill whole rounds of the GPU's workgroup slots) and the
+ * per density partial plane of the FP64 and FP32 passes (nob; 0: as the
+ * workgroup slots of plane_density_occupancy, a table that stands for the
+ * rounding of the density sum and no longer counts what a CU holds, are best
+ * filled) and the
  * split-K workgroup target of the small-output products (wgt).  The
  * buffers whose sizes depend on it (density partials, split-K partials)
  * grow as needed; graphs captured before are dropped. */

@@ -164,11 +164,7 @@ template<int DIR> struct DFT<10, DIR> { template<typename V> static __device__ _
 template<int DIR> struct DFT<12, DIR> { template<typename V> static __device__ __forceinline__ void run(V *v) { dft_composite<4, 3, DIR>(v); } };
 template<int DIR> struct DFT<16, DIR> { template<typename V> static __device__ __forceinline__ void run(V *v) { dft_composite<4, 4, DIR>(v); } };
 
-/* logical index held by slot s in the transposed order of N = N1*N2 */
-template<int N1, int N2>
-__device__ __forceinline__ int tr_index(int s) { return s / N2 + N1 * (s % N2); }
-
-/* slot holding logical index j in the transposed order */
+/* slot holding logical index j in the transposed order of N = N1*N2 */
 template<int N1, int N2>
 __device__ __forceinline__ int tr_slot(int j) { return N2 * (j % N1) + j / N1; }
 

@@ -30,8 +30,11 @@
  * Stages are kept from contracting into each other (opaque), so results are
  * those of one trip per pass.  At 128^3 and 256 orbitals V psi takes 2.37 ms
  * (3.27 with eleven trips and 0.27 more of T), the density 1.16 (1.41), FP32
- * 1.26 (1.47) and 0.73 (0.97): bound by the vector ALU, about 18,000 cycles a
- * plane and CU, next to HBM, 14,000 (FP32 half of that).
+ * 1.26 (1.47) and 0.73 (0.97).  An FP64 V psi plane takes a CU about 44,000
+ * cycles: 25,000 of HBM traffic at the rate of a large copy, 18,000 of vector ALU
+ * (busy 0.44) and 13,000 of LDS (twelve passes over the plane at 128 bytes a
+ * cycle), in part one after the other, as one workgroup of eight waves fits a CU.
+ * The FP32 passes are bound by the vector ALU (busy 0.87 and 0.72).
  */
 #include "cpsd_internal.h"
 #include "fft_core.h"
@@ -59,7 +62,7 @@ __device__ __forceinline__ int zpass_index(const ColTable &t, int kz, int c)
    return c < t.P ? at(t.gmap, kz * t.P + c) : -1;
 }
 
-/* waves per SIMD: what the LDS column block admits, at most 4 */
+/* waves per SIMD: what the LDS column block admits, at most 3 */
 template<int N, typename V>
 constexpr int zpass_waves()
 {
@@ -690,7 +693,7 @@ __global__ void __launch_bounds__((plane_threads<N, MODE, V>()), (plane_min_wave
          }
       }
    } else if constexpr (MODE == PM_VPSI) {
-         /* orbitals [b0, b1) of plane z; with prefetch the potential stays in
+      /* orbitals [b0, b1) of plane z; with prefetch the potential stays in
        * registers for all of them */
       V vv[IX2][X2];
       auto load_v = [&]() {

@@ -16,7 +16,7 @@
  *                      applied to the A operand.
  *   k_gemm_tall      : tall output [ncol][K] = X^T A with a short reduction
  *                      (projectors or orbitals), 128-, 64- or 32-column x 128-row
- *                      output tiles over 8 waves, SD epilogues fused; the
+ *                      output tiles over 4 waves, SD epilogues fused; the
  *                      nonlocal force (ccpsdv3/cpsd.c:291-304) reduces its
  *                      output against the projectors instead of storing it.
  */
@@ -288,7 +288,11 @@ k_gemm_tn_splitk(const double *__restrict__ A, size_t lda, int M,
 }
 
 /* K splits of a symmetric product: the tiles above the diagonal take sp_off
- * and the diagonal tiles sp_dd, in the ratio 16 : 18 */
+ * and the diagonal tiles sp_dd, in the ratio 16 : 18 of a full tile's blocks to
+ * those of two diagonal tiles, `splits` workgroups per full tile and pair of
+ * diagonal tiles.  The launch forms every diagonal tile by itself, which gives
+ * it more workgroups than that; the counts stay because they decide the rounding
+ * of the sums */
 void gemm_tn_symm_splits(int M, size_t K, int splits, int *sp_off, int *sp_dd)
 {
    const int ntm = (M + TT - 1) / TT;
@@ -325,7 +329,8 @@ void gemm_tn_list_splits(int noff, int nd, size_t K, long wgs, int *sp_off, int 
    *sp_dd = sd;
 }
 
-/* tiles of one K split (pairs of diagonal tiles count as one) */
+/* tiles of one K split; pairs of diagonal tiles count as one, for the reason
+ * given at gemm_tn_symm_splits */
 int gemm_tn_tiles(int M, int N, int symm)
 {
    if (symm) {
@@ -464,9 +469,9 @@ int launch_gram_c2(const double *A, size_t lda, int M, int c2row, const double *
  * `splits`, or for a symmetric product (symm = block edge of the formed
  * blocks) sp_dd inside the 128 x 128 diagonal tiles and `splits` elsewhere;
  * only blocks with block(m) <= block(n) exist and the rest is mirrored.  A
- * workgroup covers 64 consecutive outputs with four thread groups: group g
- * sums the splits z = g mod 4 in two interleaved chains, and the four group
- * sums are added in g order, so the result does not depend on scheduling. */
+ * workgroup covers 64 consecutive outputs with RW waves: wave g sums the splits
+ * z = g mod RW in eight interleaved chains, and the waves' sums are added in g
+ * order, so the result does not depend on scheduling. */
 #define RW 16   /* waves per reduction workgroup, each over every RW-th split */
 
 /* with X non-null (KB projections: out = P, nproj x ne), also the apply

@@ -12,7 +12,10 @@
  * up, provided its accumulators stay in place: a kernel that may use more
  * than 256 registers per lane (__launch_bounds__(256) and no minimum of
  * waves) gets them copied between the two register files around every loop
- * and drops to 37-51, so the kernels below are all bounded to 256 or fewer.
+ * and drops to 37-51, so the GEMM kernels are bounded to 256 or fewer.  The
+ * Lagrange and carried-overlap kernels are not bound by the instruction (it
+ * keeps the matrix cores busy 0.05 of k_lagrange_str's time): of them only
+ * k_lagrange_res is bounded.
  */
 #pragma once
 #include <hip/hip_runtime.h>

@@ -2,7 +2,7 @@
 pass, with a last group that is not full: every orbital and the density against
 the same steps with one orbital per launch.
 
-A z-pass workgroup takes 2 (4) orbitals from 19 (37) at 128^3 and from 35 (69)
+A z-pass workgroup takes 2 (4) orbitals from 19 (37) at 128^3 and from 33 (65)
 at 96^3, a V psi workgroup at 128^3 one for every 8 orbitals, up to 4."""
 import numpy as np
 import pytest
