@@ -263,6 +263,7 @@ public:
       bool kept = false;
       for (Ring &r : rings) {
          if (!r.mem) continue;
+         r.busy = 0;   /* the streams of its calls are gone */
          if (!kept) { kept = true; continue; }
          for (hipEvent_t e : r.ev) (void)hipEventDestroy(e);
          (void)hipHostFree(r.mem);
@@ -331,7 +332,6 @@ static void ctx_free(cpsd_dev *c)
    free(c->gidx_h);
    free(c->Gp_h);
    for (int i = 0; i < c->ngc; ++i) (void)hipGraphExecDestroy(c->gcache[i].exec);
-   if (c->stager) StageRings::leave();
    if (c->hout) (void)hipHostFree(c->hout);
    if (c->herr) (void)hipHostFree(c->herr);
    if (c->pool) {
@@ -340,6 +340,7 @@ static void ctx_free(cpsd_dev *c)
       free(c->pool_ph);
    }
    if (c->stream) (void)hipStreamDestroy(c->stream);
+   if (c->stager) StageRings::leave();
    memset(c, 0, sizeof(*c));
 }
 
@@ -1608,11 +1609,9 @@ public:
       }
       for (std::thread &t : th)
          if (t.joinable()) t.join();
-      if (ring) {
-         /* a call that failed may have chunks on their way */
-         if (!finished) (void)hipStreamSynchronize(c->stream);
-         StageRings::give(ring);
-      }
+      /* a call that failed may have chunks on their way: the ring is nobody's
+       * until they have arrived */
+      if (ring && (finished || hipStreamSynchronize(c->stream) == hipSuccess)) StageRings::give(ring);
    }
    /* after what is on the stream; the data is there after finish().  Where a
     * caller passes the same memory for several arrays, the last one stays in

@@ -187,3 +187,29 @@ def test_contexts_share_the_ring(gpu):
         d.close()
     assert np.array_equal(devs[-1].get(c2=True)["c2"], want)
     devs[-1].close()
+
+
+def test_refused_read_backs_leave_the_next_ones_whole(gpu):
+    """while a stream is captured in global mode the runtime refuses the call's
+    wait, so it fails, with its copies on their way; more often than there are rings"""
+    print("[gpu-readback] refused during a capture", flush=True)
+    devs = [resident(20), resident(20, steps=3)]
+    want = [d.get(c2=True)["c2"] for d in devs]
+    hip = Hip()
+    for _ in range(6):
+        s, g = C.c_void_p(), C.c_void_p()
+        hip.ok(hip.L.hipStreamCreate(C.byref(s)), "hipStreamCreate")
+        hip.ok(hip.L.hipStreamBeginCapture(s, 0), "hipStreamBeginCapture")
+        a = np.empty_like(want[0])
+        p = [None, a.ctypes.data_as(C.c_void_p), None, None, None, None]
+        assert cpsd_amd.hip_lib().cpsd_dev_get(devs[0].h, *p) == -1
+        hip.L.hipStreamEndCapture(s, C.byref(g))     # invalidated by the call
+        hip.L.hipGetLastError()
+        hip.ok(hip.L.hipStreamDestroy(s), "hipStreamDestroy")
+        for d, w in zip(devs, want):
+            assert np.array_equal(d.get(c2=True)["c2"], w)
+    for d in devs:
+        d.close()
+    dev = resident(20)
+    assert np.array_equal(dev.get(c2=True)["c2"], want[0])
+    dev.close()
