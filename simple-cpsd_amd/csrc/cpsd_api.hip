@@ -1576,9 +1576,9 @@ class HostCopier {
    static bool known(const void *host)
    {
       hipPointerAttribute_t at;
-      const bool ok = hipPointerGetAttributes(&at, host) == hipSuccess && at.type != hipMemoryTypeUnregistered;
-      (void)hipGetLastError();
-      return ok;
+      if (hipPointerGetAttributes(&at, host) == hipSuccess) return at.type != hipMemoryTypeUnregistered;
+      (void)hipGetLastError();   /* the question's own error */
+      return false;
    }
    /* the ring and its threads, when the first array needs them */
    bool start()
